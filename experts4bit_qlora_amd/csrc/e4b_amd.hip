@@ -24,6 +24,7 @@
 #include "gemv.h"
 #include "lora.h"
 #include "lora_mfma.h"
+#include "quantize.h"
 #include "route.h"
 #include "scale.h"
 #include "train.h"
@@ -251,6 +252,18 @@ int launch_dequant_fmt(const e4b_qweight& w, int eb, int ec, int od, void* out, 
   return check_launch("dequant_kernel");
 }
 
+template <int DT>
+void launch_quantize_dt(const void* w, int64_t pieces, const e4b::QuantCode& q, bool cells, void* packed, float* absmax,
+                        hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(cdiv(pieces, e4b::kQuantThreads * e4b::kQuantUnroll)));
+  uint32_t* out = static_cast<uint32_t*>(packed);
+  if (cells)
+    hipLaunchKernelGGL((e4b::quantize4_kernel<DT, true>), grid, dim3(e4b::kQuantThreads), 0, s, w, pieces, q, out, absmax);
+  else
+    hipLaunchKernelGGL((e4b::quantize4_kernel<DT, false>), grid, dim3(e4b::kQuantThreads), 0, s, w, pieces, q, out,
+                       absmax);
+}
+
 // GEMV lanes per weight row: about four 16-byte chunks per lane.
 int gemv_group(int64_t k) {
   const int64_t chunks = k / 32;
@@ -405,6 +418,44 @@ int e4b_dequant(const e4b_qweight* w, int32_t expert_begin, int32_t expert_count
       return launch_dequant_fmt<E4B_FMT_NF4_DQ>(*w, expert_begin, expert_count, out_dtype, out, stream);
     default: return launch_dequant_fmt<E4B_FMT_MXFP4>(*w, expert_begin, expert_count, out_dtype, out, stream);
   }
+}
+
+int e4b_quantize_4bit(const void* w, int32_t dtype, int64_t values, const float* mids, const uint8_t* codes,
+                      int32_t zero_code, void* packed, float* absmax, hipStream_t stream) {
+  if (values < 0 || values % 64) return fail(E4B_EINVAL, "%lld values are not whole blocks of 64", (long long)values);
+  if (!any_dtype_ok(dtype)) return fail(E4B_EINVAL, "bad dtype %d", dtype);
+  if (!mids || !codes || zero_code < 0 || zero_code > 15) return fail(E4B_EINVAL, "bad code table");
+  if (values == 0) return E4B_OK;
+  if (!w || !packed || !absmax) return fail(E4B_EINVAL, "w/packed/absmax pointer is NULL");
+  if (!aligned16(w) || !aligned16(packed) || !aligned16(absmax))
+    return fail(E4B_EINVAL, "w, packed and absmax must be 16-byte aligned");
+  const int64_t pieces = values / 8;
+  if (cdiv(pieces, e4b::kQuantThreads * e4b::kQuantUnroll) > 0x7fffffff)
+    return fail(E4B_EUNSUPPORTED, "%lld values are more than one launch covers", (long long)values);
+  e4b::QuantCode q{};
+  q.zero = zero_code;
+  // cells: a code in sorted order whose midpoints lie in distinct cells of 1 / 16
+  bool cells = true;
+  int last = -1;
+  for (int i = 0; i < 15; ++i) {
+    q.mids[i] = mids[i];
+    if (i && !(mids[i] >= mids[i - 1])) return fail(E4B_EINVAL, "code midpoints must ascend");
+    const bool inside = mids[i] > -1.0f && mids[i] < 1.0f;
+    const int c = inside ? static_cast<int>(__builtin_fmaf(mids[i], 16.0f, 16.0f)) : -1;
+    if (c <= last) cells = false;
+    last = c;
+  }
+  for (int i = 0; i < 16; ++i) {
+    if (codes[i] > 15) return fail(E4B_EINVAL, "code %d out of range", codes[i]);
+    if (codes[i] != i) cells = false;
+    q.perm |= static_cast<uint64_t>(codes[i]) << (4 * i);
+  }
+  switch (dtype) {
+    case E4B_FP32: launch_quantize_dt<E4B_FP32>(w, pieces, q, cells, packed, absmax, stream); break;
+    case E4B_BF16: launch_quantize_dt<E4B_BF16>(w, pieces, q, cells, packed, absmax, stream); break;
+    default: launch_quantize_dt<E4B_FP16>(w, pieces, q, cells, packed, absmax, stream); break;
+  }
+  return check_launch("quantize4_kernel");
 }
 
 int e4b_route(const int64_t* top_k_index, int64_t tokens, int32_t top_k, int32_t num_experts, const e4b_routing* rt,

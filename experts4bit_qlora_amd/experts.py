@@ -237,7 +237,7 @@ class ExpertsNbit(nn.Module):
         if self.bits == 16:
             return flat.to(_PASSTHROUGH_DTYPES[self.quant_type]).contiguous(), None
         if self.bits == 4:
-            packed, absmax = Q.quantize_4bit(flat.float(), self.quant_type, self.blocksize)
+            packed, absmax = Q.quantize_4bit(flat, self.quant_type, self.blocksize)
             return packed.contiguous(), absmax.contiguous()
         q, absmax = Q.quantize_blocks(flat.float(), self.code.to(flat.device), self.blocksize)
         return q.contiguous(), absmax.contiguous()

@@ -147,6 +147,26 @@ def dequant(qw: QW, expert_begin: int = 0, expert_count: int | None = None, dtyp
     return out
 
 
+def quantize_4bit(w: torch.Tensor, mids, codes, zero_code: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """``[..., n]`` dense weights (``n`` a multiple of 64) -> (packed uint8 ``[..., n/2]``, absmax fp32
+    ``[..., n/64]``) in blocks of 64: ``mids`` the 15 ascending midpoints of the code, ``codes`` the
+    code at each of the 16 positions, ``zero_code`` that of an all-zero block."""
+    _require_cuda(w)
+    x = w.detach()
+    x = (x if x.dtype in _DT else x.float()).contiguous()
+    if x.data_ptr() % 16:  # a view that starts inside another tensor
+        x = x.clone()
+    n = x.shape[-1]
+    packed = torch.empty(*x.shape[:-1], n // 2, dtype=torch.uint8, device=x.device)
+    absmax = torch.empty(*x.shape[:-1], n // 64, dtype=torch.float32, device=x.device)
+    with torch.cuda.device(x.device):
+        N.check("e4b_quantize_4bit",
+                N.lib().e4b_quantize_4bit(x.data_ptr(), dtype_code(x.dtype), x.numel(), (ctypes.c_float * 15)(*mids),
+                                          (ctypes.c_uint8 * 16)(*codes), zero_code, packed.data_ptr(),
+                                          absmax.data_ptr(), _stream(x.device)))
+    return packed, absmax
+
+
 # ------------------------------------------------------------------------------ routing
 
 

@@ -17,6 +17,8 @@ On a HIP device the 4-bit dequantizers run the library's ``e4b_dequant`` kernel.
 """
 from __future__ import annotations
 
+import functools
+
 import torch
 
 NF4_CODE = (
@@ -86,14 +88,18 @@ def fp8_map(signed: bool = True, exponent_bits: int = 4, precision_bits: int = 3
     return t
 
 
+def _thresholds(code: torch.Tensor):
+    """Sorted positions of a code: (fp32 midpoints between neighbours, the sort permutation)."""
+    sc, perm = torch.sort(code.to(torch.float64).cpu(), stable=True)
+    return ((sc[:-1] + sc[1:]) / 2.0).to(torch.float32), perm
+
+
 def _nearest(code: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """Index into ``code`` of its nearest entry (midpoint thresholds over the sorted values, ties
     to the lower value). The fp4 table is not sorted, so the search runs on a sorted copy and
     maps back through the sort permutation."""
-    c = code.to(torch.float64).cpu()
-    sc, perm = torch.sort(c, stable=True)
-    mids = ((sc[:-1] + sc[1:]) / 2.0).to(torch.float32).to(x.device)
-    pos = torch.bucketize(x, mids, right=False)
+    mids, perm = _thresholds(code)
+    pos = torch.bucketize(x, mids.to(x.device), right=False)
     return perm.to(x.device)[pos]
 
 
@@ -112,9 +118,36 @@ def quantize_blocks(w: torch.Tensor, code: torch.Tensor, blocksize: int):
     return idx.reshape(w.shape).to(torch.uint8), absmax
 
 
+@functools.lru_cache(maxsize=None)
+def _host_table_4bit(quant_type: str):
+    """(midpoints, code per sorted position, code of zero) of a 4-bit code as host values."""
+    code = code_4bit(quant_type)
+    mids, perm = _thresholds(code)
+    return tuple(mids.tolist()), tuple(perm.tolist()), int(torch.argmin(code.abs()).item())
+
+
+def _on_kernel(w: torch.Tensor, blocksize: int) -> bool:
+    """Whether a stack goes through ``e4b_quantize_4bit``: plain device tensors in blocks of 64 that
+    no transform or graph follows. The rest (other block sizes, the CPU, a stack that autograd
+    records, tensor subclasses) takes the torch formulation, which is the kernel's definition."""
+    return (w.is_cuda and blocksize == 64 and w.numel() > 0 and w.dim() > 0 and w.shape[-1] % 64 == 0
+            and type(w) in (torch.Tensor, torch.nn.Parameter) and w.is_floating_point()
+            and not (w.requires_grad and torch.is_grad_enabled())
+            and not torch._C._functorch.is_functorch_wrapped_tensor(w))
+
+
 def quantize_4bit(w: torch.Tensor, quant_type: str = "nf4", blocksize: int = 64):
     """Row-major ``[..., n]`` weights -> (packed uint8 ``[..., n/2]``, absmax ``[..., n/bs]``).
-    Two values per byte, the first (even) value in the HIGH nibble."""
+    Two values per byte, the first (even) value in the HIGH nibble. On a HIP device one pass of
+    the library's kernel, bit for bit the torch formulation below it."""
+    if _on_kernel(w, blocksize):
+        from . import ops
+
+        return ops.quantize_4bit(w, *_host_table_4bit(quant_type))
+    return _quantize_4bit_torch(w, quant_type, blocksize)
+
+
+def _quantize_4bit_torch(w: torch.Tensor, quant_type: str, blocksize: int):
     code = code_4bit(quant_type, device=w.device)
     out_p, out_a = [], []
     flat = w.reshape(-1, w.shape[-1]) if w.dim() > 1 else w.reshape(1, -1)

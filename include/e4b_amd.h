@@ -101,6 +101,17 @@ int32_t e4b_mfma_tile_m(void);
 int e4b_dequant(const e4b_qweight* w, int32_t expert_begin, int32_t expert_count, int32_t out_dtype,
                 void* out, hipStream_t stream);
 
+/* Quantize `values` dense weights (E4B_BF16 / E4B_FP16 / E4B_FP32, a multiple of 64) in blocks of
+ * 64 to a 16-entry code: absmax[b] is the block's largest magnitude (a NaN stays one), each value
+ * times fp32(1 / absmax) takes the code of its position among the 15 ascending midpoints `mids`
+ * (the count of midpoints below it), codes[position]; a block whose absmax is zero or NaN takes
+ * zero_code throughout. packed is u8 [values / 2], first value of a pair in the high nibble,
+ * absmax fp32 [values / 64]. mids and codes are host arrays of 15 and 16 entries, read before the
+ * call returns. w, packed and absmax are 16-byte aligned.
+ * Replaces: bitsandbytes quantize_4bit at experts4bit_qlora/_vendor/experts.py:408-426. */
+int e4b_quantize_4bit(const void* w, int32_t dtype, int64_t values, const float* mids, const uint8_t* codes,
+                      int32_t zero_code, void* packed, float* absmax, hipStream_t stream);
+
 /* Per-expert weight exponents for the fp16 matrix-core mode of e4b_moe_forward: shift[e] =
  * 141 - max(E_e, 20), E_e the largest biased fp32 exponent of expert e's block scales (the
  * decoded ones for NF4_DQ), so every |code * absmax| * 2^shift[e] is below 2^15 and the scaled
