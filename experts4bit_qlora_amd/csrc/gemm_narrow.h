@@ -38,6 +38,7 @@
 #pragma once
 
 #include "gemm.h"
+#include "lora_mfma.h"
 #include "gemm_wide.h"
 
 namespace e4b {

@@ -26,7 +26,6 @@
 #pragma once
 
 #include "gemm.h"
-#include "lora_mfma.h"
 
 namespace e4b {
 
@@ -44,9 +43,7 @@ E4B_DEV int lds_at_w(int row, int col) { return row * kTileK + ((((col >> 3) ^ r
 
 // One tile. HALF: a tile of at most 128 rows (an expert's last, partial tile) as 128 rows x 256
 // weight rows, each wave 128 x 64 (two 32 x 32 MFMA columns), instead of padding it to 256 rows.
-// LORA: the accumulators start as the tile's LoRA delta (p.lt, p.lb), scaled like the products
-// (lora_mfma.h).
-template <int DT, int FMT, bool F16C, bool HALF, bool LORA>
+template <int DT, int FMT, bool F16C, bool HALF>
 E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2][kWideTileM * kTileK],
                        uint16_t (&Ws)[2][kWideTileN * kTileK], float* code2_s, int* row_shift_s,
                        const uint32_t* ptab) {
@@ -256,27 +253,6 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
   load_w(0, 0);
   load_w(1, min<int64_t>(1, klast));
   __syncthreads();  // code2 table, row shifts
-  if constexpr (LORA) {
-    // the accumulators start as the tile's LoRA delta, scaled like the products (lora_mfma.h):
-    // the lane's t rows (clamped to the expert's rows: the rest is never stored) times their
-    // activation shifts, the B rows of its columns (weight row 0 past n_out) times the expert's
-    // weight shift
-    const int la = lane;
-    int64_t brow[NS];
-#pragma unroll
-    for (int ns = 0; ns < NS; ++ns) {
-      const int tr = nbase[ns] + (la & 31);
-      if (pair) {
-        const int64_t jj = col0 + (tr & (BN / 2 - 1));
-        brow[ns] = jj < p.n_out ? (tr < BN / 2 ? jj : n / 2 + jj) : 0;
-      } else {
-        brow[ns] = col0 + tr < p.n_out ? col0 + tr : 0;
-      }
-    }
-    const int arow = wave_m * 128 + (la & 31);
-    lora_delta_32x32<MS, NS>(p, acc, e, row0 + arow, row_end - 1,
-                             [&](int ms) { return row_shift_s[arow + 32 * ms]; }, wsh, brow, la);
-  }
   stage(0, 0, block_scale(0));
   load_a_all(min<int64_t>(1, klast));
   load_w(0, min<int64_t>(2, klast));
@@ -466,10 +442,9 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
   });
 }
 
-template <int DT, int FMT, bool F16C = false, bool LORA = false>
+template <int DT, int FMT, bool F16C = false>
 __global__ void __launch_bounds__(kWideThreads) gemm_wide_kernel(GemmArgs p) {
   static_assert(!F16C || (DT == E4B_BF16 && FMT != E4B_FMT_MXFP4), "fp16 mode: bf16 activations, NF4 weights");
-  static_assert(!LORA || F16C, "the LoRA epilogue runs in the fp16 mode");
   constexpr int BM = kWideTileM, BN = kWideTileN;
   __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * kTileK];
   __shared__ __attribute__((aligned(16))) uint16_t Ws[2][BN * kTileK];
@@ -490,8 +465,8 @@ __global__ void __launch_bounds__(kWideThreads) gemm_wide_kernel(GemmArgs p) {
     for (int j = 0; j < 16; ++j) ptab[j * kWideThreads + threadIdx.x] = cvt_pair<E4B_FP16>(p.w.code[j], lo);
   }
   const int rows = p.rt.offsets[item.e + 1] - item.row0;  // the tile's rows, capped at BM below
-  if (rows <= BM / 2) wide_tile<DT, FMT, F16C, true, LORA>(p, tile, n_tile, As, Ws, code2_s, row_shift_s, ptab);
-  else wide_tile<DT, FMT, F16C, false, LORA>(p, tile, n_tile, As, Ws, code2_s, row_shift_s, ptab);
+  if (rows <= BM / 2) wide_tile<DT, FMT, F16C, true>(p, tile, n_tile, As, Ws, code2_s, row_shift_s, ptab);
+  else wide_tile<DT, FMT, F16C, false>(p, tile, n_tile, As, Ws, code2_s, row_shift_s, ptab);
 }
 
 }  // namespace e4b

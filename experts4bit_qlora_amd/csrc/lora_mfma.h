@@ -1,5 +1,5 @@
 // The LoRA delta of a grouped GEMM tile, on the matrix cores, in the tile's fp32 accumulators
-// (the LORA instances of gemm_wide_kernel and gemm_narrow_kernel):
+// (the LORA instances of gemm_wide8_kernel and gemm_narrow_kernel):
 //
 //   acc[m, j] += lscale * sum_q t[m, q] * B[e, row(j), q]
 //
@@ -82,29 +82,26 @@ E4B_DEV void lora_b_piece(const GemmArgs& p, int ex, int64_t row, int q0, int e2
   split_bf16x8(v, hi, lo);
 }
 
-// The delta of 32 x 32 accumulator blocks (v_mfma_f32_32x32x16: lane l supplies row / column
-// l % 32 and the eight ranks 8 (l / 32) .. of each 16-rank step), scaled like the fp16 mode's
-// products: t row of block row ms = min(arow0 + 32 ms, arow_last), times 2^ashift(ms) (its
-// activation row's shift, exact); B rows brow[ns], times 2^bshift (the expert's weight shift). Run
-// on zeroed accumulators before a tile's main loop, where its loads overlap the tile's first loads
-// and few registers are live; the epilogue then removes the scales from the sum.
-template <int MS, int NS, class AS>
-E4B_DEV void lora_delta_32x32(const GemmArgs& p, f32x16_t (&acc)[MS][NS], int e, int64_t arow0, int64_t arow_last,
-                              AS&& ashift, int bshift, const int64_t (&brow)[NS], int lane) {
+// The delta of a wave's 32 x 32 accumulator blocks, weights first (v_mfma_f32_32x32x16: lane l
+// supplies weight / tile row l % 32 and the eight ranks 8 (l / 32) .. of each 16-rank step), scaled
+// like the fp16 mode's products: t row of block ms = min(arow0 + 32 ms, arow_last), times
+// 2^ashift(ms) (its activation row's shift, exact); B row brow, times 2^bshift (the expert's weight
+// shift). Run on zeroed accumulators before a tile's main loop, where its loads overlap the tile's
+// first loads and few registers are live; the epilogue then removes the scales from the sum.
+template <int MS, class AS>
+E4B_DEV void lora_delta_32x32(const GemmArgs& p, f32x16_t (&acc)[MS], int e, int64_t arow0, int64_t arow_last,
+                              AS&& ashift, int bshift, int64_t brow, int lane) {
   const int g8 = 8 * (lane >> 5);
   const bool b_lo = p.lbdt != E4B_BF16;  // a bf16 B has no lo half
   for (int q0 = 0; q0 < p.lr; q0 += 16) {
-    uint4 bh[NS], bl[NS];
-#pragma unroll
-    for (int ns = 0; ns < NS; ++ns) lora_b_piece(p, e, brow[ns], q0 + g8, bshift, bh[ns], bl[ns]);
+    uint4 bh, bl;
+    lora_b_piece(p, e, brow, q0 + g8, bshift, bh, bl);
     static_for<MS>([&](auto ms) {
       uint4 ah, al;
       lora_t_piece(p, min(arow0 + 32 * int(ms), arow_last), q0 + g8, ashift(int(ms)), ah, al);
-      static_for<NS>([&](auto ns) {
-        acc[ms][ns] = mfma_32x32x16<E4B_BF16>(ah, bh[ns], acc[ms][ns]);
-        acc[ms][ns] = mfma_32x32x16<E4B_BF16>(al, bh[ns], acc[ms][ns]);
-        if (b_lo) acc[ms][ns] = mfma_32x32x16<E4B_BF16>(ah, bl[ns], acc[ms][ns]);
-      });
+      acc[ms] = mfma_32x32x16<E4B_BF16>(bh, ah, acc[ms]);
+      acc[ms] = mfma_32x32x16<E4B_BF16>(bh, al, acc[ms]);
+      if (b_lo) acc[ms] = mfma_32x32x16<E4B_BF16>(bl, ah, acc[ms]);
     });
   }
 }
