@@ -803,12 +803,13 @@ int e4b_lora_wgrad(const float* u, int32_t rank, const void* a, int32_t a_dtype,
   if (gather_k < 0) return fail(E4B_EINVAL, "gather_k must be >= 0");
   if (!rt || !rt->offsets || (gather_k > 0 && !rt->sorted_flat)) return fail(E4B_EINVAL, "routing offsets / order are NULL");
   if (!out || (M > 0 && (!u || !a))) return fail(E4B_EINVAL, "NULL pointer");
-  if (cdiv(cols, e4b::kWgradThreads) > 0x7fffffffLL) return fail(E4B_EUNSUPPORTED, "too many columns");
+  if (cdiv(cols, e4b::kWgradCols) > 0x7fffffffLL) return fail(E4B_EUNSUPPORTED, "too many columns");
   // every expert's block writes its rows of out (zeros for an expert without rows)
-  const dim3 grid(static_cast<unsigned>(cdiv(cols, e4b::kWgradThreads)), static_cast<unsigned>(num_experts));
+  const dim3 grid(static_cast<unsigned>(cdiv(cols, e4b::kWgradCols)), static_cast<unsigned>(num_experts));
 #define E4B_WG(XD, RB)                                                                                            \
-  hipLaunchKernelGGL((e4b::lora_wgrad_kernel<XD, RB>), grid, dim3(e4b::kWgradThreads), 0, stream, u, rank,       \
-                     static_cast<const uint16_t*>(a), gather_k, rt->sorted_flat, rt->offsets, cols, scale, out)
+  hipLaunchKernelGGL((e4b::lora_wgrad_kernel<XD, RB, false>), grid, dim3(e4b::kWgradThreads), 0, stream, u, rank, \
+                     static_cast<const uint16_t*>(a), gather_k, rt->sorted_flat, rt->offsets, cols, scale, out,   \
+                     E4B_FP32)
 #define E4B_WG_R(XD)                                     \
   if (rank <= 16) E4B_WG(XD, 16);                        \
   else if (rank <= 32) E4B_WG(XD, 32);                   \

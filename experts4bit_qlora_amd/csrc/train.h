@@ -14,16 +14,16 @@
 //                      v_mfma_f32_16x16x32 with fp32 accumulators; two register stages of global
 //                      loads ahead of the MFMAs, double-buffered LDS, one barrier per 64-deep step,
 //                      the decode of step s + 1 interleaved with the MFMAs of step s.
-//   lora_wgrad_kernel  out[e, j, c] = scale * sum over expert e's rows m of u[m, j] * a_m[c] (in
-//                      row order): dL/dA = scaling * (g . B)^T . x and dL/dB^T = scaling * t^T . g
-//                      of a LoRA projection, per expert. Block (expert, 256 columns); the rows'
-//                      u entries are staged in LDS 32 at a time and broadcast to the block.
+//   lora_wgrad_kernel  out[e, j, c] = scale * sum over expert e's rows m of u[m, j] * a_m[c]:
+//                      dL/dA = scaling * (g . B)^T . x and dL/dB^T = scaling * t^T . g of a LoRA
+//                      projection, per expert, on the matrix cores.
 #pragma once
 
 #include <type_traits>
 
 #include "common.h"
 #include "gemm.h"
+#include "lora_mfma.h"
 
 namespace e4b {
 
@@ -264,62 +264,186 @@ __global__ void __launch_bounds__(dgrad_threads(BM)) dgrad_mfma_kernel(DgradArgs
 }
 
 constexpr int kWgradThreads = 256;
-constexpr int kWgradRows = 32;  // u rows staged per round
+constexpr int kWgradRows = 64;   // rows per round
+constexpr int kWgradCols = 128;  // columns per block, 32 per wave
 
-// out[e, j, c] = scale * sum_{m in expert e's rows, in order} u[m, j] * a_m[c], for j < r,
-// c < cols; zero for an expert without rows. Block = (expert blockIdx.y, columns 256 *
-// blockIdx.x ..); a_m = row sorted_flat[m] / gather_k of a (gather_k > 0) or row m.
-template <int XDT, int RB>
+// 4 x 16-bit transposing LDS read: the 16 lanes of a group name the 16 8-byte pieces of a 4-row x
+// 16-column block (lane i: row i / 4, columns 4 (i % 4) ..) and lane i receives column i, rows 0..3.
+E4B_DEV uint2 lds_read_tr(const uint16_t* p) {
+  typedef short s4_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s4_t* lds_t;
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(p)));
+}
+
+// Element offset of column col (a multiple of 4) of row `row` in a tile of 16-bit rows of COLS columns:
+// the row's 32-byte pieces are XOR-ed with row bits 0, 1 and 3, so the eight rows of a half-wave's
+// transposing read (four neighbours, and the four eight further on) lie in distinct banks.
+template <int COLS>
+E4B_DEV int wgrad_at(int row, int col) {
+  constexpr int kMask = COLS / 16 >= 8 ? 7 : COLS / 16 - 1;
+  return row * COLS + ((((col >> 4) ^ ((row & 3) | ((row >> 1) & 4))) & kMask) << 4) + ((col >> 4) & ~kMask) * 16 +
+         (col & 15);
+}
+
+// The leading bf16 part of v, taken off it: truncated, so it never overflows and three parts hold
+// any finite fp32 value exactly; an infinity or NaN is its own first part and leaves zeros.
+E4B_DEV uint16_t bf16_part(float& v) {
+  const uint32_t b = __float_as_uint(v);
+  const bool fin = (b & 0x7f800000u) != 0x7f800000u;
+  const uint16_t part = fin ? static_cast<uint16_t>(b >> 16) : from_f<E4B_BF16>(v);
+  v = fin ? v - __uint_as_float(b & 0xffff0000u) : 0.0f;
+  return part;
+}
+
+// out[e, j, c] = scale * sum_{m in expert e's rows} u[m, j] * a_m[c], for j < r, c < cols; zero for an
+// expert without rows. Block = (columns 128 * blockIdx.x .., expert blockIdx.y); a_m = row
+// sorted_flat[m] / gather_k of a (gather_k > 0) or row m. TRANS: out[e, c, j] (a B gradient in its
+// parameter's layout); odt: the dtype out is rounded to.
+//
+// A product over rows, so both operands are read along their row axis: 64 rows at a time are staged
+// in LDS as they lie in memory and the MFMA operands (eight rows of one column per lane) come from
+// transposing reads. u is fp32: its three bf16 parts (each what is left of it, cut to 8 bits) hold all 24
+// significant bits, so every product on the bf16 matrix cores is exact and only the fp32 order of
+// the sum differs from a multiply-add loop; fp16 rows are two bf16 parts, exact too. Bound by
+// reading a once per 128 columns: the next round's rows are in flight while this one's multiply.
+// OLMoE, 2,048 tokens, rank 16: the four gradients 243 -> 83 us; Qwen3, 509 tokens, rank 32,
+// 487 -> 111 us (VALU multiply-adds with u broadcast from LDS before).
+template <int XDT, int RB, bool TRANS>
 __global__ void __launch_bounds__(kWgradThreads) lora_wgrad_kernel(const float* __restrict__ u, int r,
                                                                    const uint16_t* __restrict__ a, int gather_k,
                                                                    const int32_t* __restrict__ sorted_flat,
                                                                    const int32_t* __restrict__ offsets, int64_t cols,
-                                                                   float scale, float* __restrict__ out) {
-  __shared__ float4 us[kWgradRows][RB / 4];
+                                                                   float scale, void* __restrict__ out, int odt) {
+  constexpr int NSM = RB / 16;
+  constexpr int AP = kWgradRows * kWgradCols / 8 / kWgradThreads;  // 16-byte pieces of a per thread
+  constexpr int UP = kWgradRows * RB / kWgradThreads;              // u values per thread
+  __shared__ __attribute__((aligned(16))) uint16_t as[kWgradRows * kWgradCols];
+  __shared__ __attribute__((aligned(16))) uint16_t us[3][kWgradRows * RB];
   const int e = static_cast<int>(blockIdx.y);
-  const int64_t c = int64_t(blockIdx.x) * kWgradThreads + threadIdx.x;
+  const int64_t c0 = int64_t(blockIdx.x) * kWgradCols;
   const int beg = offsets[e], end = offsets[e + 1];
-  float acc[RB];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
+  const int l16 = lane & 15, g = lane >> 4;
+
+  // a pieces: piece i of thread t is row t / 16 + 16 i of the round, columns 8 (t % 16) ..; whole
+  // pieces (cols % 8 == 0, aligned) or single elements; columns past the end read column 0 (their
+  // sums are never stored)
+  const int ac = 8 * (tid & 15);
+  const bool vec = (cols & 7) == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
+  auto row_of = [&](int m) -> int64_t { return gather_k > 0 ? static_cast<int64_t>(sorted_flat[m] / gather_k) : m; };
+  uint4 av[AP];
+  float uv[UP];
+  auto load = [&](int m0) {
 #pragma unroll
-  for (int j = 0; j < RB; ++j) acc[j] = 0.0f;
-  const int64_t cl = c < cols ? c : 0;  // columns past the end read column 0 (never stored)
-  float* usf = reinterpret_cast<float*>(&us[0][0]);
-  for (int m0 = beg; m0 < end; m0 += kWgradRows) {
-    const int nr = min(kWgradRows, end - m0);
-    __syncthreads();  // the previous round's reads are done
-    for (int i = threadIdx.x; i < kWgradRows * RB; i += kWgradThreads) {
-      const int row = i / RB, j = i % RB;
-      usf[i] = (row < nr && j < r) ? u[int64_t(m0 + row) * r + j] : 0.0f;
-    }
-    __syncthreads();
-    for (int i0 = 0; i0 < nr; i0 += 8) {
-      float av[8];
+    for (int i = 0; i < AP; ++i) {
+      const int m = m0 + (tid >> 4) + 16 * i;
+      const uint16_t* row = a + row_of(min(m, end - 1)) * cols;
+      if (vec) {
+        av[i] = *reinterpret_cast<const uint4*>(row + (c0 + ac < cols ? c0 + ac : 0));
+      } else {
+        uint32_t w[4];
 #pragma unroll
-      for (int b = 0; b < 8; ++b) {  // the batch's loads go out together
-        const int m = m0 + min(i0 + b, nr - 1);
-        const int64_t row = gather_k > 0 ? static_cast<int64_t>(sorted_flat[m] / gather_k) : m;
-        av[b] = to_f<XDT>(a[row * cols + cl]);
+        for (int q = 0; q < 4; ++q) {
+          const int64_t ca = c0 + ac + 2 * q;
+          w[q] = pack2(row[ca < cols ? ca : 0], row[ca + 1 < cols ? ca + 1 : 0]);
+        }
+        av[i] = make_uint4(w[0], w[1], w[2], w[3]);
       }
+      if (m >= end) av[i] = make_uint4(0, 0, 0, 0);
+    }
+    // u value i of thread t: row (t + 256 i) / RB, rank (t + 256 i) % RB
 #pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        if (i0 + b < nr) {
-          const float4* ur = us[i0 + b];
+    for (int i = 0; i < UP; ++i) {
+      const int idx = tid + kWgradThreads * i, row = idx / RB, j = idx % RB;
+      const bool in = m0 + row < end && j < r;
+      const float v = u[int64_t(min(m0 + row, end - 1)) * r + (j < r ? j : 0)];
+      uv[i] = in ? v : 0.0f;
+    }
+  };
+  auto stage = [&]() {
 #pragma unroll
-          for (int q4 = 0; q4 < RB / 4; ++q4) {
-            const float4 uv = ur[q4];
-            acc[4 * q4] = __builtin_fmaf(uv.x, av[b], acc[4 * q4]);
-            acc[4 * q4 + 1] = __builtin_fmaf(uv.y, av[b], acc[4 * q4 + 1]);
-            acc[4 * q4 + 2] = __builtin_fmaf(uv.z, av[b], acc[4 * q4 + 2]);
-            acc[4 * q4 + 3] = __builtin_fmaf(uv.w, av[b], acc[4 * q4 + 3]);
+    for (int i = 0; i < AP; ++i)
+      *reinterpret_cast<uint4*>(&as[wgrad_at<kWgradCols>((tid >> 4) + 16 * i, ac)]) = av[i];
+#pragma unroll
+    for (int i = 0; i < UP; ++i) {
+      const int idx = tid + kWgradThreads * i, row = idx / RB, j = idx % RB;
+      const int at = wgrad_at<RB>(row, j & ~3) + (j & 3);
+      float v = uv[i];
+      us[0][at] = bf16_part(v);
+      us[1][at] = bf16_part(v);
+      us[2][at] = bf16_part(v);
+    }
+  };
+  // operand of a 32-row step: rows 32 s + 8 g .. + 7 of column base + lane % 16
+  auto operand = [&](const uint16_t* tile, auto cols_c, int s, int base) -> uint4 {
+    constexpr int COLS = decltype(cols_c)::value;
+    const int row = 32 * s + 8 * g + (l16 >> 2), col = base + 4 * (l16 & 3);
+    const uint2 lo = lds_read_tr(tile + wgrad_at<COLS>(row, col));
+    const uint2 hi = lds_read_tr(tile + wgrad_at<COLS>(row + 4, col));
+    return make_uint4(lo.x, lo.y, hi.x, hi.y);
+  };
+
+  f32x4_t acc[2][NSM];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int q = 0; q < NSM; ++q) acc[t][q] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  if (beg < end) load(beg);
+  for (int m0 = beg; m0 < end; m0 += kWgradRows) {
+    __syncthreads();  // the previous round's reads are done
+    stage();
+    __syncthreads();
+    if (m0 + kWgradRows < end) load(m0 + kWgradRows);
+#pragma unroll
+    for (int s = 0; s < kWgradRows / 32; ++s) {
+      uint4 ah[2], al[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        ah[t] = operand(as, std::integral_constant<int, kWgradCols>{}, s, 32 * wid + 16 * t);
+        if constexpr (XDT == E4B_FP16) {
+          const uint32_t w[4] = {ah[t].x, ah[t].y, ah[t].z, ah[t].w};
+          uint32_t h[4], l[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float v0 = lo_f<XDT>(w[i]), v1 = hi_f<XDT>(w[i]);
+            const uint16_t h0 = bf16_part(v0), h1 = bf16_part(v1);
+            h[i] = pack2(h0, h1);
+            l[i] = cvt_pair<E4B_BF16>(v0, v1);
           }
+          ah[t] = make_uint4(h[0], h[1], h[2], h[3]);
+          al[t] = make_uint4(l[0], l[1], l[2], l[3]);
         }
       }
+#pragma unroll
+      for (int q = 0; q < NSM; ++q)
+#pragma unroll
+        for (int part = 0; part < 3; ++part) {
+          const uint4 uo = operand(us[part], std::integral_constant<int, RB>{}, s, 16 * q);
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            acc[t][q] = mfma_16x16x32<E4B_BF16>(uo, ah[t], acc[t][q]);
+            if constexpr (XDT == E4B_FP16) acc[t][q] = mfma_16x16x32<E4B_BF16>(uo, al[t], acc[t][q]);
+          }
+        }
     }
   }
-  if (c >= cols) return;
+  // lane holds ranks 16 q + 4 g + i of column 32 wid + 16 t + lane % 16
+  auto put = [&](int64_t at, float v) {
+    if (odt == E4B_FP32) static_cast<float*>(out)[at] = v;
+    else static_cast<uint16_t*>(out)[at] = odt == E4B_BF16 ? from_f<E4B_BF16>(v) : from_f<E4B_FP16>(v);
+  };
 #pragma unroll
-  for (int j = 0; j < RB; ++j)
-    if (j < r) out[(int64_t(e) * r + j) * cols + c] = scale * acc[j];
+  for (int t = 0; t < 2; ++t) {
+    const int64_t c = c0 + 32 * wid + 16 * t + l16;
+#pragma unroll
+    for (int q = 0; q < NSM; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = 16 * q + 4 * g + i;
+        if (c < cols && j < r)
+          put(TRANS ? (int64_t(e) * cols + c) * r + j : (int64_t(e) * r + j) * cols + c, scale * acc[t][q][i]);
+      }
+  }
 }
 
 }  // namespace e4b

@@ -253,3 +253,29 @@ def test_training_lane_is_bit_identical_across_runs(n_tok, E_, top):
         assert torch.equal(dx, dx0), f"run {run}: dL/dx differs"
         for n in g0:
             assert torch.equal(grads[n], g0[n]), f"run {run}: dL/d{n} differs"
+
+
+@pytest.mark.parametrize("r,adt,top,cols", [(1, torch.bfloat16, 1, 8), (16, torch.float16, 2, 136), (17, torch.bfloat16, 3, 100),
+                                            (33, torch.float16, 2, 392), (64, torch.bfloat16, 4, 129)])
+def test_lora_wgrad_edges(r, adt, top, cols):
+    """Ranks and columns off the 16-rank and 128-column tiles, row counts around the 64-row rounds, rows
+    that are not whole 16-byte pieces, both 16-bit types. Products are exact and summed in fp32, so
+    2^-16 of the sum of magnitudes holds up to 256 rows (2^-24 each)."""
+    _announce(f"lora wgrad edges r={r} {adt} cols={cols}")
+    sizes = [63, 0, 64, 65, 1, 128, 200]
+    E_ = len(sizes)
+    rb = ops._routing_from_sizes(sizes, list(range(E_)), E_, DEV)[0]
+    M = sum(sizes)
+    g_ = torch.Generator(device=DEV).manual_seed(12)
+    u = torch.randn(M, r, generator=g_, device=DEV) * torch.logspace(-6, 6, M, device=DEV).unsqueeze(1)
+    a = torch.randn(M, cols, generator=g_, device=DEV).to(adt)
+    got = ops.lora_wgrad(u, a, rb, M, E_, 0.5).double()
+    at = 0
+    for e, s in enumerate(sizes):
+        ue, ae = u[at:at + s].double(), a[at:at + s].double()
+        want, bound = 0.5 * ue.T @ ae, 0.5 * ue.abs().T @ ae.abs()
+        assert torch.all((got[e] - want).abs() <= bound * 2.0 ** -16 + 1e-30), e
+        at += s
+    u[70, 0] = float("inf")  # expert 2's alone
+    got = ops.lora_wgrad(u, a, rb, M, E_, 0.5)
+    assert not got[2, 0].isfinite().any() and got[[0, 1, 3, 4, 5, 6]].isfinite().all()
