@@ -53,6 +53,10 @@ EXPORTS = (
     "e4b_moe_lora_workspace_bytes",
     "e4b_moe_lora_forward",
     "e4b_set_probe",
+    "e4b_train_saved_bytes",
+    "e4b_train_workspace_bytes",
+    "e4b_train_forward",
+    "e4b_train_backward",
 )
 
 
@@ -173,6 +177,15 @@ def _bind(L):
     L.e4b_moe_lora_forward.restype = ctypes.c_int
     L.e4b_moe_lora_forward.argtypes = [P, I32, I64, P, P, I32, I32, QW, QW, ctypes.POINTER(Lora), I32, F32, I32, P,
                                        ctypes.c_size_t, P, I32, P]
+    Z, LO = ctypes.c_size_t, ctypes.POINTER(Lora)
+    L.e4b_train_saved_bytes.restype = Z
+    L.e4b_train_saved_bytes.argtypes = [I64, I32, I32, I64, I64, I32, I32]
+    L.e4b_train_workspace_bytes.restype = Z
+    L.e4b_train_workspace_bytes.argtypes = [I64, I32, I32, I64, I64, I32, I32, I32]
+    L.e4b_train_forward.restype = ctypes.c_int
+    L.e4b_train_forward.argtypes = [P, I64, P, P, I32, I32, QW, QW, LO, I32, F32, P, Z, P, Z, P, I32, P]
+    L.e4b_train_backward.restype = ctypes.c_int
+    L.e4b_train_backward.argtypes = [P, I32, P, I64, P, I32, I32, QW, QW, LO, I32, F32, P, Z, P, Z, P, P, P, P, P, P, P]
     L.e4b_set_probe.restype = ctypes.c_int
     L.e4b_set_probe.argtypes = [I32, P, P]
     return L

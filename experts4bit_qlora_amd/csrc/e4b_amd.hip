@@ -28,6 +28,7 @@
 #include "route.h"
 #include "scale.h"
 #include "train.h"
+#include "train_layer.h"
 
 namespace {
 
@@ -308,6 +309,8 @@ int launch_gemm_dt(const e4b::GemmArgs& a, bool gemv, int64_t max_active, hipStr
   return check_launch(gemv ? "gemv_kernel" : "gemm_mfma_kernel");
 }
 
+using e4b::kUnitWeights;
+
 template <int DDT, int WDT, bool SC>
 void launch_combine_w(const void* down, const int32_t* inv, const void* w, int64_t T, int k, int64_t H,
                       void* out, int od, const e4b::CombineScale& cs, hipStream_t s) {
@@ -333,6 +336,9 @@ template <int DDT, bool SC = false>
 void launch_combine_dt(const void* down, const int32_t* inv, const void* w, int wd, int64_t T, int k, int64_t H,
                        void* out, int od, hipStream_t s, const e4b::CombineScale& cs = {}) {
   switch (wd) {
+    case kUnitWeights:
+      if constexpr (DDT == E4B_FP32) launch_combine_w<DDT, kUnitWeights, SC>(down, inv, w, T, k, H, out, od, cs, s);
+      break;
     case E4B_FP32: launch_combine_w<DDT, E4B_FP32, SC>(down, inv, w, T, k, H, out, od, cs, s); break;
     case E4B_BF16: launch_combine_w<DDT, E4B_BF16, SC>(down, inv, w, T, k, H, out, od, cs, s); break;
     default: launch_combine_w<DDT, E4B_FP16, SC>(down, inv, w, T, k, H, out, od, cs, s); break;
@@ -629,7 +635,7 @@ static int grouped_gemm_impl(const void* a, int32_t act_dtype, int32_t gather_k,
     return fail(E4B_EINVAL, "the fp16 matrix-core mode needs the MFMA path, bf16 activations and NF4 weight shifts");
   args.a_exp = a_exp;
   if (out_f16_shift && (!f16c || out_dtype != E4B_FP32 || epilogue != E4B_EPI_NONE || w->bias || lora ||
-                        !e4b::lora_gemm_fits(rt->tile_m, w->k)))
+                        !e4b::f16_rows_fit(rt->tile_m, w->k)))
     return fail(E4B_EINVAL, "fp16 down rows need the fp16 mode over 256-row tiles or 32-row tiles with k %% 256 == "
                             "0, fp32 rows, and no epilogue, bias or LoRA");
   args.out_f16_shift = out_f16_shift;
@@ -639,8 +645,8 @@ static int grouped_gemm_impl(const void* a, int32_t act_dtype, int32_t gather_k,
   args.lr = 0;
   args.lscale = 0.0f;
   if (lora) {
-    if (!f16c || !e4b::lora_gemm_fits(rt->tile_m, w->k))
-      return fail(E4B_EINVAL, "the LoRA epilogue needs the fp16 mode over 256-row tiles or 32-row tiles with k %% 256 == 0");
+    if (!f16c || !e4b::lora_gemm_fits(rt->tile_m))
+      return fail(E4B_EINVAL, "the LoRA delta needs the fp16 mode over 256-row or 32-row tiles");
     args.lt = lora->t;
     args.lb = lora->b;
     args.lbdt = lora->dtype;
@@ -757,6 +763,28 @@ int lora_b_pass(const float* t_workspace, const e4b_routing* rt, int64_t M, int3
   return check_launch("lora kernels");
 }
 
+extern "C++" {
+// out [E, rank, cols] (TRANS: [E, cols, rank]) in odt; every expert's block writes its part (zeros for
+// an expert without rows).
+template <bool TRANS>
+int lora_wgrad(const float* u, int rank, const void* a, int a_dtype, int gather_k, const e4b_routing* rt,
+               int num_experts, int64_t cols, float scale, void* out, int odt, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>(cdiv(cols, e4b::kWgradCols)), static_cast<unsigned>(num_experts));
+#define E4B_WG(XD, RB)                                                                                            \
+  hipLaunchKernelGGL((e4b::lora_wgrad_kernel<XD, RB, TRANS>), grid, dim3(e4b::kWgradThreads), 0, stream, u, rank, \
+                     static_cast<const uint16_t*>(a), gather_k, rt->sorted_flat, rt->offsets, cols, scale, out, odt)
+#define E4B_WG_R(XD)                                     \
+  if (rank <= 16) E4B_WG(XD, 16);                        \
+  else if (rank <= 32) E4B_WG(XD, 32);                   \
+  else E4B_WG(XD, e4b::kLoraMaxRank);
+  if (a_dtype == E4B_BF16) { E4B_WG_R(E4B_BF16) }
+  else { E4B_WG_R(E4B_FP16) }
+#undef E4B_WG_R
+#undef E4B_WG
+  return check_launch("lora_wgrad_kernel");
+}
+}  // extern "C++"
+
 }  // namespace
 
 int e4b_lora_delta(const void* x, int32_t x_dtype, int32_t gather_k, const e4b_routing* rt, int64_t M,
@@ -804,21 +832,7 @@ int e4b_lora_wgrad(const float* u, int32_t rank, const void* a, int32_t a_dtype,
   if (!rt || !rt->offsets || (gather_k > 0 && !rt->sorted_flat)) return fail(E4B_EINVAL, "routing offsets / order are NULL");
   if (!out || (M > 0 && (!u || !a))) return fail(E4B_EINVAL, "NULL pointer");
   if (cdiv(cols, e4b::kWgradCols) > 0x7fffffffLL) return fail(E4B_EUNSUPPORTED, "too many columns");
-  // every expert's block writes its rows of out (zeros for an expert without rows)
-  const dim3 grid(static_cast<unsigned>(cdiv(cols, e4b::kWgradCols)), static_cast<unsigned>(num_experts));
-#define E4B_WG(XD, RB)                                                                                            \
-  hipLaunchKernelGGL((e4b::lora_wgrad_kernel<XD, RB, false>), grid, dim3(e4b::kWgradThreads), 0, stream, u, rank, \
-                     static_cast<const uint16_t*>(a), gather_k, rt->sorted_flat, rt->offsets, cols, scale, out,   \
-                     E4B_FP32)
-#define E4B_WG_R(XD)                                     \
-  if (rank <= 16) E4B_WG(XD, 16);                        \
-  else if (rank <= 32) E4B_WG(XD, 32);                   \
-  else E4B_WG(XD, e4b::kLoraMaxRank);
-  if (a_dtype == E4B_BF16) { E4B_WG_R(E4B_BF16) }
-  else { E4B_WG_R(E4B_FP16) }
-#undef E4B_WG_R
-#undef E4B_WG
-  return check_launch("lora_wgrad_kernel");
+  return lora_wgrad<false>(u, rank, a, a_dtype, gather_k, rt, num_experts, cols, scale, out, E4B_FP32, stream);
 }
 
 int e4b_grouped_dgrad(const void* grad, int32_t grad_dtype, const e4b_qweight* w, const e4b_routing* rt, int64_t M,
@@ -1121,7 +1135,7 @@ static int moe_forward_impl(const void* hidden, int32_t act_dtype, int64_t token
   // fp32 rows, written once and read once by the combine. (Mid-size batches keep fp32 rows: their
   // rows are few, and the combine's scale lookups cost more than the bytes saved.)
   int f16_shift = 0;
-  if (f16c && split && e4b::lora_gemm_fits(e4b::kTileMSmall, w2->k)) {
+  if (f16c && split && e4b::f16_rows_fit(e4b::kTileMSmall, w2->k)) {
     int lg = 0;
     while ((int64_t(1) << lg) < w2->k) ++lg;
     f16_shift = 16 + lg;
@@ -1207,12 +1221,11 @@ namespace {
 
 // Whether the grouped LoRA forward runs in the fp16 mode with the deltas in the GEMM epilogues.
 bool lora_fused_ok(int32_t act_dtype, const e4b_qweight* w1, const e4b_qweight* w2) {
-  return act_dtype == E4B_BF16 && w1->format != E4B_FMT_MXFP4 && w1->shift && w2->shift &&
-         e4b::lora_gemm_fits(e4b::kTileMSmall, w1->k) && e4b::lora_gemm_fits(e4b::kTileMSmall, w2->k);
+  return act_dtype == E4B_BF16 && w1->format != E4B_FMT_MXFP4 && w1->shift && w2->shift;
 }
 
-// t = x . A^T for the sorted rows of rt's tiles on the matrix cores (bf16 x, in a multiple of 64,
-// which the narrow kernel's k limit of that path implies): 64-row parts of 128-row tiles, whole
+// t = x . A^T for the sorted rows of rt's tiles on the matrix cores (bf16 x, in a multiple of 64, as
+// every k is): 64-row parts of 128-row tiles, whole
 // 32-row tiles, the ranks in 16-rank blocks.
 int lora_t_mfma(const void* x, int32_t gather_k, const e4b_routing& rt, const void* A, int32_t adt, int rank,
                 int64_t in, float* t, hipStream_t stream) {
@@ -1417,8 +1430,7 @@ int e4b_moe_lora_forward(const void* hidden, int32_t act_dtype, int64_t tokens, 
   }
 
   // Grouped path in the fp16 matrix-core mode with each delta inside its GEMM's epilogue (bf16
-  // activations, NF4 weights carrying shifts, both projections' k taken by the 32-row narrow
-  // kernel): t1 = x . A1^T; gate_up GEMM + lscale t1 . B1^T + epilogue -> h; t2 = h . A2^T; h as
+  // activations, NF4 weights carrying shifts): t1 = x . A1^T; gate_up GEMM + lscale t1 . B1^T + epilogue -> h; t2 = h . A2^T; h as
   // scaled fp16 rows; down GEMM + lscale t2 . B2^T -> fp32 rows; combine. No fp32 gate_up rows
   // and no pass over the down rows: the deltas ride the GEMM tiles' accumulators.
   const bool gemv_path = flags == E4B_PATH_GEMV || (flags == E4B_PATH_AUTO && tokens <= 4);
@@ -1549,6 +1561,345 @@ int e4b_moe_forward_noalloc(const void* hidden, int32_t act_dtype, int64_t token
   if (rc) return rc;
   return moe_forward_impl(hidden, act_dtype, tokens, top_k_index, top_k_weights, weight_dtype, top_k, w1, w2, epilogue,
                           alpha, limit, flags, ws, size_t(E4B_NOALLOC_WORKSPACE_BYTES), out, out_dtype, stream, false);
+}
+
+}  // extern "C"
+
+// ------------------------------------------------------------------------- training layer
+
+namespace {
+
+struct TrainShape {
+  int64_t tokens, M, H, I, n1;
+  int E, k, r;
+  bool split;
+};
+TrainShape train_shape(int64_t tokens, int32_t top_k, int E, int64_t n1, int64_t n2, int32_t epilogue, int32_t rank) {
+  TrainShape s{};
+  s.tokens = tokens;
+  s.M = tokens * top_k;
+  s.H = n2;
+  s.I = is_gated_epi(epilogue) ? n1 / 2 : n1;
+  s.n1 = n1;
+  s.E = E;
+  s.k = top_k;
+  s.r = std::max(rank, 1);
+  s.split = mfma_tile_for(s.M, E) == e4b::kTileM;  // 256-row tiles plus 32-row tails, as the fused forward
+  return s;
+}
+
+// What the forward leaves for the backward, carved from one buffer (p may be NULL: the size alone).
+struct TrainSaved {
+  e4b_routing rt, rbig, rsmall;
+  uint16_t *proj, *h, *down;  // bf16 rows [M, n1], [M, I], [M, H]
+  float *t1, *t2;             // [M, r]
+  size_t bytes;
+};
+TrainSaved carve_saved(char* p, const TrainShape& s) {
+  TrainSaved v{};
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    char* q = p ? p + off : nullptr;
+    off += align256(bytes);
+    return q;
+  };
+  auto ints = [&](int64_t n) { return reinterpret_cast<int32_t*>(take(sizeof(int32_t) * n)); };
+  auto tiles = [&](e4b_routing& r, int tile_m, int64_t max_tiles) {
+    r.tile_m = tile_m;
+    r.max_tiles = static_cast<int32_t>(max_tiles);
+    r.tiles = ints(2 * max_tiles);
+    r.meta = ints(4);
+  };
+  v.rt.sorted_flat = ints(s.M);
+  v.rt.inv = ints(s.M);
+  v.rt.offsets = ints(s.E + 1);
+  v.rt.active = ints(s.E);
+  const int tm = mfma_tile_for(s.M, s.E);
+  tiles(v.rt, tm, max_tiles_for(s.M, s.E, tm));
+  v.rbig = v.rsmall = v.rt;
+  if (s.split) {
+    tiles(v.rbig, e4b::kTileMBig, max_tiles_for(s.M, s.E, e4b::kTileMBig));
+    tiles(v.rsmall, e4b::kTileMSmall, max_small_tiles(s.M, s.E));
+  }
+  v.proj = reinterpret_cast<uint16_t*>(take(sizeof(uint16_t) * s.M * s.n1));
+  v.h = reinterpret_cast<uint16_t*>(take(sizeof(uint16_t) * s.M * s.I));
+  v.down = reinterpret_cast<uint16_t*>(take(sizeof(uint16_t) * s.M * s.H));
+  v.t1 = reinterpret_cast<float*>(take(sizeof(float) * s.M * s.r));
+  v.t2 = reinterpret_cast<float*>(take(sizeof(float) * s.M * s.r));
+  v.bytes = off;
+  return v;
+}
+
+// Scratch of either direction: the rows that both GEMMs of it read as scaled fp16 and their exponents,
+// and in the backward the gradient rows between its stages.
+struct TrainWork {
+  int32_t *scratch, *xexp, *rexp;  // forward: routing scratch, token and h exponents
+  uint16_t *x16, *r16;
+  uint16_t *d, *d16, *dh, *dp, *dp16;  // backward: down, h and proj gradient rows
+  int32_t *dexp, *pexp;
+  float *u, *da;                       // [M, r]; [M, H] fp32
+  size_t bytes;
+};
+TrainWork carve_work(char* p, const TrainShape& s, bool backward) {
+  TrainWork v{};
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    char* q = p ? p + off : nullptr;
+    off += align256(bytes);
+    return q;
+  };
+  auto ints = [&](int64_t n) { return reinterpret_cast<int32_t*>(take(sizeof(int32_t) * n)); };
+  auto rows = [&](int64_t n, int64_t c) { return reinterpret_cast<uint16_t*>(take(sizeof(uint16_t) * n * c)); };
+  if (!backward) {
+    v.scratch = ints(e4b_route_scratch_ints(s.M, s.E));
+    v.xexp = ints(s.tokens);
+    v.rexp = ints(s.M);
+    v.x16 = rows(s.tokens, s.H);
+    v.r16 = rows(s.M, s.I);
+  } else {
+    v.dexp = ints(s.M);
+    v.pexp = ints(s.M);
+    v.u = reinterpret_cast<float*>(take(sizeof(float) * s.M * s.r));
+    v.dh = rows(s.M, s.I);
+    v.dp = rows(s.M, s.n1);
+    v.dp16 = rows(s.M, s.n1);
+    // the down gradient rows are done with before the token gradient's fp32 rows are written
+    v.d = rows(s.M, s.H);
+    v.d16 = rows(s.M, s.H);
+    v.da = reinterpret_cast<float*>(v.d);
+  }
+  v.bytes = off;
+  return v;
+}
+
+template <class F>
+void by_row_pieces(int64_t cols, F&& f) {
+  switch (e4b::row_exp_pieces(cols)) {
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    default: f(std::integral_constant<int, 8>{}); break;
+  }
+}
+dim3 row_grid(int64_t rows) { return dim3(static_cast<unsigned>(cdiv(rows, e4b::kRowThreads / e4b::kWave))); }
+
+int lora_u_mfma(const uint16_t* g, const e4b_routing& rt, const void* B, int bdt, int rank, int64_t n, float* u,
+                hipStream_t stream) {
+  const int bm = rt.tile_m % 64 == 0 ? 64 : 32;
+  const int64_t blocks = int64_t(rt.max_tiles) * (rt.tile_m / bm);
+  if (blocks > 0x7fffffffLL) return fail(E4B_EUNSUPPORTED, "LoRA u grid too large");
+  const dim3 grid(static_cast<unsigned>(blocks));
+  const int nsm = rank <= 16 ? 1 : (rank <= 32 ? 2 : 4);
+#define E4B_UM(AD, BM, NS)                                                                                     \
+  if (bdt == AD && bm == BM && nsm == NS)                                                                     \
+    hipLaunchKernelGGL((e4b::lora_u_mfma_kernel<AD, BM, NS>), grid, dim3(BM / 16 * e4b::kWave), 0, stream, g, rt, B, \
+                       rank, n, u);
+#define E4B_UM_AD(AD) E4B_UM(AD, 64, 1) E4B_UM(AD, 64, 2) E4B_UM(AD, 64, 4) E4B_UM(AD, 32, 1) E4B_UM(AD, 32, 2) \
+  E4B_UM(AD, 32, 4)
+  E4B_UM_AD(E4B_BF16) E4B_UM_AD(E4B_FP16) E4B_UM_AD(E4B_FP32)
+#undef E4B_UM_AD
+#undef E4B_UM
+  return check_launch("lora_u_mfma_kernel");
+}
+
+// One tile list of the input gradient: 256-row tiles on the wide kernel, 32-row tiles on the narrow one.
+int dgrad16(const e4b::Dgrad16Args& base, const e4b_routing* rt, hipStream_t s) {
+  e4b::Dgrad16Args a = base;
+  a.rt = *rt;
+  const int64_t grid = e4b::kXcds * cdiv(rt->max_tiles, e4b::kXcds) * cdiv(a.w.k, e4b::kDgradCols);
+  if (grid > 0x7fffffffLL) return fail(E4B_EUNSUPPORTED, "dgrad grid too large");
+  const dim3 g(static_cast<unsigned>(grid));
+  const bool wide = rt->tile_m == e4b::kTileMBig, dq = a.w.format == E4B_FMT_NF4_DQ;
+  if (wide && dq) hipLaunchKernelGGL(e4b::dgrad_wide_kernel<E4B_FMT_NF4_DQ>, g, dim3(e4b::kDgradWideThreads), 0, s, a);
+  else if (wide) hipLaunchKernelGGL(e4b::dgrad_wide_kernel<E4B_FMT_NF4>, g, dim3(e4b::kDgradWideThreads), 0, s, a);
+  else if (dq) hipLaunchKernelGGL(e4b::dgrad_narrow_kernel<E4B_FMT_NF4_DQ>, g, dim3(e4b::kDgradNarrowThreads), 0, s, a);
+  else hipLaunchKernelGGL(e4b::dgrad_narrow_kernel<E4B_FMT_NF4>, g, dim3(e4b::kDgradNarrowThreads), 0, s, a);
+  return check_launch("dgrad kernels");
+}
+
+// The arguments both directions share.
+int check_train(int64_t tokens, int32_t top_k, const e4b_qweight* w1, const e4b_qweight* w2, const e4b_lora* lora,
+                int32_t epilogue, int32_t weight_dtype) {
+  int rc = check_weight(w1);
+  if (rc) return rc;
+  rc = check_weight(w2);
+  if (rc) return rc;
+  if (!lora) return fail(E4B_EINVAL, "lora is NULL");
+  if (w1->num_experts != w2->num_experts || w1->format != w2->format) return fail(E4B_EINVAL, "w1 and w2 do not match");
+  if (w1->format == E4B_FMT_MXFP4 || !w1->shift || !w2->shift)
+    return fail(E4B_EUNSUPPORTED, "the training layer takes NF4 weights with their shifts");
+  const bool pair = epilogue == E4B_EPI_SWIGLU || epilogue == E4B_EPI_CLAMP_SWIGLU;
+  if (!pair && epilogue != E4B_EPI_ACT) return fail(E4B_EUNSUPPORTED, "epilogue %d: SWIGLU, CLAMP_SWIGLU or ACT", epilogue);
+  if (w1->bias || w2->bias) return fail(E4B_EUNSUPPORTED, "the training layer takes no biases");
+  if ((pair ? w1->n / 2 : w1->n) != w2->k || (pair && w1->n % 2) || w1->k != w2->n)
+    return fail(E4B_EINVAL, "w1 [%lld, %lld] and w2 [%lld, %lld] do not chain", (long long)w1->n, (long long)w1->k,
+                (long long)w2->n, (long long)w2->k);
+  if (w1->n % 64 || w2->n % 64) return fail(E4B_EUNSUPPORTED, "output features must be multiples of 64");
+  if (lora->rank <= 0 || lora->rank > e4b::kLoraMaxRank)
+    return fail(E4B_EUNSUPPORTED, "rank=%d outside [1, %d]", lora->rank, e4b::kLoraMaxRank);
+  if (!any_dtype_ok(lora->dtype) || !any_dtype_ok(weight_dtype)) return fail(E4B_EINVAL, "bad adapter or weight dtype");
+  if (!lora->a1 || !lora->b1 || !lora->a2 || !lora->b2) return fail(E4B_EINVAL, "NULL adapter");
+  if (!aligned16(lora->a1) || !aligned16(lora->a2)) return fail(E4B_EINVAL, "the A matrices must be 16-byte aligned");
+  if (tokens < 0 || top_k <= 0) return fail(E4B_EINVAL, "bad tokens/top_k");
+  if (tokens * top_k > 0x7fffffffLL) return fail(E4B_EUNSUPPORTED, "more than 2^31 - 1 routed rows");
+  if (w1->num_experts > e4b::kRouteMaxExperts) return fail(E4B_EUNSUPPORTED, "too many experts");
+  return E4B_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t e4b_train_saved_bytes(int64_t tokens, int32_t top_k, int32_t num_experts, int64_t n1, int64_t n2,
+                             int32_t epilogue, int32_t rank) {
+  return carve_saved(nullptr, train_shape(tokens, top_k, num_experts, n1, n2, epilogue, rank)).bytes;
+}
+
+size_t e4b_train_workspace_bytes(int64_t tokens, int32_t top_k, int32_t num_experts, int64_t n1, int64_t n2,
+                                 int32_t epilogue, int32_t rank, int32_t backward) {
+  return carve_work(nullptr, train_shape(tokens, top_k, num_experts, n1, n2, epilogue, rank), backward != 0).bytes;
+}
+
+int e4b_train_forward(const void* hidden, int64_t tokens, const int64_t* top_k_index, const void* top_k_weights,
+                      int32_t weight_dtype, int32_t top_k, const e4b_qweight* w1, const e4b_qweight* w2,
+                      const e4b_lora* lora, int32_t epilogue, float limit, void* saved, size_t saved_bytes,
+                      void* workspace, size_t workspace_bytes, void* out, int32_t out_dtype, hipStream_t stream) {
+  int rc = check_train(tokens, top_k, w1, w2, lora, epilogue, weight_dtype);
+  if (rc) return rc;
+  if (!any_dtype_ok(out_dtype)) return fail(E4B_EINVAL, "bad out dtype");
+  if (tokens == 0) return E4B_OK;
+  const TrainShape sh = train_shape(tokens, top_k, w1->num_experts, w1->n, w2->n, epilogue, lora->rank);
+  if (!hidden || !top_k_index || !top_k_weights || !out || !saved || !workspace) return fail(E4B_EINVAL, "NULL pointer");
+  if (!aligned16(hidden) || !aligned16(saved) || !aligned16(workspace))
+    return fail(E4B_EINVAL, "hidden, saved and workspace must be 16-byte aligned");
+  TrainSaved sv = carve_saved(static_cast<char*>(saved), sh);
+  const TrainWork wk = carve_work(static_cast<char*>(workspace), sh, false);
+  if (saved_bytes < sv.bytes || workspace_bytes < wk.bytes)
+    return fail(E4B_ESPACE, "saved %zu / workspace %zu bytes < %zu / %zu needed", saved_bytes, workspace_bytes, sv.bytes,
+                wk.bytes);
+  sv.rt.scratch = wk.scratch;
+  const RowExpArgs rx{static_cast<const uint16_t*>(hidden), w1->k, wk.xexp, wk.x16};
+  rc = route_impl(top_k_index, tokens, top_k, sh.E, &sv.rt, &rx, stream,
+                  e4b::SplitTiles{sv.rbig, sv.rsmall, sh.split ? 1 : 0});
+  if (rc) return rc;
+  SideLease lease(stream, sh.split);
+  auto tiles = [&](int site, auto&& launch) {
+    return sh.split ? run_tile_heights(lease.get(), stream, &sv.rbig, &sv.rsmall, site, launch) : launch(&sv.rt, stream);
+  };
+  rc = lora_t_mfma(hidden, top_k, sv.rt, lora->a1, lora->dtype, sh.r, w1->k, sv.t1, stream);
+  if (rc) return rc;
+  const LoraEpi l1{sv.t1, lora->b1, lora->dtype, sh.r, lora->scaling};
+  rc = tiles(E4B_PROBE_GATE_UP_BIG, [&](const e4b_routing* r, hipStream_t s) {
+    return grouped_gemm_impl(wk.x16, E4B_BF16, top_k, w1, r, tokens, sh.M, E4B_EPI_NONE, 1.0f, 0.0f, E4B_PATH_MFMA,
+                             sv.proj, E4B_BF16, wk.xexp, s, &l1);
+  });
+  if (rc) return rc;
+  by_row_pieces(sh.I, [&](auto rp) {
+    constexpr int RP = decltype(rp)::value;
+    if (is_gated_epi(epilogue))
+      hipLaunchKernelGGL((e4b::train_act_kernel<true, RP>), row_grid(sh.M), dim3(e4b::kRowThreads), 0, stream, sv.proj,
+                         sv.rt.offsets, sh.E, sh.I, epilogue, limit, sv.h, wk.r16, wk.rexp);
+    else
+      hipLaunchKernelGGL((e4b::train_act_kernel<false, RP>), row_grid(sh.M), dim3(e4b::kRowThreads), 0, stream, sv.proj,
+                         sv.rt.offsets, sh.E, sh.I, epilogue, limit, sv.h, wk.r16, wk.rexp);
+  });
+  rc = check_launch("train_act_kernel");
+  if (rc) return rc;
+  rc = lora_t_mfma(sv.h, 0, sv.rt, lora->a2, lora->dtype, sh.r, w2->k, sv.t2, stream);
+  if (rc) return rc;
+  const LoraEpi l2{sv.t2, lora->b2, lora->dtype, sh.r, lora->scaling};
+  rc = tiles(E4B_PROBE_DOWN_BIG, [&](const e4b_routing* r, hipStream_t s) {
+    return grouped_gemm_impl(wk.r16, E4B_BF16, 0, w2, r, tokens, sh.M, E4B_EPI_NONE, 1.0f, 0.0f, E4B_PATH_MFMA, sv.down,
+                             E4B_BF16, wk.rexp, s, &l2);
+  });
+  if (rc) return rc;
+  return e4b_combine(sv.down, E4B_BF16, sv.rt.inv, top_k_weights, weight_dtype, tokens, top_k, sh.H, out, out_dtype,
+                     stream);
+}
+
+int e4b_train_backward(const void* grad_out, int32_t grad_dtype, const void* hidden, int64_t tokens,
+                       const void* top_k_weights, int32_t weight_dtype, int32_t top_k, const e4b_qweight* w1,
+                       const e4b_qweight* w2, const e4b_lora* lora, int32_t epilogue, float limit, const void* saved,
+                       size_t saved_bytes, void* workspace, size_t workspace_bytes, void* grad_hidden,
+                       void* grad_weights, void* grad_a1, void* grad_b1, void* grad_a2, void* grad_b2,
+                       hipStream_t stream) {
+  int rc = check_train(tokens, top_k, w1, w2, lora, epilogue, weight_dtype);
+  if (rc) return rc;
+  if (!any_dtype_ok(grad_dtype)) return fail(E4B_EINVAL, "bad gradient dtype");
+  if (tokens == 0) return E4B_OK;
+  const TrainShape sh = train_shape(tokens, top_k, w1->num_experts, w1->n, w2->n, epilogue, lora->rank);
+  if (!grad_out || !hidden || !top_k_weights || !saved || !workspace) return fail(E4B_EINVAL, "NULL pointer");
+  if (!aligned16(grad_out) || !aligned16(hidden) || !aligned16(saved) || !aligned16(workspace))
+    return fail(E4B_EINVAL, "grad_out, hidden, saved and workspace must be 16-byte aligned");
+  const TrainSaved sv = carve_saved(static_cast<char*>(const_cast<void*>(saved)), sh);
+  const TrainWork wk = carve_work(static_cast<char*>(workspace), sh, true);
+  if (saved_bytes < sv.bytes || workspace_bytes < wk.bytes)
+    return fail(E4B_ESPACE, "saved %zu / workspace %zu bytes < %zu / %zu needed", saved_bytes, workspace_bytes, sv.bytes,
+                wk.bytes);
+  SideLease lease(stream, sh.split);
+  auto dgrad = [&](e4b::Dgrad16Args a) {
+    auto launch = [&](const e4b_routing* r, hipStream_t s) { return dgrad16(a, r, s); };
+    return sh.split ? run_tile_heights(lease.get(), stream, &sv.rbig, &sv.rsmall, E4B_PROBE_OFF - 2, launch)
+                    : launch(&sv.rt, stream);
+  };
+  // dL/ddown rows and the router weights' gradients
+  by_row_pieces(sh.H, [&](auto rp) {
+    constexpr int RP = decltype(rp)::value;
+#define E4B_CB(GD)                                                                                                   \
+  hipLaunchKernelGGL((e4b::combine_bwd_kernel<GD, RP>), row_grid(sh.M), dim3(e4b::kRowThreads), 0, stream, grad_out, \
+                     sv.down, sv.rt.inv, top_k_weights, weight_dtype, sh.M, top_k, sh.H, wk.d, wk.d16, wk.dexp,      \
+                     grad_weights)
+    if (grad_dtype == E4B_BF16) E4B_CB(E4B_BF16);
+    else if (grad_dtype == E4B_FP16) E4B_CB(E4B_FP16);
+    else E4B_CB(E4B_FP32);
+#undef E4B_CB
+  });
+  rc = check_launch("combine_bwd_kernel");
+  if (rc) return rc;
+  // the down projection: u2 = d . B2, its adapter gradients, dL/dh
+  const float s = lora->scaling;
+  rc = lora_u_mfma(wk.d, sv.rt, lora->b2, lora->dtype, sh.r, sh.H, wk.u, stream);
+  if (rc) return rc;
+  if (grad_a2) {
+    rc = lora_wgrad<false>(wk.u, sh.r, sv.h, E4B_BF16, 0, &sv.rt, sh.E, sh.I, s, grad_a2, lora->dtype, stream);
+    if (rc) return rc;
+  }
+  if (grad_b2) {
+    rc = lora_wgrad<true>(sv.t2, sh.r, wk.d, E4B_BF16, 0, &sv.rt, sh.E, sh.H, s, grad_b2, lora->dtype, stream);
+    if (rc) return rc;
+  }
+  if (!grad_hidden && !grad_a1 && !grad_b1) return E4B_OK;
+  rc = dgrad({wk.d16, wk.dexp, *w2, sv.rt, wk.u, lora->a2, lora->dtype, sh.r, s, wk.dh, 0});
+  if (rc) return rc;
+  by_row_pieces(sh.n1, [&](auto rp) {
+    constexpr int RP = decltype(rp)::value;
+    if (is_gated_epi(epilogue))
+      hipLaunchKernelGGL((e4b::train_act_bwd_kernel<true, RP>), row_grid(sh.M), dim3(e4b::kRowThreads), 0, stream, wk.dh,
+                         sv.proj, sv.rt.offsets, sh.E, sh.I, epilogue, limit, wk.dp, wk.dp16, wk.pexp);
+    else
+      hipLaunchKernelGGL((e4b::train_act_bwd_kernel<false, RP>), row_grid(sh.M), dim3(e4b::kRowThreads), 0, stream, wk.dh,
+                         sv.proj, sv.rt.offsets, sh.E, sh.I, epilogue, limit, wk.dp, wk.dp16, wk.pexp);
+  });
+  rc = check_launch("train_act_bwd_kernel");
+  if (rc) return rc;
+  // the gate_up projection
+  if (grad_b1) {
+    rc = lora_wgrad<true>(sv.t1, sh.r, wk.dp, E4B_BF16, 0, &sv.rt, sh.E, sh.n1, s, grad_b1, lora->dtype, stream);
+    if (rc) return rc;
+  }
+  if (!grad_hidden && !grad_a1) return E4B_OK;
+  rc = lora_u_mfma(wk.dp, sv.rt, lora->b1, lora->dtype, sh.r, sh.n1, wk.u, stream);
+  if (rc) return rc;
+  if (grad_a1) {
+    rc = lora_wgrad<false>(wk.u, sh.r, hidden, E4B_BF16, top_k, &sv.rt, sh.E, sh.H, s, grad_a1, lora->dtype, stream);
+    if (rc) return rc;
+  }
+  if (!grad_hidden) return E4B_OK;
+  rc = dgrad({wk.dp16, wk.pexp, *w1, sv.rt, wk.u, lora->a1, lora->dtype, sh.r, s, wk.da, 1});
+  if (rc) return rc;
+  // a token's gradient: its routed rows summed in slot order
+  launch_combine_dt<E4B_FP32>(wk.da, sv.rt.inv, nullptr, kUnitWeights, tokens, top_k, sh.H, grad_hidden, E4B_BF16, stream);
+  return check_launch("combine_kernel");
 }
 
 }  // extern "C"

@@ -303,10 +303,16 @@ E4B_DEV uint32_t pk_mul_f16(uint32_t a, uint32_t b) {
 constexpr int gemm_tile_nw(int bm) { return bm >= kTileM ? kTileNWWide : kTileNW; }
 constexpr int gemm_threads(int bm) { return bm == kTileM ? 512 : 256; }
 
+template <int MS, int NS, class AS>
+E4B_DEV void lora_delta_16x16(const GemmArgs& p, f32x4_t (&acc)[MS][NS], int e, int64_t arow0, int64_t arow_last,
+                              AS&& ashift, int bshift, const int64_t (&brow)[NS], int lane);  // lora_mfma.h
+
 // F16C: fp16 mode, the A rows already stored as scaled fp16 by row_exp_kernel; else the
 // operands are in the activation dtype.
-template <int DT, int FMT, int BM, bool F16C = false>
+// LORA (fp16 mode): the accumulators start as the tile's LoRA delta (lora_mfma.h).
+template <int DT, int FMT, int BM, bool F16C = false, bool LORA = false>
 __global__ void __launch_bounds__(gemm_threads(BM)) gemm_mfma_kernel(GemmArgs p) {
+  static_assert(!LORA || F16C, "the LoRA delta runs in the fp16 mode");
   static_assert(!F16C || (DT == E4B_BF16 && FMT != E4B_FMT_MXFP4), "fp16 mode: bf16 activations, NF4 weights");
   constexpr int CT = F16C ? E4B_FP16 : DT;  // MFMA operand type
   constexpr int NT = gemm_threads(BM);
@@ -522,6 +528,18 @@ __global__ void __launch_bounds__(gemm_threads(BM)) gemm_mfma_kernel(GemmArgs p)
   const int64_t klast = ksteps - 1;
   load_step(0, 0);
   __syncthreads();  // code2 table
+  if constexpr (LORA) {
+    int64_t brow[NS];
+#pragma unroll
+    for (int ns = 0; ns < NS; ++ns) {
+      const int lr = nbase[ns] + (lane & 15);
+      const int64_t jj = col0 + (pair ? (lr & (BN / 2 - 1)) : lr);
+      brow[ns] = jj < p.n_out ? (pair && lr >= BN / 2 ? n / 2 + jj : jj) : 0;
+    }
+    const int arow = wave_m * WM + (lane & 15);
+    lora_delta_16x16<MS, NS>(p, acc, e, row0 + arow, row_end - 1, [&](int ms) { return row_shift_s[arow + 16 * ms]; },
+                             wsh, brow, lane);
+  }
   stage(0, 0);
 #pragma unroll
   for (int j = 1; j <= ST; ++j) load_step(j % ST, min<int64_t>(j, klast));

@@ -3,6 +3,7 @@
 // pair, in parallel).
 #include "gemm.h"
 #include "gemm_launch.h"
+#include "lora_mfma.h"
 #include "gemm_narrow.h"
 #include "gemm_wide.h"
 #include "gemm_wide8.h"
@@ -63,14 +64,17 @@ dim3 gemm_grid(const GemmArgs& a, int64_t nw) {
 template <int DT, int FMT>
 void launch_mfma_gemm(const GemmArgs& a, hipStream_t s) {
   if constexpr (DT == E4B_BF16 && FMT != E4B_FMT_MXFP4) {
-    // the LoRA epilogue: fp16 mode, 256-row tiles (wide) or 32-row tiles the narrow kernel takes
-    // (the host checks lora_gemm_fits before asking)
+    // a LoRA delta: fp16 mode, 256-row tiles (wide) or 32-row tiles -- the narrow kernel where K is a
+    // whole number of its steps (the host checks lora_gemm_fits before asking)
     if (a.lt) {
       if (a.rt.tile_m == kTileMBig)
         hipLaunchKernelGGL((gemm_wide8_kernel<DT, FMT, true, true>), gemm_grid(a, kWideTileN), dim3(kWide8Threads), 0,
                            s, a);
-      else
+      else if (narrow_fits(a.w.k))
         hipLaunchKernelGGL((gemm_narrow_kernel<FMT, true>), gemm_grid(a, kNarrowN), dim3(kNarrowThreads), 0, s, a);
+      else
+        hipLaunchKernelGGL((gemm_mfma_kernel<DT, FMT, kTileMSmall, true, true>), gemm_grid(a, kTileNW),
+                           dim3(gemm_threads(kTileMSmall)), 0, s, a);
       return;
     }
     // 32-row tiles in the fp16 mode: the narrow kernel, when K is a whole number of its steps

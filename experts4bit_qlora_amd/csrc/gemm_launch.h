@@ -16,12 +16,13 @@ struct GemmArgs;
 template <int DT, int FMT>
 void launch_mfma_gemm(const GemmArgs& a, hipStream_t s);
 
-// Whether a grouped GEMM with a LoRA epilogue (GemmArgs::lt) or fp16 down rows
-// (GemmArgs::out_f16_shift) can run: fp16 mode over 256-row tiles (the eight-wave wide kernel), or
-// over 32-row tiles with K a whole number of the narrow kernel's step pairs.
-inline bool lora_gemm_fits(int tile_m, int64_t k) {
+// Whether the down rows of a tile list can leave as fp16 rows (GemmArgs::out_f16_shift): 256-row tiles
+// (the eight-wave wide kernel), or 32-row tiles with K a whole number of the narrow kernel's step pairs.
+inline bool f16_rows_fit(int tile_m, int64_t k) {
   return tile_m == 256 || (tile_m == 32 && k > 0 && k % 256 == 0 && k <= 256 * 64);
 }
+// Whether a grouped GEMM can start from a LoRA delta (GemmArgs::lt): the fp16 mode's 256- and 32-row tiles.
+inline bool lora_gemm_fits(int tile_m) { return tile_m == 256 || tile_m == 32; }
 
 #define E4B_GEMM_EXTERN(DT, FMT) extern template void launch_mfma_gemm<DT, FMT>(const GemmArgs&, hipStream_t);
 E4B_GEMM_EXTERN(E4B_BF16, E4B_FMT_NF4)

@@ -33,7 +33,8 @@ E4B_DEV void split_bf16x8(const float (&v)[8], uint4& hi, uint4& lo) {
 
 // 2^e * lscale * t[m, q0 + i] (0 past the rank), i = 0..7, split. With the rank a multiple of 8
 // the eight values are two 16-byte loads, else eight element loads.
-E4B_DEV void lora_t_piece(const GemmArgs& p, int64_t m, int q0, int e2, uint4& hi, uint4& lo) {
+template <class Args>
+E4B_DEV void lora_t_piece(const Args& p, int64_t m, int q0, int e2, uint4& hi, uint4& lo) {
   float v[8];
   const float* t = p.lt + m * p.lr;
   if ((p.lr & 7) == 0) {

@@ -460,9 +460,12 @@ __global__ void __launch_bounds__(kRouteChunk) route_place_kernel(const int64_t*
 // out[t, :] = out_t( sum_s float(down[inv[t*k+s], :]) * w[t, s] ), s ascending, fp32 adds of
 // rounded fp32 products -- engines/fast.py:158 and 276-278 (buf[order] = down.float() * w;
 // buf.view(T, k, H).sum(1).to(dtype)). Dropped slots (inv < 0) contribute nothing.
+constexpr int kUnitWeights = 3;  // a weight "dtype": every weight is 1 (a plain sum of rows)
 template <int WDT>
 E4B_DEV float load_weight(const void* w, int64_t i) {
-  if constexpr (WDT == E4B_FP32) {
+  if constexpr (WDT == kUnitWeights) {
+    return 1.0f;
+  } else if constexpr (WDT == E4B_FP32) {
     return static_cast<const float*>(w)[i];
   } else {
     return to_f<WDT>(static_cast<const uint16_t*>(w)[i]);

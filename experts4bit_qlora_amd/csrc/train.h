@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "dgrad.h"
 #include "gemm.h"
 #include "lora_mfma.h"
 
@@ -266,14 +267,6 @@ __global__ void __launch_bounds__(dgrad_threads(BM)) dgrad_mfma_kernel(DgradArgs
 constexpr int kWgradThreads = 256;
 constexpr int kWgradRows = 64;   // rows per round
 constexpr int kWgradCols = 128;  // columns per block, 32 per wave
-
-// 4 x 16-bit transposing LDS read: the 16 lanes of a group name the 16 8-byte pieces of a 4-row x
-// 16-column block (lane i: row i / 4, columns 4 (i % 4) ..) and lane i receives column i, rows 0..3.
-E4B_DEV uint2 lds_read_tr(const uint16_t* p) {
-  typedef short s4_t __attribute__((ext_vector_type(4)));
-  typedef __attribute__((address_space(3))) s4_t* lds_t;
-  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(p)));
-}
 
 // Element offset of column col (a multiple of 4) of row `row` in a tile of 16-bit rows of COLS columns:
 // the row's 32-byte pieces are XOR-ed with row bits 0, 1 and 3, so the eight rows of a half-wave's

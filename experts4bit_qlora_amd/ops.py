@@ -508,6 +508,52 @@ def moe_lora_forward(hidden: torch.Tensor, top_k_index: torch.Tensor, top_k_weig
     return out
 
 
+def _lora_struct(a1, b1, a2, b2, scaling) -> N.Lora:
+    return N.Lora(a1=a1.data_ptr(), b1=b1.data_ptr(), a2=a2.data_ptr(), b2=b2.data_ptr(), dtype=dtype_code(a1.dtype),
+                  rank=int(a1.shape[1]), scaling=float(scaling))
+
+
+def train_forward(x: torch.Tensor, idx: torch.Tensor, w: torch.Tensor, w1: QW, w2: QW, lora, scaling: float, epilogue: int,
+                  limit: float, out_dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
+    """The training layer's forward (``e4b_train_forward``): ``(out [T, H], saved)``, ``saved`` the bytes
+    its backward reads. ``x`` bf16 ``[T, H]``, ``idx`` int64 and ``w`` ``[T, k]``, ``lora = (A1, B1, A2,
+    B2)`` in one dtype, all contiguous."""
+    _require_cuda(x, idx, w, w1.packed, w2.packed, *lora)
+    L = N.lib()
+    T, k = idx.shape
+    r = int(lora[0].shape[1])
+    shape = (T, k, w1.num_experts, w1.n, w2.n, epilogue, r)
+    saved = torch.empty(max(1, int(L.e4b_train_saved_bytes(*shape))), dtype=torch.uint8, device=x.device)
+    ws = torch.empty(max(1, int(L.e4b_train_workspace_bytes(*shape, 0))), dtype=torch.uint8, device=x.device)
+    out = torch.empty(T, w2.n, dtype=out_dtype, device=x.device)
+    lo = _lora_struct(*lora, scaling)
+    N.check("e4b_train_forward",
+            L.e4b_train_forward(x.data_ptr(), T, idx.data_ptr(), w.data_ptr(), dtype_code(w.dtype), k, w1.ref(), w2.ref(),
+                                ctypes.byref(lo), epilogue, float(limit), saved.data_ptr(), saved.numel(), ws.data_ptr(),
+                                ws.numel(), out.data_ptr(), dtype_code(out_dtype), _stream(x.device)))
+    return out, saved
+
+
+def train_backward(grad: torch.Tensor, x: torch.Tensor, w: torch.Tensor, w1: QW, w2: QW, lora, scaling: float,
+                   epilogue: int, limit: float, saved: torch.Tensor, need) -> list:
+    """Its backward (``e4b_train_backward``): gradients of (x, w, A1, B1, A2, B2), None where ``need`` is
+    False."""
+    _require_cuda(grad, x, w, saved, w1.packed, w2.packed, *lora)
+    L = N.lib()
+    T, k = w.shape
+    r = int(lora[0].shape[1])
+    ws_bytes = int(L.e4b_train_workspace_bytes(T, k, w1.num_experts, w1.n, w2.n, epilogue, r, 1))
+    ws = torch.empty(max(1, ws_bytes), dtype=torch.uint8, device=x.device)
+    outs = [torch.empty_like(t) if n else None for t, n in zip((x, w, *lora), need)]
+    lo = _lora_struct(*lora, scaling)
+    N.check("e4b_train_backward",
+            L.e4b_train_backward(grad.data_ptr(), dtype_code(grad.dtype), x.data_ptr(), T, w.data_ptr(),
+                                 dtype_code(w.dtype), k, w1.ref(), w2.ref(), ctypes.byref(lo), epilogue, float(limit),
+                                 saved.data_ptr(), saved.numel(), ws.data_ptr(), ws.numel(), *[_ptr(t) for t in outs],
+                                 _stream(x.device)))
+    return outs
+
+
 # ------------------------------------------------- the nf4_grouped / mxfp4_grouped API shape
 
 

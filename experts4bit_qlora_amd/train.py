@@ -1,8 +1,10 @@
 """The training lane: ``enable_fast_train`` routes an ``ExpertsLoRA``'s training forward AND
 backward through the gfx950 kernels (reference ``experts4bit_qlora/engines/fast.py:453-674``).
 
-Forward, per projection (``_GroupedLoraProj``), over expert-sorted rows and with no host sync
-(the reference sorts with ``argsort`` and reads group sizes back with ``.tolist()``):
+With bf16 compute and an activation the kernels know, the layer is ``_FusedLoraLayer``: one library call
+each way (``e4b_train_forward`` / ``e4b_train_backward``). Other layers go projection by projection
+(``_GroupedLoraProj``), over expert-sorted rows; neither syncs with the host (the reference sorts
+with ``argsort`` and reads group sizes back with ``.tolist()``). Forward, per projection:
 
     proj[m] = a_m . deq(W[e_m])^T + scaling * (a_m . A[e_m]^T) . B[e_m]^T
 
@@ -81,6 +83,51 @@ class _GroupedLoraProj(torch.autograd.Function):
         return grad_a, grad_A, grad_B, None, None, None, None, None, None, None, None
 
 
+class _FusedLoraLayer(torch.autograd.Function):
+    """The whole layer as two library calls (``e4b_train_forward`` / ``e4b_train_backward``): both
+    projections with their deltas in the GEMM tiles, the activation and the router-weighted combine.
+    Inputs are contiguous; ``saved`` holds the forward's rows as one byte tensor."""
+
+    @staticmethod
+    def forward(ctx, x, w, a1, b1, a2, b2, idx, qw1, qw2, scaling, epi, limit, out_dtype):
+        out, saved = ops.train_forward(x, idx, w, qw1, qw2, (a1, b1, a2, b2), scaling, epi, limit, out_dtype)
+        ctx.save_for_backward(x, w, a1, b1, a2, b2, saved)
+        ctx.args = (qw1, qw2, scaling, epi, limit)
+        return out
+
+    @staticmethod
+    def backward(ctx, g):
+        x, w, a1, b1, a2, b2, saved = ctx.saved_tensors
+        qw1, qw2, scaling, epi, limit = ctx.args
+        grads = ops.train_backward(_aligned(g), x, w, qw1, qw2, (a1, b1, a2, b2), scaling, epi, limit, saved,
+                                   ctx.needs_input_grad[:6])
+        return (*grads, None, None, None, None, None, None, None)
+
+
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """``t`` contiguous at a 16-byte address (a view can start anywhere inside another tensor)."""
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
+
+
+def _layer_inputs(lora_mod, x, top_k_index, top_k_weights):
+    """(epilogue, limit, weights, adapters) for ``_FusedLoraLayer``, or None where the layer goes through the
+    per-projection functions: a compute dtype other than bf16, a base whose activation only its own
+    Python code knows, adapters of mixed dtypes, dtypes and shapes the library does not take."""
+    from . import fast as F
+
+    base = lora_mod.base
+    epi = F._fused_epilogue(base)
+    adapters = (lora_mod.gate_up_lora_A, lora_mod.gate_up_lora_B, lora_mod.down_lora_A, lora_mod.down_lora_B)
+    known = (torch.bfloat16, torch.float16, torch.float32)
+    if (epi is None or x.dtype != torch.bfloat16 or top_k_weights.dtype not in known
+            or any(a.dtype != adapters[0].dtype for a in adapters) or adapters[0].dtype not in known
+            or x.dim() != 2 or x.shape[1] != base._down_shape[0] or top_k_index.shape != top_k_weights.shape
+            or top_k_index.shape[0] != x.shape[0] or base._down_shape[1] % 64):
+        return None
+    return epi[0], epi[1], top_k_weights.contiguous(), [_aligned(a) for a in adapters]
+
+
 def _train_tile_m(M: int, E: int) -> int:
     """Row tiles of the training GEMMs: 128 once experts average 64 rows or more, else 32 (the
     forward's rule)."""
@@ -110,6 +157,12 @@ def fused_experts_train_forward(lora_mod, hidden_states, top_k_index, top_k_weig
     E = base.num_experts
     M = tokens * k
     w1, w2 = F._qweights(base)
+    layer = _layer_inputs(lora_mod, x, top_k_index, top_k_weights)
+    if layer is not None and input_dtype in (torch.bfloat16, torch.float16, torch.float32):
+        epi, limit, w, adapters = layer
+        w1, w2 = F._for_tokens((w1, w2), tokens + F._SHIFT_FREE_TOKENS)  # the shifts, whatever the batch
+        return _FusedLoraLayer.apply(_aligned(x), w, *adapters, top_k_index.to(torch.int64).contiguous(), w1, w2,
+                                     float(lora_mod.scaling), epi, limit, input_dtype)
     rb = ops.route(top_k_index, E, tile_m=_train_tile_m(M, E))
     s = float(lora_mod.scaling)
     proj = _GroupedLoraProj.apply(x, lora_mod.gate_up_lora_A, lora_mod.gate_up_lora_B, w1, rb, M, E, k, tokens, s,

@@ -365,6 +365,35 @@ enum e4b_probe_site {
  * stream that kernel is launched on. */
 int e4b_set_probe(int32_t site, hipEvent_t before, hipEvent_t after);
 
+/* The training layer of an ExpertsLoRA (fast.py:453-556 with nf4_qlora.fused_grouped_lora at
+ * fast.py:509-540), forward and backward: bf16 activations, NF4 / NF4_DQ weights carrying their
+ * shifts and no bias, output features a multiple of 64, epilogue SWIGLU, CLAMP_SWIGLU or ACT.
+ *
+ *   proj[m] = bf16(x_m . deq(W1[e])^T + scaling * (x_m . A1[e]^T) . B1[e]^T)   h = bf16(act(proj))
+ *   down[m] = bf16(h_m . deq(W2[e])^T + scaling * (h_m . A2[e]^T) . B2[e]^T)
+ *   out[t]  = sum over slots of top_k_weights[t, s] * down[row of (t, s)]      (fp32 sum, out_dtype)
+ *
+ * over expert-sorted rows m, the GEMMs in the fp16 matrix-core mode. The forward leaves what the
+ * backward reads in `saved` (e4b_train_saved_bytes, 16-byte aligned): routing, proj, h, down and both
+ * inner products. The backward takes dL/dout [tokens, H] in grad_dtype and writes what is asked for (a
+ * NULL output is skipped): grad_hidden bf16 [tokens, H], grad_weights in weight_dtype [tokens, top_k],
+ * and the adapters' gradients in their dtype and layout. Ids outside [0, E) contribute nothing and
+ * get zero gradients. Nothing synchronises; both directions are deterministic. */
+size_t e4b_train_saved_bytes(int64_t tokens, int32_t top_k, int32_t num_experts, int64_t n1, int64_t n2,
+                             int32_t epilogue, int32_t rank);
+size_t e4b_train_workspace_bytes(int64_t tokens, int32_t top_k, int32_t num_experts, int64_t n1, int64_t n2,
+                                 int32_t epilogue, int32_t rank, int32_t backward);
+int e4b_train_forward(const void* hidden, int64_t tokens, const int64_t* top_k_index, const void* top_k_weights,
+                      int32_t weight_dtype, int32_t top_k, const e4b_qweight* w1, const e4b_qweight* w2,
+                      const e4b_lora* lora, int32_t epilogue, float limit, void* saved, size_t saved_bytes,
+                      void* workspace, size_t workspace_bytes, void* out, int32_t out_dtype, hipStream_t stream);
+int e4b_train_backward(const void* grad_out, int32_t grad_dtype, const void* hidden, int64_t tokens,
+                       const void* top_k_weights, int32_t weight_dtype, int32_t top_k, const e4b_qweight* w1,
+                       const e4b_qweight* w2, const e4b_lora* lora, int32_t epilogue, float limit, const void* saved,
+                       size_t saved_bytes, void* workspace, size_t workspace_bytes, void* grad_hidden,
+                       void* grad_weights, void* grad_a1, void* grad_b1, void* grad_a2, void* grad_b2,
+                       hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -15,7 +15,7 @@ import torch
 import experts4bit_qlora_amd as e4b
 from experts4bit_qlora_amd import _native as N
 from experts4bit_qlora_amd import fast as F
-from experts4bit_qlora_amd import ops
+from experts4bit_qlora_amd import ops, train
 from oracle_weights import oracle_weights
 
 pytestmark = pytest.mark.gpu
@@ -279,3 +279,104 @@ def test_lora_wgrad_edges(r, adt, top, cols):
     u[70, 0] = float("inf")  # expert 2's alone
     got = ops.lora_wgrad(u, a, rb, M, E_, 0.5)
     assert not got[2, 0].isfinite().any() and got[[0, 1, 3, 4, 5, 6]].isfinite().all()
+
+
+def _layer_fp64(base, mod, x, idx, w, grad, act):
+    """The layer and its gradients in fp64 autograd over the oracle-decoded weights, nothing rounded."""
+    W1, W2 = ([torch.from_numpy(W[e]).double().to(DEV) for e in range(base.num_experts)] for W in oracle_weights(base))
+    x, w = x.double().requires_grad_(), w.double().requires_grad_()
+    p = {n: t.detach().double().requires_grad_() for n, t in mod.named_parameters() if "lora" in n}
+    out = torch.zeros_like(x)
+    for e in range(base.num_experts):
+        tok, slot = torch.where(idx == e)
+        if not len(tok):
+            continue
+        proj = x[tok] @ W1[e].T + mod.scaling * (x[tok] @ p["gate_up_lora_A"][e].T) @ p["gate_up_lora_B"][e].T
+        h = act(proj)
+        down = h @ W2[e].T + mod.scaling * (h @ p["down_lora_A"][e].T) @ p["down_lora_B"][e].T
+        out = out.index_add(0, tok, down * w[tok, slot, None])
+    out.backward(grad.double())
+    return {"out": out.detach(), "x": x.grad, "w": w.grad, **{n: t.grad for n, t in p.items()}}
+
+
+def _swiglu64(limit=0.0):
+    """With a limit the gradient jumps at it, and a value within the layer's rounding of the limit may lie on
+    either side: a share of 2^-8 of the limit times the density there, its root in norm (0.7 under a
+    density of 0.2: 2e-2). So the clamp sees proj as the layer stores it, rounded to bf16 (gradient
+    passed straight through), and the limit of 4 lies beyond two standard deviations, where the
+    weights' own rounding (2^-11) moves few values across (a density of 0.015: 4e-3)."""
+    def act(proj):
+        if limit:
+            proj = proj + (proj.to(torch.bfloat16).double() - proj).detach()
+        g, u = proj.chunk(2, -1)
+        if limit:
+            g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+        return torch.nn.functional.silu(g) * u
+
+    return act
+
+
+@pytest.mark.parametrize("T,E_,top,hid,inter,r,adt,dq,kind,xdt", [
+    (2048, 8, 2, 256, 128, 16, torch.float32, False, "swiglu", torch.bfloat16),   # 256-row tiles, whole step pairs
+    (700, 4, 2, 192, 320, 20, torch.bfloat16, True, "swiglu", torch.bfloat16),    # halved tiles; k off 256 and 128
+    (300, 3, 1, 320, 192, 64, torch.float16, False, "clamp", torch.float32),      # tails of 1..32 rows, fp32 tokens
+    (33, 16, 4, 128, 64, 1, torch.float32, True, "act", torch.bfloat16),          # 32-row tiles only, one gate half
+    (1, 8, 2, 64, 64, 8, torch.float32, False, "swiglu", torch.bfloat16),
+])
+def test_fused_layer_matches_fp64(T, E_, top, hid, inter, r, adt, dq, kind, xdt):
+    """The two-call layer against fp64 autograd: outputs and every gradient. bf16 rounds x, proj, h, the down
+    rows and their gradients (2^-9 each, independent): 1e-2 in norm is the contract's bar. Dropped ids
+    (-1 and E) contribute nothing and get zero router gradients."""
+    _announce(f"fused layer T={T} E={E_} hid={hid} inter={inter} r={r} {kind}")
+    torch.manual_seed(21)
+    gated = kind != "act"
+    gu = (torch.randn(E_, (2 if gated else 1) * inter, hid) * 0.1).to(DEV)
+    dn = (torch.randn(E_, hid, inter) * 0.1).to(DEV)
+    if kind == "clamp":
+        base = e4b.DeepseekV4Experts4bit.from_deepseek_v4(gu, dn, limit=4.0, compute_dtype=torch.bfloat16,
+                                                          compress_statistics=dq)
+    else:
+        base = e4b.Experts4bit.from_float(gu, dn, has_gate=gated, compute_dtype=torch.bfloat16, compress_statistics=dq)
+    mod = e4b.ExpertsLoRA(base, r=r, alpha=2 * r, dtype=adt).to(DEV).train()
+    with torch.no_grad():
+        for p in (mod.gate_up_lora_B, mod.down_lora_B):
+            p.normal_(0, 0.05)
+    assert e4b.enable_fast_train(mod) == 1
+    x = torch.randn(T, hid, device=DEV).to(torch.bfloat16).to(xdt).requires_grad_()
+    idx = torch.rand(T, E_, device=DEV).argsort(1)[:, :top].contiguous()
+    if T > 2:
+        idx[1, 0], idx[2, top - 1] = -1, E_
+    w = torch.rand(T, top, device=DEV).to(torch.bfloat16).requires_grad_()
+    grad = torch.randn(T, hid, device=DEV).to(xdt)
+    assert train._layer_inputs(mod, x.detach().to(torch.bfloat16), idx, w) is not None
+    out = mod(x, idx, w)
+    out.backward(grad)
+    got = {"out": out.detach(), "x": x.grad, "w": w.grad, **{n: p.grad for n, p in mod.named_parameters() if "lora" in n}}
+    act = {"swiglu": _swiglu64(), "clamp": _swiglu64(4.0), "act": torch.nn.functional.silu}[kind]
+    want = _layer_fp64(base, mod, x.detach(), idx, w.detach(), grad, act)
+    assert out.dtype == xdt and x.grad.dtype == xdt
+    for n in want:
+        assert _rel(got[n], want[n]) < GRAD_TOL, (n, _rel(got[n], want[n]))
+    if T > 2:
+        assert w.grad[1, 0] == 0 and w.grad[2, top - 1] == 0
+
+
+def test_fused_layer_gives_only_the_gradients_asked_for():
+    """Each subset of leaves alone gives the bits that all of them together give."""
+    _announce("fused layer partial gradients")
+    mod = _build(seed=9)
+    assert e4b.enable_fast_train(mod) == 1
+    hs, idx, wts, loss_w = _inputs(n_tok=90, seed=11)
+    names = ("gate_up_lora_A", "gate_up_lora_B", "down_lora_A", "down_lora_B")
+
+    def grads(leaves):
+        x, w = hs.clone().requires_grad_("x" in leaves), wts.clone().requires_grad_("w" in leaves)
+        for n in names:
+            getattr(mod, n).requires_grad_(n in leaves).grad = None
+        mod(x, idx, w).backward(loss_w.to(torch.bfloat16))
+        return {"x": x.grad, "w": w.grad, **{n: getattr(mod, n).grad for n in names}}
+
+    full = grads(("x", "w", *names))
+    for n in full:
+        only = grads((n,))
+        assert torch.equal(only[n], full[n]) and all(only[m] is None for m in only if m != n), n
