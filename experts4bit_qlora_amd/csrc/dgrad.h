@@ -367,29 +367,34 @@ dgrad_narrow_kernel(Dgrad16Args p) {
       ptab[(wid + 4 * i) * kCopies + lane] = cvt_pair<E4B_FP16>(p.w.code[i >> 2], lo[i & 3]);
     if constexpr (FMT == E4B_FMT_NF4_DQ) code2_s[tid] = p.w.code2[tid];
   }
+  // uniform bases plus 32-bit lane offsets (one expert's weights and scales stay below 4 GB)
   const int64_t nb = n * (K / 64), nb2 = (nb + 255) / 256;
-  const uint8_t* const wbase = p.w.packed + int64_t(e) * n * (K / 2) + cl / 2;
-  const uint16_t* const gbase = p.g + int64_t(grow) * n + 8 * half;
+  const uint8_t* const wbase = p.w.packed + int64_t(e) * n * (K / 2);
+  const uint32_t w_off = static_cast<uint32_t>(8 * half * (K / 2) + cl / 2);
+  const uint16_t* const gbase = p.g + int64_t(row0) * n;
+  const uint32_t g_off = static_cast<uint32_t>((grow - row0) * n + 8 * half);
 
-  // step t (16 weight rows): the lane's words and scales of rows 16 t + 8 half + i, its gradient piece
+  // step t (16 weight rows): the lane's words of rows 16 t + 8 half + i, its gradient piece, and ONE block
+  // scale: eight neighbouring lanes hold the 64 columns of one block, and lane i of them loads and
+  // decodes row i's scale for all (every lane loading its eight rows' scales kept the load pipeline
+  // busy: 25 load instructions per step instead of 11, 322 -> 263 us for both projections of the
+  // Qwen3 step at 509 tokens, with the loads kept in order below)
   uint32_t wq[2][8];
-  float sa[2][8];
-  uint32_t sq[2][8];
+  float sa[2];
+  uint32_t sq[2];
   uint4 gv[2];
+  const uint32_t s_off = static_cast<uint32_t>((8 * half + (lane & 7)) * (K / 64) + cl / 64);
   auto load = [&](auto set_c, int64_t t) {
     constexpr int set = decltype(set_c)::value;
-    gv[set] = *reinterpret_cast<const uint4*>(gbase + 16 * t);
+    gv[set] = *reinterpret_cast<const uint4*>(gbase + 16 * t + g_off);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int64_t row = 16 * t + 8 * half + i;
-      wq[set][i] = *reinterpret_cast<const uint32_t*>(wbase + row * (K / 2));
-      const int64_t blk = row * (K / 64) + cl / 64;
-      if constexpr (FMT == E4B_FMT_NF4) {
-        sa[set][i] = static_cast<const float*>(p.w.absmax)[int64_t(e) * nb + blk];
-      } else {
-        sq[set][i] = static_cast<const uint8_t*>(p.w.absmax)[int64_t(e) * nb + blk];
-        sa[set][i] = p.w.absmax2[int64_t(e) * nb2 + blk / 256];
-      }
+    for (int i = 0; i < 8; ++i)
+      wq[set][i] = *reinterpret_cast<const uint32_t*>(wbase + (16 * t + i) * (K / 2) + w_off);
+    if constexpr (FMT == E4B_FMT_NF4) {
+      sa[set] = (static_cast<const float*>(p.w.absmax) + int64_t(e) * nb + 16 * t * (K / 64))[s_off];
+    } else {
+      sq[set] = (static_cast<const uint8_t*>(p.w.absmax) + int64_t(e) * nb + 16 * t * (K / 64))[s_off];
+      sa[set] = (p.w.absmax2 + int64_t(e) * nb2)[(static_cast<uint32_t>(16 * t * (K / 64)) + s_off) / 256];
     }
   };
   f32x16_t acc[NB];
@@ -398,15 +403,19 @@ dgrad_narrow_kernel(Dgrad16Args p) {
   auto step = [&](auto set_c) {
     constexpr int set = decltype(set_c)::value;
     uint32_t sc[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      float scale = sa[set][i];
+    {
+      float scale = sa[set];
       if constexpr (FMT == E4B_FMT_NF4_DQ) {
-        const float prod = code2_s[sq[set][i]] * sa[set][i];
+        const float prod = code2_s[sq[set]] * sa[set];
         scale = prod + offset;
       }
       scale = __builtin_amdgcn_ldexpf(scale, wsh);
-      sc[i] = cvt_pair<E4B_FP16>(scale, scale);
+      const int own = static_cast<int>(cvt_pair<E4B_FP16>(scale, scale));
+      static_for<8>([&](auto ic) {  // row_newbcast: lane i of each 16 to its lower eight, lane 8 + i to its upper
+        constexpr int i = decltype(ic)::value;
+        const int lower = __builtin_amdgcn_update_dpp(0, own, 0x150 + i, 0xf, 0x3, false);
+        sc[i] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(lower, own, 0x158 + i, 0xf, 0xc, false));
+      });
     }
     static_for<4>([&](auto bc) {  // packed byte: columns 8 c + 2 b and + 1
       constexpr int b = decltype(bc)::value;
@@ -456,10 +465,15 @@ dgrad_narrow_kernel(Dgrad16Args p) {
   }
   int64_t i = 0;
   for (; i + 2 <= steps; i += 2) {
+    // the order is kept by hand: loads moved across a step make its wait one for the newest loads
     step(std::integral_constant<int, 0>{});
+    __builtin_amdgcn_sched_barrier(0);
     load(std::integral_constant<int, 0>{}, at(i + 2));
+    __builtin_amdgcn_sched_barrier(0);
     step(std::integral_constant<int, 1>{});
+    __builtin_amdgcn_sched_barrier(0);
     load(std::integral_constant<int, 1>{}, at(i + 3));
+    __builtin_amdgcn_sched_barrier(0);
   }
   if (i < steps) step(std::integral_constant<int, 0>{});
 

@@ -770,16 +770,21 @@ template <bool TRANS>
 int lora_wgrad(const float* u, int rank, const void* a, int a_dtype, int gather_k, const e4b_routing* rt,
                int num_experts, int64_t cols, float scale, void* out, int odt, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>(cdiv(cols, e4b::kWgradCols)), static_cast<unsigned>(num_experts));
-#define E4B_WG(XD, RB)                                                                                            \
-  hipLaunchKernelGGL((e4b::lora_wgrad_kernel<XD, RB, TRANS>), grid, dim3(e4b::kWgradThreads), 0, stream, u, rank, \
-                     static_cast<const uint16_t*>(a), gather_k, rt->sorted_flat, rt->offsets, cols, scale, out, odt)
+  const bool vec = cols % 8 == 0 && aligned16(a);
+#define E4B_WG(XD, RB, GA, VE)                                                                                    \
+  hipLaunchKernelGGL((e4b::lora_wgrad_kernel<XD, RB, TRANS, GA, VE>), grid, dim3(e4b::kWgradThreads), 0, stream, u, \
+                     rank, static_cast<const uint16_t*>(a), gather_k, rt->sorted_flat, rt->offsets, cols, scale, out, odt)
+#define E4B_WG_V(XD, RB)                                                                 \
+  if (gather_k > 0) { if (vec) E4B_WG(XD, RB, true, true); else E4B_WG(XD, RB, true, false); } \
+  else { if (vec) E4B_WG(XD, RB, false, true); else E4B_WG(XD, RB, false, false); }
 #define E4B_WG_R(XD)                                     \
-  if (rank <= 16) E4B_WG(XD, 16);                        \
-  else if (rank <= 32) E4B_WG(XD, 32);                   \
-  else E4B_WG(XD, e4b::kLoraMaxRank);
+  if (rank <= 16) { E4B_WG_V(XD, 16) }                   \
+  else if (rank <= 32) { E4B_WG_V(XD, 32) }              \
+  else { E4B_WG_V(XD, e4b::kLoraMaxRank) }
   if (a_dtype == E4B_BF16) { E4B_WG_R(E4B_BF16) }
   else { E4B_WG_R(E4B_FP16) }
 #undef E4B_WG_R
+#undef E4B_WG_V
 #undef E4B_WG
   return check_launch("lora_wgrad_kernel");
 }
@@ -1690,10 +1695,16 @@ int lora_u_mfma(const uint16_t* g, const e4b_routing& rt, const void* B, int bdt
   if (blocks > 0x7fffffffLL) return fail(E4B_EUNSUPPORTED, "LoRA u grid too large");
   const dim3 grid(static_cast<unsigned>(blocks));
   const int nsm = rank <= 16 ? 1 : (rank <= 32 ? 2 : 4);
+  const bool vec = rank % 8 == 0 && aligned16(B);
 #define E4B_UM(AD, BM, NS)                                                                                     \
-  if (bdt == AD && bm == BM && nsm == NS)                                                                     \
-    hipLaunchKernelGGL((e4b::lora_u_mfma_kernel<AD, BM, NS>), grid, dim3(BM / 16 * e4b::kWave), 0, stream, g, rt, B, \
-                       rank, n, u);
+  if (bdt == AD && bm == BM && nsm == NS) {                                                                   \
+    if (vec)                                                                                                  \
+      hipLaunchKernelGGL((e4b::lora_u_mfma_kernel<AD, BM, NS, true>), grid, dim3(BM / 16 * e4b::kWave), 0, stream, \
+                         g, rt, B, rank, n, u);                                                               \
+    else                                                                                                      \
+      hipLaunchKernelGGL((e4b::lora_u_mfma_kernel<AD, BM, NS, false>), grid, dim3(BM / 16 * e4b::kWave), 0, stream, \
+                         g, rt, B, rank, n, u);                                                               \
+  }
 #define E4B_UM_AD(AD) E4B_UM(AD, 64, 1) E4B_UM(AD, 64, 2) E4B_UM(AD, 64, 4) E4B_UM(AD, 32, 1) E4B_UM(AD, 32, 2) \
   E4B_UM(AD, 32, 4)
   E4B_UM_AD(E4B_BF16) E4B_UM_AD(E4B_FP16) E4B_UM_AD(E4B_FP32)

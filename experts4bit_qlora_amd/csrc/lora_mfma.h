@@ -143,10 +143,10 @@ namespace e4b {
 // its rows (NSM 16-rank blocks) on v_mfma_f32_16x16x32_bf16. x rows are bf16 (exact operands); A
 // (bf16, fp16 or fp32) is staged per 64-deep chunk in LDS as bf16 hi / lo halves (lo = bf16(a -
 // hi), the split of split_bf16x8), so t carries about 16 significant bits of each product of an
-// fp32 or fp16 adapter and every product of a bf16 one exactly. The chunks are double-buffered:
-// chunk c + 1's A is loaded into registers and its x fragments are loaded while chunk c's MFMAs
-// run, one barrier per chunk. The LDS is 8 KB per rank block (4 KB without lo halves), so many
-// workgroups share a CU and keep enough x loads in flight.
+// fp32 or fp16 adapter and every product of a bf16 one exactly. The chunks are double-buffered,
+// one barrier per chunk, with A two chunks and x three chunks ahead in registers: a launch has only
+// a workgroup or two per CU, so the x loads in flight per wave set its rate (one chunk ahead: 43 us
+// for both of an OLMoE layer's t at 1,531 tokens, 31 us so).
 constexpr int kLoraTK = 64;  // K per chunk
 constexpr int kLoraTGroups = kLoraTK / 8;
 
@@ -180,10 +180,12 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
   const int64_t src = gather_k > 0 ? rt.sorted_flat[rr] / gather_k : rr;
   const uint16_t* xr = x + src * in;
   const int nchunks = static_cast<int>(in / kLoraTK);
+  auto chunk = [&](int c) { return min(c, nchunks - 1); };  // past the last chunk it is re-read
 
   // staging: thread tid takes groups j = tid + NT i of the chunk's [16 NSM ranks][8 groups]
-  float sv[SPT][8];
-  auto load_a = [&](int c) {
+  float sets[2][SPT][8];
+  auto load_a = [&](auto set, int c) {
+    float (&sv)[SPT][8] = sets[decltype(set)::value];
 #pragma unroll
     for (int i = 0; i < SPT; ++i) {
       const int j = tid + NT * i;
@@ -206,7 +208,8 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
       }
     }
   };
-  auto store_a = [&](int buf) {
+  auto store_a = [&](auto set, int buf) {
+    const float (&sv)[SPT][8] = sets[decltype(set)::value];
 #pragma unroll
     for (int i = 0; i < SPT; ++i) {
       const int j = tid + NT * i;
@@ -231,37 +234,41 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
   f32x4_t acc[NSM];
 #pragma unroll
   for (int i = 0; i < NSM; ++i) acc[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  // chunk c from LDS buffer c % 2 and x fragments xc, with chunk c + 1 loaded meanwhile
-  auto step = [&](int c, const uint4 (&xc)[2], uint4 (&xn)[2]) {
-    const int cur = c & 1;
-    const int nc = min(c + 1, nchunks - 1);  // past the last chunk: a cached re-read, never used
-    load_a(nc);
-    load_x(xn, nc);
+  // chunk c from LDS buffer c % 2 and x set c % 4; meanwhile chunk c + 1's A goes from registers (set
+  // (c + 1) % 2) into the other buffer, chunk c + 2's A and chunk c + 3's x are requested
+  uint4 xs[4][2];
+  auto step = [&](auto uc, int c) __attribute__((always_inline)) {
+    constexpr int u = decltype(uc)::value;  // c % 4
+    constexpr int cur = u & 1;
+    load_a(std::integral_constant<int, cur>{}, chunk(c + 2));
+    load_x(xs[(u + 3) & 3], chunk(c + 3));
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
 #pragma unroll
       for (int ns = 0; ns < NSM; ++ns) {
         const int at = lora_t_at(16 * ns + l16, 4 * s + g);
         const uint4 bh = *reinterpret_cast<const uint4*>(&ah[cur][at]);
-        acc[ns] = mfma_16x16x32<E4B_BF16>(xc[s], bh, acc[ns]);
+        acc[ns] = mfma_16x16x32<E4B_BF16>(xs[u][s], bh, acc[ns]);
         if constexpr (LO) {
           const uint4 bl = *reinterpret_cast<const uint4*>(&al[cur][at]);
-          acc[ns] = mfma_16x16x32<E4B_BF16>(xc[s], bl, acc[ns]);
+          acc[ns] = mfma_16x16x32<E4B_BF16>(xs[u][s], bl, acc[ns]);
         }
       }
     }
-    store_a(cur ^ 1);  // the other buffer: its last readers passed the previous barrier
+    store_a(std::integral_constant<int, cur ^ 1>{}, cur ^ 1);  // its last readers passed the previous barrier
     __syncthreads();
   };
-  uint4 xa[2], xb[2];
-  load_a(0);
-  load_x(xa, 0);
-  store_a(0);
+  load_a(std::integral_constant<int, 0>{}, chunk(0));
+#pragma unroll
+  for (int i = 0; i < 3; ++i) load_x(xs[i], chunk(i));
+  load_a(std::integral_constant<int, 1>{}, chunk(1));
+  store_a(std::integral_constant<int, 0>{}, 0);
   __syncthreads();
-  for (int c = 0; c < nchunks; c += 2) {  // two chunks per trip: the fragment sets stay in registers
-    step(c, xa, xb);
-    if (c + 1 < nchunks) step(c + 1, xb, xa);
-  }
+  int c = 0;
+  for (; c + 4 <= nchunks; c += 4) static_for<4>([&](auto u) { step(u, c + int(u)); });
+  static_for<3>([&](auto u) {
+    if (c + int(u) < nchunks) step(u, c + int(u));
+  });
   // lane holds t[row 16 w + 4 g + i][rank 16 ns + l16]
 #pragma unroll
   for (int ns = 0; ns < NSM; ++ns) {

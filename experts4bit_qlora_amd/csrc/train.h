@@ -299,9 +299,9 @@ E4B_DEV uint16_t bf16_part(float& v) {
 // significant bits, so every product on the bf16 matrix cores is exact and only the fp32 order of
 // the sum differs from a multiply-add loop; fp16 rows are two bf16 parts, exact too. Bound by
 // reading a once per 128 columns: the next round's rows are in flight while this one's multiply.
-// OLMoE, 2,048 tokens, rank 16: the four gradients 243 -> 83 us; Qwen3, 509 tokens, rank 32,
-// 487 -> 111 us (VALU multiply-adds with u broadcast from LDS before).
-template <int XDT, int RB, bool TRANS>
+// OLMoE, 2,048 tokens, rank 16: the four gradients 243 -> 73 us; Qwen3, 509 tokens, rank 32,
+// 487 -> 94 us (VALU multiply-adds with u broadcast from LDS before).
+template <int XDT, int RB, bool TRANS, bool GATHER, bool VEC>
 __global__ void __launch_bounds__(kWgradThreads) lora_wgrad_kernel(const float* __restrict__ u, int r,
                                                                    const uint16_t* __restrict__ a, int gather_k,
                                                                    const int32_t* __restrict__ sorted_flat,
@@ -319,11 +319,14 @@ __global__ void __launch_bounds__(kWgradThreads) lora_wgrad_kernel(const float* 
   const int l16 = lane & 15, g = lane >> 4;
 
   // a pieces: piece i of thread t is row t / 16 + 16 i of the round, columns 8 (t % 16) ..; whole
-  // pieces (cols % 8 == 0, aligned) or single elements; columns past the end read column 0 (their
-  // sums are never stored)
+  // pieces (VEC: cols % 8 == 0, aligned) or single elements; columns past the end read column 0
+  // (their sums are never stored). GATHER and VEC are template arguments because a branch around a
+  // load makes every later wait a wait for all loads in flight
   const int ac = 8 * (tid & 15);
-  const bool vec = (cols & 7) == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
-  auto row_of = [&](int m) -> int64_t { return gather_k > 0 ? static_cast<int64_t>(sorted_flat[m] / gather_k) : m; };
+  auto row_of = [&](int m) -> int64_t {
+    if constexpr (GATHER) return sorted_flat[m] / gather_k;
+    else return m;
+  };
   uint4 av[AP];
   float uv[UP];
   auto load = [&](int m0) {
@@ -331,7 +334,7 @@ __global__ void __launch_bounds__(kWgradThreads) lora_wgrad_kernel(const float* 
     for (int i = 0; i < AP; ++i) {
       const int m = m0 + (tid >> 4) + 16 * i;
       const uint16_t* row = a + row_of(min(m, end - 1)) * cols;
-      if (vec) {
+      if constexpr (VEC) {
         av[i] = *reinterpret_cast<const uint4*>(row + (c0 + ac < cols ? c0 + ac : 0));
       } else {
         uint32_t w[4];
@@ -342,26 +345,26 @@ __global__ void __launch_bounds__(kWgradThreads) lora_wgrad_kernel(const float* 
         }
         av[i] = make_uint4(w[0], w[1], w[2], w[3]);
       }
-      if (m >= end) av[i] = make_uint4(0, 0, 0, 0);
     }
     // u value i of thread t: row (t + 256 i) / RB, rank (t + 256 i) % RB
 #pragma unroll
     for (int i = 0; i < UP; ++i) {
       const int idx = tid + kWgradThreads * i, row = idx / RB, j = idx % RB;
-      const bool in = m0 + row < end && j < r;
-      const float v = u[int64_t(min(m0 + row, end - 1)) * r + (j < r ? j : 0)];
-      uv[i] = in ? v : 0.0f;
+      uv[i] = u[int64_t(min(m0 + row, end - 1)) * r + (j < r ? j : 0)];
     }
   };
-  auto stage = [&]() {
+  auto stage = [&](int m0) {  // rows past the expert's end are zeros in both operands
 #pragma unroll
-    for (int i = 0; i < AP; ++i)
-      *reinterpret_cast<uint4*>(&as[wgrad_at<kWgradCols>((tid >> 4) + 16 * i, ac)]) = av[i];
+    for (int i = 0; i < AP; ++i) {
+      const uint32_t keep = m0 + (tid >> 4) + 16 * i < end ? ~0u : 0u;
+      *reinterpret_cast<uint4*>(&as[wgrad_at<kWgradCols>((tid >> 4) + 16 * i, ac)]) =
+          make_uint4(av[i].x & keep, av[i].y & keep, av[i].z & keep, av[i].w & keep);
+    }
 #pragma unroll
     for (int i = 0; i < UP; ++i) {
       const int idx = tid + kWgradThreads * i, row = idx / RB, j = idx % RB;
       const int at = wgrad_at<RB>(row, j & ~3) + (j & 3);
-      float v = uv[i];
+      float v = m0 + row < end && j < r ? uv[i] : 0.0f;
       us[0][at] = bf16_part(v);
       us[1][at] = bf16_part(v);
       us[2][at] = bf16_part(v);
@@ -384,9 +387,10 @@ __global__ void __launch_bounds__(kWgradThreads) lora_wgrad_kernel(const float* 
   if (beg < end) load(beg);
   for (int m0 = beg; m0 < end; m0 += kWgradRows) {
     __syncthreads();  // the previous round's reads are done
-    stage();
+    stage(m0);
     __syncthreads();
-    if (m0 + kWgradRows < end) load(m0 + kWgradRows);
+    load(min(m0 + kWgradRows, end - 1));  // past the last round: a re-read that is not used
+    __builtin_amdgcn_sched_barrier(0);    // (the next stage's splitting stays behind the MFMAs)
 #pragma unroll
     for (int s = 0; s < kWgradRows / 32; ++s) {
       uint4 ah[2], al[2];
@@ -419,6 +423,7 @@ __global__ void __launch_bounds__(kWgradThreads) lora_wgrad_kernel(const float* 
           }
         }
     }
+    __builtin_amdgcn_sched_barrier(0);
   }
   // lane holds ranks 16 q + 4 g + i of column 32 wid + 16 t + lane % 16
   auto put = [&](int64_t at, float v) {
