@@ -32,6 +32,7 @@ EXPORTS = (
     "e4b_mfma_tile_m",
     "e4b_dequant",
     "e4b_quantize_4bit",
+    "e4b_quantize_8bit",
     "e4b_weight_shift",
     "e4b_route_scratch_ints",
     "e4b_route",
@@ -133,6 +134,8 @@ def _bind(L):
     L.e4b_dequant.argtypes = [QW, I32, I32, I32, P, P]
     L.e4b_quantize_4bit.restype = ctypes.c_int
     L.e4b_quantize_4bit.argtypes = [P, I32, I64, ctypes.POINTER(F32), ctypes.POINTER(ctypes.c_uint8), I32, P, P, P]
+    L.e4b_quantize_8bit.restype = ctypes.c_int
+    L.e4b_quantize_8bit.argtypes = [P, P, I64, I64, P, I32, P, P, P]
     L.e4b_weight_shift.restype = ctypes.c_int
     L.e4b_weight_shift.argtypes = [QW, P, P]
     L.e4b_route_scratch_ints.restype = I64

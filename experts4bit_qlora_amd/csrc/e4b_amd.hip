@@ -464,6 +464,19 @@ int e4b_quantize_4bit(const void* w, int32_t dtype, int64_t values, const float*
   return check_launch("quantize4_kernel");
 }
 
+int e4b_quantize_8bit(const float* values, const float* offset, int64_t rows, int64_t n, const float* mids,
+                      int32_t zero_code, uint8_t* codes, float* absmax, hipStream_t stream) {
+  if (rows < 0 || n < 0) return fail(E4B_EINVAL, "negative sizes");
+  if (zero_code < 0 || zero_code > 255) return fail(E4B_EINVAL, "bad zero code");
+  if (rows == 0 || n == 0) return E4B_OK;
+  if (!values || !offset || !mids || !codes || !absmax) return fail(E4B_EINVAL, "NULL pointer");
+  const int64_t blocks = cdiv(n, e4b::kQuant8Block);
+  if (blocks > 0x7fffffffLL / rows) return fail(E4B_EUNSUPPORTED, "more blocks than one launch covers");
+  hipLaunchKernelGGL(e4b::quantize8_kernel, dim3(static_cast<unsigned>(rows * blocks)), dim3(e4b::kQuant8Block), 0,
+                     stream, values, offset, n, blocks, mids, zero_code, codes, absmax);
+  return check_launch("quantize8_kernel");
+}
+
 int e4b_route(const int64_t* top_k_index, int64_t tokens, int32_t top_k, int32_t num_experts, const e4b_routing* rt,
               hipStream_t stream) {
   return route_impl(top_k_index, tokens, top_k, num_experts, rt, nullptr, stream);

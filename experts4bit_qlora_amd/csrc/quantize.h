@@ -121,4 +121,38 @@ __global__ void __launch_bounds__(kQuantThreads) quantize4_kernel(const void* __
   }
 }
 
+constexpr int kQuant8Block = 256;
+
+// Second level of double quantization: rows of n values, each less its row's offset, in blocks of 256 to
+// a sorted 256-entry code whose 255 midpoints lie in device memory (`double_quant` in quant.py bit for
+// bit). A row's last block is padded with zeros. Block (row, 256-value block), one value per thread: its
+// code by an eight-step search of the midpoints in LDS. Small (1 / 64 of the weights), so bound by
+// launches: ~25 torch operations with two device-to-host copies each became this one.
+__global__ void __launch_bounds__(kQuant8Block) quantize8_kernel(const float* __restrict__ values,
+                                                                 const float* __restrict__ offset, int64_t n,
+                                                                 int64_t blocks, const float* __restrict__ mids,
+                                                                 int zero, uint8_t* __restrict__ codes,
+                                                                 float* __restrict__ absmax) {
+  __shared__ float mid_s[kQuant8Block];
+  __shared__ uint32_t top[kQuant8Block / kWave];
+  const int64_t row = blockIdx.x / blocks, b = blockIdx.x % blocks;
+  const int64_t i = b * kQuant8Block + threadIdx.x;
+  mid_s[threadIdx.x] = threadIdx.x < kQuant8Block - 1 ? mids[threadIdx.x] : 0.0f;
+  const float c = i < n ? values[row * n + i] - offset[row] : 0.0f;
+  uint32_t m = __float_as_uint(c) & 0x7fffffffu;  // a NaN stays the maximum
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), o)));
+  if ((threadIdx.x & (kWave - 1)) == 0) top[threadIdx.x / kWave] = m;
+  __syncthreads();
+  m = max(max(top[0], top[1]), max(top[2], top[3]));
+  const float am = __uint_as_float(m);
+  const bool some = am > 0.0f;
+  const float x = c * (some ? 1.0f / am : 0.0f);
+  int pos = 0;  // midpoints below x: the search keeps mids[pos - 1] < x (a NaN passes them all)
+#pragma unroll
+  for (int s = kQuant8Block / 2; s > 0; s >>= 1) pos += !(mid_s[pos + s - 1] >= x) ? s : 0;
+  if (i < n) codes[row * n + i] = static_cast<uint8_t>(some ? pos : zero);
+  if (threadIdx.x == 0) absmax[blockIdx.x] = am;
+}
+
 }  // namespace e4b

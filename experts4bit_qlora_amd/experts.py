@@ -221,7 +221,7 @@ class ExpertsNbit(nn.Module):
             packed, absmax = module._quantize_stack(w)
             setattr(module, f"{name}_proj", nn.Parameter(packed, requires_grad=False))
             if module.compress_statistics:
-                q, a2, off = Q.double_quant(absmax, code2=module.code2)
+                q, a2, off = Q.double_quant(absmax)  # to the map that module.code2 holds
                 setattr(module, f"{name}_absmax", q)
                 setattr(module, f"{name}_absmax2", a2)
                 setattr(module, f"{name}_absmax_offset", off)

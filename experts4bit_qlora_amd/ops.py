@@ -167,6 +167,21 @@ def quantize_4bit(w: torch.Tensor, mids, codes, zero_code: int) -> tuple[torch.T
     return packed, absmax
 
 
+def quantize_8bit(values: torch.Tensor, offset: torch.Tensor, mids: torch.Tensor, zero_code: int):
+    """fp32 rows ``[..., n]`` less ``offset [...]`` -> (uint8 codes ``[..., n]``, absmax ``[..., ceil(n/256)]``)
+    in blocks of 256: ``mids`` the 255 midpoints of a sorted code on the device."""
+    _require_cuda(values, offset, mids)
+    v, o = values.contiguous(), offset.contiguous()
+    n = v.shape[-1]
+    codes = torch.empty(v.shape, dtype=torch.uint8, device=v.device)
+    absmax = torch.empty(*v.shape[:-1], -(-n // 256), dtype=torch.float32, device=v.device)
+    with torch.cuda.device(v.device):
+        N.check("e4b_quantize_8bit",
+                N.lib().e4b_quantize_8bit(v.data_ptr(), o.data_ptr(), o.numel(), n, mids.data_ptr(), zero_code,
+                                          codes.data_ptr(), absmax.data_ptr(), _stream(v.device)))
+    return codes, absmax
+
+
 # ------------------------------------------------------------------------------ routing
 
 

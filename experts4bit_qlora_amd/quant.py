@@ -126,14 +126,32 @@ def _host_table_4bit(quant_type: str):
     return tuple(mids.tolist()), tuple(perm.tolist()), int(torch.argmin(code.abs()).item())
 
 
-def _on_kernel(w: torch.Tensor, blocksize: int) -> bool:
-    """Whether a stack goes through ``e4b_quantize_4bit``: plain device tensors in blocks of 64 that
-    no transform or graph follows. The rest (other block sizes, the CPU, a stack that autograd
-    records, tensor subclasses) takes the torch formulation, which is the kernel's definition."""
-    return (w.is_cuda and blocksize == 64 and w.numel() > 0 and w.dim() > 0 and w.shape[-1] % 64 == 0
-            and type(w) in (torch.Tensor, torch.nn.Parameter) and w.is_floating_point()
+_DYNAMIC: dict = {}
+
+
+def _dynamic_table_on(device):
+    """(midpoints on ``device``, code of zero) of the dynamic map, made once per device."""
+    key = torch.device(device)
+    t = _DYNAMIC.get(key)
+    if t is None:
+        code = dynamic_map()
+        mids, perm = _thresholds(code)
+        assert torch.equal(perm, torch.arange(256))  # already sorted: a position is its code
+        t = _DYNAMIC[key] = (mids.to(key), int(torch.argmin(code.abs()).item()))
+    return t
+
+
+def _plain_on_device(w: torch.Tensor) -> bool:
+    """A device tensor that no transform or graph follows (a tensor subclass, or one that autograd
+    records, takes the torch formulation, which is the kernels' definition)."""
+    return (w.is_cuda and type(w) in (torch.Tensor, torch.nn.Parameter) and w.is_floating_point()
             and not (w.requires_grad and torch.is_grad_enabled())
             and not torch._C._functorch.is_functorch_wrapped_tensor(w))
+
+
+def _on_kernel(w: torch.Tensor, blocksize: int) -> bool:
+    """Whether a stack goes through ``e4b_quantize_4bit``: plain device tensors in blocks of 64."""
+    return (blocksize == 64 and w.numel() > 0 and w.dim() > 0 and w.shape[-1] % 64 == 0 and _plain_on_device(w))
 
 
 def quantize_4bit(w: torch.Tensor, quant_type: str = "nf4", blocksize: int = 64):
@@ -165,11 +183,18 @@ def _quantize_4bit_torch(w: torch.Tensor, quant_type: str, blocksize: int):
 def double_quant(absmax: torch.Tensor, blocksize2: int = _DQ_BLOCKSIZE2, code2: torch.Tensor | None = None):
     """Compress fp32 absmax ``[..., nb]`` -> (u8 codes, fp32 absmax2 ``[..., ceil(nb/256)]``,
     fp32 offset ``[...]``). ``offset`` is the mean (accumulated in fp64); the centred values are
-    quantized blockwise with the signed dynamic map."""
-    if code2 is None:
-        code2 = dynamic_map().to(absmax.device)
+    quantized blockwise with the signed dynamic map (on a HIP device, with the default map and
+    block size, by the library's kernel: bit for bit the torch formulation)."""
     a = absmax.float()
     offset = a.double().mean(dim=-1).float()
+    if code2 is None and blocksize2 == _DQ_BLOCKSIZE2 and a.numel() and _plain_on_device(a):
+        from . import ops
+
+        mids, zero = _dynamic_table_on(a.device)
+        q, absmax2 = ops.quantize_8bit(a.detach(), offset.detach(), mids, zero)
+        return q, absmax2, offset
+    if code2 is None:
+        code2 = dynamic_map().to(absmax.device)
     c = a - offset.unsqueeze(-1)
     nb = a.shape[-1]
     nb2 = -(-nb // blocksize2)

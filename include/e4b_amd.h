@@ -112,6 +112,13 @@ int e4b_dequant(const e4b_qweight* w, int32_t expert_begin, int32_t expert_count
 int e4b_quantize_4bit(const void* w, int32_t dtype, int64_t values, const float* mids, const uint8_t* codes,
                       int32_t zero_code, void* packed, float* absmax, hipStream_t stream);
 
+/* The second level of double quantization: rows [rows, n] of fp32 values, each less offset[row], in
+ * blocks of 256 (a row's last one padded with zeros) to a sorted 256-entry code given by its 255
+ * ascending midpoints `mids` on the device: absmax fp32 [rows, ceil(n / 256)] and codes u8 [rows, n] as
+ * e4b_quantize_4bit forms them. */
+int e4b_quantize_8bit(const float* values, const float* offset, int64_t rows, int64_t n, const float* mids,
+                      int32_t zero_code, uint8_t* codes, float* absmax, hipStream_t stream);
+
 /* Per-expert weight exponents for the fp16 matrix-core mode of e4b_moe_forward: shift[e] =
  * 141 - max(E_e, 20), E_e the largest biased fp32 exponent of expert e's block scales (the
  * decoded ones for NF4_DQ), so every |code * absmax| * 2^shift[e] is below 2^15 and the scaled

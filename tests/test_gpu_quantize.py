@@ -54,3 +54,18 @@ def test_views_other_dtypes_and_the_torch_route():
     assert not Q._on_kernel(w[:4096].view(64, 64), 32)
     recorded = w[:4096].view(64, 64).clone().requires_grad_()
     assert not Q._on_kernel(recorded, 64) and Q.quantize_4bit(recorded)[1].requires_grad
+
+
+@pytest.mark.parametrize("shape", ((1, 1), (3, 255), (2, 256), (5, 257), (7, 1000), (4096,)))
+def test_double_quant_is_the_torch_formulation(shape):
+    """Block edges, a padded last block, blocks of equal values (all zeros once the offset is off), a NaN."""
+    g = torch.Generator().manual_seed(3)
+    a = (torch.rand(shape, generator=g) * 0.1).to(DEV)
+    cases = [a, torch.full_like(a, 0.25), torch.zeros_like(a)]
+    if len(shape) == 2 and shape[0] > 2:
+        bad = a.clone()
+        bad[1, -1] = float("nan")
+        cases.append(bad)
+    for c in cases:
+        got, want = Q.double_quant(c), Q.double_quant(c, code2=Q.dynamic_map().to(DEV))
+        assert all(torch.equal(p.nan_to_num(-1.0), q.nan_to_num(-1.0)) and p.dtype == q.dtype for p, q in zip(got, want))
