@@ -87,6 +87,14 @@ void launch_mfma_gemm(const GemmArgs& a, hipStream_t s) {
       return;
     }
   }
+  if constexpr (DT == E4B_FP16 && FMT != E4B_FMT_MXFP4) {
+    // fp16 activations over 32-row tiles: the narrow kernel on exact weights, where K fits its steps
+    if (a.rt.tile_m == kTileMSmall && narrow_fits(a.w.k)) {
+      hipLaunchKernelGGL((gemm_narrow_kernel<FMT, false, false, true>), gemm_grid(a, kNarrowN), dim3(kNarrowThreads), 0,
+                         s, a);
+      return;
+    }
+  }
   const dim3 grid = gemm_grid(a, gemm_tile_nw(a.rt.tile_m));
   if (a.rt.tile_m == kTileMSmall) launch_mfma_bm<DT, FMT, kTileMSmall>(a, grid, s);
   else if (a.rt.tile_m == kTileMBig) launch_mfma_bm<DT, FMT, kTileMBig>(a, grid, s);

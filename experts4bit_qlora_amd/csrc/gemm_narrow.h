@@ -57,11 +57,18 @@ constexpr bool narrow_fits(int64_t k) { return k > 0 && k % (2 * kNarrowK) == 0 
 // LORA: the accumulators start as the tile's LoRA delta (p.lt, p.lb), scaled like the products
 // (lora_mfma.h).
 // H16: the down rows as fp16 with the operand scales left on (GemmArgs::out_f16_shift).
-template <int FMT, bool LORA = false, bool H16 = false>
+// EXACT: fp16 activations as they are and the reference's fp16 weights, fp16(code * scale) in one
+// rounding: the table holds fp32 code pairs (32 copies of 8 bytes: the same 64 KB) and each pair
+// takes two multiplies and a conversion instead of one packed multiply. Its lookups run one weight
+// sub-tile ahead, not one MFMA group (twice the registers per lookup). Against staging the weights
+// through LDS (gemm_mfma_kernel's 32-row tiles) the OLMoE layer at 150 tokens went 119 -> 97 us.
+template <int FMT, bool LORA = false, bool H16 = false, bool EXACT = false>
 __global__ void __launch_bounds__(kNarrowThreads) __attribute__((amdgpu_waves_per_eu(2)))
 gemm_narrow_kernel(GemmArgs p) {
   static_assert(FMT == E4B_FMT_NF4 || FMT == E4B_FMT_NF4_DQ, "narrow tiles: NF4 weights in fp16 mode");
   static_assert(!(H16 && LORA), "fp16 down rows without LoRA");
+  static_assert(!(EXACT && (LORA || H16)), "the exact form is the plain GEMM");
+  constexpr int DT = EXACT ? E4B_FP16 : E4B_BF16;  // activations and 16-bit outputs
   constexpr int BM = kTileMSmall, BN = kNarrowN, KS = kNarrowK, ST = kNarrowStages;
   constexpr int NS = BN / (kNarrowThreads / kWave) / 16;  // 4 weight sub-tiles per wave
   static_assert(kNarrowUnroll % ST == 0 && kNarrowUnroll % 6 == 0, "unroll: whole weight sets and scale sets");
@@ -136,7 +143,7 @@ gemm_narrow_kernel(GemmArgs p) {
     }
   }
   const float offset = (FMT == E4B_FMT_NF4_DQ) ? p.w.offset[e] : 0.0f;
-  const int wsh = p.w.shift[e];
+  const int wsh = EXACT ? 0 : p.w.shift[e];
 
   // ---- activation rows: thread t stages row t / 8, the 16-byte groups 2 c and 2 c + 1 of a
   // step (c = t % 8): K = 64 (c / 2) + 32 t + 16 (c % 2) .. + 15 of the pair, t the step in it
@@ -153,7 +160,7 @@ gemm_narrow_kernel(GemmArgs p) {
   // the row's exponent, loaded ahead of the activation and weight loads: stored to row_shift_s
   // before the first barrier, it was the last load of the prologue, and the wait for it was a
   // wait for all of them (step 2's weights included)
-  const int a_exp_row = p.a_exp[src];
+  const int a_exp_row = EXACT ? 0 : p.a_exp[src];
 
   // The tile's rows as MS 16-row MFMA sub-tiles: one when the tile holds at most 16 rows (a
   // mid-size batch's experts and most prefill tails hold a few rows each), halving the MFMAs and
@@ -210,14 +217,23 @@ gemm_narrow_kernel(GemmArgs p) {
     float hi[16], lo[4];
 #pragma unroll
     for (int c = 0; c < 16; ++c) hi[c] = p.w.code[c];
+    if constexpr (EXACT) {  // copy t % 32 of entries (t / 32) + 8 i
+      const int e0 = tid >> 5;
+      lo[0] = p.w.code[e0];
+      lo[1] = p.w.code[e0 + 8];
+      float2* const fill = reinterpret_cast<float2*>(ptab) + e0 * (kNarrowCopies / 2) + (tid & 31);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) lo[c] = p.w.code[w0 + 4 * c];
+      for (int i = 0; i < 256 / 8; ++i) fill[8 * i * (kNarrowCopies / 2)] = make_float2(hi[i >> 1], lo[i & 1]);
+    } else {
 #pragma unroll
-    for (int i = 0; i < 256 / 4; ++i)
-      ptab[(w0 + 4 * i) * kNarrowCopies + lane] = cvt_pair<E4B_FP16>(hi[i >> 2], lo[i & 3]);
+      for (int c = 0; c < 4; ++c) lo[c] = p.w.code[w0 + 4 * c];
+#pragma unroll
+      for (int i = 0; i < 256 / 4; ++i)
+        ptab[(w0 + 4 * i) * kNarrowCopies + lane] = cvt_pair<E4B_FP16>(hi[i >> 2], lo[i & 3]);
+    }
   }
   if constexpr (FMT == E4B_FMT_NF4_DQ) code2_s[tid] = p.w.code2[tid];
-  if ((tid & 7) == 0) row_shift_s[ar] = exp_shift(a_exp_row);
+  if (!EXACT && (tid & 7) == 0) row_shift_s[ar] = exp_shift(a_exp_row);
   store_a(0);
   load_a(0, min(2, last));
   __syncthreads();
@@ -250,11 +266,12 @@ gemm_narrow_kernel(GemmArgs p) {
   // fragment group slots of the lane for MFMA j: (4 g + j) ^ (row % 16), row % 16 = lane % 16
   const int fslot = (4 * g) ^ l16;
   const int frow = l16 * KS;
-  const uint32_t copy_off = static_cast<uint32_t>(lane) * 4u;
+  const uint32_t copy_off = EXACT ? static_cast<uint32_t>(lane & 31) * 8u : static_cast<uint32_t>(lane) * 4u;
   auto lookup = [&](uint32_t w, uint32_t sel) -> uint32_t {
     const uint32_t addr = __builtin_amdgcn_perm(w, copy_off, sel);
     return *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(ptab) + addr);
   };
+  // a block's scale: as an fp16 pair with 2^shift applied, EXACT: the fp32 scale's bits
   auto scale_pair = [&](int pset, int ns, int pr) -> uint32_t {
     float sc;
     if constexpr (FMT == E4B_FMT_NF4) {
@@ -265,6 +282,7 @@ gemm_narrow_kernel(GemmArgs p) {
       const float prod = code2_s[sq[pset][ns]] * a2;
       sc = prod + offset;
     }
+    if constexpr (EXACT) return __float_as_uint(sc);
     sc = __builtin_amdgcn_ldexpf(sc, wsh);  // exact: a power of two
     return cvt_pair<E4B_FP16>(sc, sc);
   };
@@ -272,7 +290,16 @@ gemm_narrow_kernel(GemmArgs p) {
   uint32_t s2[NS];  // the block scale pairs of the current pair of steps
   // Table lookups of the four words (MFMA j) of each weight sub-tile: raw[j % 2], issued one
   // MFMA group ahead of their use, so that their LDS latency runs under the MFMAs.
-  uint32_t raw[2][NS][4];
+  uint32_t raw[EXACT ? 1 : 2][EXACT ? 1 : NS][4];
+  float2 rawx[EXACT ? 2 : 1][4];
+  auto look_exact = [&](const uint4& wv, auto J, float2 (&dst)[4]) {
+    constexpr int j = decltype(J)::value;
+    const uint32_t w = j == 0 ? wv.x : j == 1 ? wv.y : j == 2 ? wv.z : wv.w;
+    static_for<4>([&](auto b) {
+      const uint32_t addr = __builtin_amdgcn_perm(w, copy_off, 0x0c0c0400u + 0x100u * int(b));
+      dst[int(b)] = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(ptab) + addr);
+    });
+  };
   auto look = [&](const uint4& wv, auto J, uint32_t (&dst)[4]) {
     constexpr int j = decltype(J)::value;
     const uint32_t w = j == 0 ? wv.x : j == 1 ? wv.y : j == 2 ? wv.z : wv.w;
@@ -314,11 +341,26 @@ gemm_narrow_kernel(GemmArgs p) {
       static_for<NS>([&](auto NSI) {
         constexpr int ns = decltype(NSI)::value;
         uint4 bv;
-        bv.x = pk_mul_f16(raw[j & 1][ns][0], s2[ns]);
-        bv.y = pk_mul_f16(raw[j & 1][ns][1], s2[ns]);
-        bv.z = pk_mul_f16(raw[j & 1][ns][2], s2[ns]);
-        bv.w = pk_mul_f16(raw[j & 1][ns][3], s2[ns]);
-        if constexpr (j < 3) look(wq[set][ns], std::integral_constant<int, j + 1>{}, raw[(j + 1) & 1][ns]);
+        if constexpr (EXACT) {
+          const float sc = __uint_as_float(s2[ns]);
+          uint32_t o[4];
+#pragma unroll
+          for (int b = 0; b < 4; ++b) {
+            const float2 c = rawx[(NS * j + ns) & 1][b];
+            o[b] = cvt_pair<E4B_FP16>(c.x * sc, c.y * sc);
+          }
+          bv = make_uint4(o[0], o[1], o[2], o[3]);
+          constexpr int nx = ns + 1 < NS ? ns + 1 : 0, jx = ns + 1 < NS ? j : (j + 1) & 3;
+          constexpr int wx = ns + 1 == NS && j == 3 ? nset : set;
+          look_exact(wq[wx][nx], std::integral_constant<int, jx>{}, rawx[(NS * j + ns + 1) & 1]);
+        } else {
+          bv.x = pk_mul_f16(raw[j & 1][ns][0], s2[ns]);
+          bv.y = pk_mul_f16(raw[j & 1][ns][1], s2[ns]);
+          bv.z = pk_mul_f16(raw[j & 1][ns][2], s2[ns]);
+          bv.w = pk_mul_f16(raw[j & 1][ns][3], s2[ns]);
+        }
+        if constexpr (EXACT) {
+        } else if constexpr (j < 3) look(wq[set][ns], std::integral_constant<int, j + 1>{}, raw[(j + 1) & 1][ns]);
         else look(wq[nset][ns], std::integral_constant<int, 0>{}, raw[0][ns]);
 #pragma unroll
         for (int ms = 0; ms < MS; ++ms) acc[ms][ns] = mfma_16x16x32<E4B_FP16>(fa[ms][j], bv, acc[ms][ns]);
@@ -330,9 +372,13 @@ gemm_narrow_kernel(GemmArgs p) {
     if constexpr (u & 1) load_scales(((u + 3) >> 1) % PS, min(s + 3, last) >> 1);
     __syncthreads();  // step s + 1's activations are in place
   };
-  // the lookups of step 0, group 0
+  // the lookups of step 0, group 0 (EXACT: its first sub-tile)
+  if constexpr (EXACT) {
+    look_exact(wq[0][0], std::integral_constant<int, 0>{}, rawx[0]);
+  } else {
 #pragma unroll
-  for (int ns = 0; ns < NS; ++ns) look(wq[0][ns], std::integral_constant<int, 0>{}, raw[0][ns]);
+    for (int ns = 0; ns < NS; ++ns) look(wq[0][ns], std::integral_constant<int, 0>{}, raw[0][ns]);
+  }
   const int smain = steps - steps % kNarrowUnroll;
   for (int s0 = 0; s0 < smain; s0 += kNarrowUnroll) {
     static_for<kNarrowUnroll>([&](auto U) { step(U, s0 + decltype(U)::value); });
@@ -343,6 +389,7 @@ gemm_narrow_kernel(GemmArgs p) {
 
   // ---- epilogue: lane holds D[4 g + i][lane % 16] of each 16 x 16 sub-tile; the operand
   // scales come off first, 2^-(row shift + expert shift), exact
+  if constexpr (!EXACT) {
 #pragma unroll
   for (int ms = 0; ms < MS; ++ms)
 #pragma unroll
@@ -351,6 +398,7 @@ gemm_narrow_kernel(GemmArgs p) {
 #pragma unroll
       for (int ns = 0; ns < NS; ++ns) acc[ms][ns][i] = __builtin_amdgcn_ldexpf(acc[ms][ns][i], d);
     }
+  }
   const bool has_bias = p.w.bias != nullptr;
   const uint16_t* bias = static_cast<const uint16_t*>(p.w.bias);
   if (!H16 && pair) {
@@ -366,7 +414,7 @@ gemm_narrow_kernel(GemmArgs p) {
 #pragma unroll
           for (int ns = 0; ns < 2; ++ns) {
             const float v = silu_f32(acc[ms][ns][i]) * acc[ms][ns + 2][i];
-            if (rr < row_end && cbase + ns * 16 < p.n_out) orow[ns * 16] = from_f<E4B_BF16>(v);
+            if (rr < row_end && cbase + ns * 16 < p.n_out) orow[ns * 16] = from_f<DT>(v);
           }
         }
       return;
@@ -381,9 +429,9 @@ gemm_narrow_kernel(GemmArgs p) {
         for (int ns = 0; ns < 2; ++ns) {
           const int64_t jj = cbase + ns * 16;
           if (jj >= p.n_out) continue;
-          const float bg = has_bias ? to_f<E4B_BF16>(bias[int64_t(e) * n + jj]) : 0.0f;
-          const float bu = has_bias ? to_f<E4B_BF16>(bias[int64_t(e) * n + n / 2 + jj]) : 0.0f;
-          store_elem<E4B_BF16>(p, int64_t(rr) * p.n_out + jj,
+          const float bg = has_bias ? to_f<DT>(bias[int64_t(e) * n + jj]) : 0.0f;
+          const float bu = has_bias ? to_f<DT>(bias[int64_t(e) * n + n / 2 + jj]) : 0.0f;
+          store_elem<DT>(p, int64_t(rr) * p.n_out + jj,
                                gated(p.epi, acc[ms][ns][i], acc[ms][ns + 2][i], p.alpha, p.limit, bg, bu));
         }
       }
@@ -428,8 +476,8 @@ gemm_narrow_kernel(GemmArgs p) {
       for (int ns = 0; ns < NS; ++ns) {
         const int64_t nn = cbase + ns * 16;
         if (nn >= p.n_out) continue;
-        const float b = has_bias ? to_f<E4B_BF16>(bias[int64_t(e) * n + nn]) : 0.0f;
-        store_elem<E4B_BF16>(p, int64_t(rr) * p.n_out + nn, single(p.epi, acc[ms][ns][i], b));
+        const float b = has_bias ? to_f<DT>(bias[int64_t(e) * n + nn]) : 0.0f;
+        store_elem<DT>(p, int64_t(rr) * p.n_out + nn, single(p.epi, acc[ms][ns][i], b));
       }
     }
   };
