@@ -113,13 +113,18 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
 def _layer_inputs(lora_mod, x, top_k_index, top_k_weights):
     """(epilogue, limit, weights, adapters) for ``_FusedLoraLayer``, or None where the layer goes through the
     per-projection functions: a compute dtype other than bf16, a base whose activation only its own
-    Python code knows, adapters of mixed dtypes, dtypes and shapes the library does not take."""
+    Python code knows, adapters of mixed dtypes or of two ranks, dtypes and shapes the library does
+    not take (it reads all four adapters by one rank, so their shapes are checked here)."""
     from . import fast as F
 
     base = lora_mod.base
     epi = F._fused_epilogue(base)
     adapters = (lora_mod.gate_up_lora_A, lora_mod.gate_up_lora_B, lora_mod.down_lora_A, lora_mod.down_lora_B)
     known = (torch.bfloat16, torch.float16, torch.float32)
+    E, r = base.num_experts, adapters[0].shape[1] if adapters[0].dim() == 3 else -1
+    (n1, k1), (n2, k2) = base._gate_up_shape, base._down_shape
+    if [tuple(a.shape) for a in adapters] != [(E, r, k1), (E, n1, r), (E, r, k2), (E, n2, r)]:
+        return None
     if (epi is None or x.dtype != torch.bfloat16 or top_k_weights.dtype not in known
             or any(a.dtype != adapters[0].dtype for a in adapters) or adapters[0].dtype not in known
             or x.dim() != 2 or x.shape[1] != base._down_shape[0] or top_k_index.shape != top_k_weights.shape
