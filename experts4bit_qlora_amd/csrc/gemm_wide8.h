@@ -12,7 +12,7 @@
 // of the tile in one wave each weight is still decoded exactly once per tile. Against staging the
 // decoded weights in LDS (eight waves of 128 x 64) a step writes 32 KB and reads 64 KB less there
 // and its barrier waits for no decode: launches alone, Qwen3 gate_up / down at 4,096 tokens
-// 272 / 173 -> 244 / 150 us, both gpt-oss projections at 2,048 tokens 665 -> ~500 us. What is left:
+// 272 / 173 -> 235 / 145 us, both gpt-oss projections at 2,048 tokens 665 -> ~500 us. What is left:
 // the matrix cores' own rate (a register-only loop of these MFMAs on random data is held to
 // 1.6 PFLOP/s by the card's power limit, 1.4 with one fragment read per MFMA), ~12 us per tile
 // before its first and after its last step, and the last round's idle CUs.
