@@ -120,8 +120,10 @@ def quantize_blocks(w: torch.Tensor, code: torch.Tensor, blocksize: int):
 
 @functools.lru_cache(maxsize=None)
 def _host_table_4bit(quant_type: str):
-    """(midpoints, code per sorted position, code of zero) of a 4-bit code as host values."""
-    code = code_4bit(quant_type)
+    """(midpoints, code per sorted position, code of zero) of a 4-bit code as host values (made on the
+    CPU whatever the default device: a model may be built under ``torch.device("meta")``)."""
+    with torch.device("cpu"):
+        code = code_4bit(quant_type)
     mids, perm = _thresholds(code)
     return tuple(mids.tolist()), tuple(perm.tolist()), int(torch.argmin(code.abs()).item())
 
@@ -134,9 +136,10 @@ def _dynamic_table_on(device):
     key = torch.device(device)
     t = _DYNAMIC.get(key)
     if t is None:
-        code = dynamic_map()
+        with torch.device("cpu"):
+            code = dynamic_map()
         mids, perm = _thresholds(code)
-        assert torch.equal(perm, torch.arange(256))  # already sorted: a position is its code
+        assert perm.tolist() == list(range(256))  # already sorted: a position is its code
         t = _DYNAMIC[key] = (mids.to(key), int(torch.argmin(code.abs()).item()))
     return t
 

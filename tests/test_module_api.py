@@ -43,6 +43,15 @@ def test_quantizer_matches_oracle_bytes():
     assert (p.numpy() != op).mean() < 1e-4  # midpoint ties are measure-zero
 
 
+@pytest.mark.parametrize("quant_type", ("nf4", "fp4"))
+def test_quantizer_tables_do_not_follow_the_default_device(quant_type):
+    want = Q._host_table_4bit(quant_type)
+    with torch.device("meta"):
+        assert Q._host_table_4bit.__wrapped__(quant_type) == want
+        Q._DYNAMIC.pop(torch.device("cpu"), None)
+        assert Q._dynamic_table_on("cpu")[0].shape == (255,) and Q._dynamic_table_on("cpu")[0].device.type == "cpu"
+
+
 def test_mxfp4_quantizer_matches_oracle_bytes():
     w = torch.randn(4, 2880) * 0.02
     b, s = Q.quantize_mxfp4(w)
