@@ -73,6 +73,13 @@ E4B_DEV uint32_t pack2(uint16_t lo, uint16_t hi) {
 // the shift and its inverse stay normal fp32 powers of two.
 __host__ __device__ inline int exp_shift(int e) { return 141 - (e > 20 ? e : 20); }
 
+// The largest weight shift of a tile whose accumulators also hold a LoRA delta (lora_mfma.h). exp_shift is 121
+// for all-zero weights, and a delta of ordinary size times 2^(row shift + 121) is beyond fp32. Capped, the
+// weights keep their fp16 bits down to block scales of 2^-74 (zeros are exact under any shift). The
+// row shift needs no cap: t shrinks with its row, |t| 2^(row shift) <= 2^15 sum |A|, so a delta fits up
+// to |lscale B| sum |A| of 2^49.
+constexpr int kDeltaShiftMax = 64;
+
 // Largest biased exponent among the 8 bf16 values of a 16-byte piece, in bits 7..14.
 E4B_DEV uint32_t bf16_exp_max(const uint4& v) {
   auto m2 = [](uint32_t w) { return max(w & 0x7f80u, (w >> 16) & 0x7f80u); };

@@ -96,7 +96,7 @@ E4B_DEV void dgrad_wide_tile(const Dgrad16Args& p, int e, int row0, int row_end,
 #pragma unroll
   for (int i = 0; i < AP; ++i)
     aoff[i] = static_cast<uint32_t>((int64_t(min(row0 + 64 * i + (tid >> 3), row_end - 1)) * n) / 8 + (tid & 7));
-  const int wsh = p.w.shift[e];
+  const int wsh = min(p.w.shift[e], kDeltaShiftMax);
   const int g_exp_row = p.g_exp[min(row0 + (tid & (BM - 1)), row_end - 1)];
   // weights: thread t decodes columns 32 (t % 8) .. + 31 of weight row t / 8 of the step (columns past k
   // read column 0: never stored)
@@ -356,7 +356,7 @@ dgrad_narrow_kernel(Dgrad16Args p) {
   // the lane's eight columns (columns past k read column 0: never stored) and its gradient row
   const int64_t cl = c0 + 8 * c32 < K ? c0 + 8 * c32 : 0;
   const int grow = min(row0 + c32, row_end - 1);
-  const int wsh = p.w.shift[e];
+  const int wsh = min(p.w.shift[e], kDeltaShiftMax);
   const int rsh = exp_shift(p.g_exp[grow]);
   const float offset = (FMT == E4B_FMT_NF4_DQ) ? p.w.offset[e] : 0.0f;
   {

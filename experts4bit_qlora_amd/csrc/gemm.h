@@ -388,7 +388,7 @@ __global__ void __launch_bounds__(gemm_threads(BM)) gemm_mfma_kernel(GemmArgs p)
   // fp16 mode: the tile row's activation shift (for the epilogue) and the expert's weight shift
   int wsh = 0;
   if constexpr (F16C) {
-    wsh = p.w.shift[e];
+    wsh = LORA ? min(p.w.shift[e], kDeltaShiftMax) : p.w.shift[e];
     if (tid % TPR == 0) row_shift_s[ar] = exp_shift(p.a_exp[src]);
   }
 

@@ -143,7 +143,7 @@ gemm_narrow_kernel(GemmArgs p) {
     }
   }
   const float offset = (FMT == E4B_FMT_NF4_DQ) ? p.w.offset[e] : 0.0f;
-  const int wsh = EXACT ? 0 : p.w.shift[e];
+  const int wsh = EXACT ? 0 : LORA ? min(p.w.shift[e], kDeltaShiftMax) : p.w.shift[e];
 
   // ---- activation rows: thread t stages row t / 8, the 16-byte groups 2 c and 2 c + 1 of a
   // step (c = t % 8): K = 64 (c / 2) + 32 t + 16 (c % 2) .. + 15 of the pair, t the step in it

@@ -98,7 +98,7 @@ E4B_DEV void wide8_tile(const GemmArgs& p, const Wide8Rows& tr, int n_tile, uint
       aoff[i] = static_cast<uint32_t>((src * k) / 8 + apart);
     }
   }
-  const int wsh = F16C ? p.w.shift[e] : 0;
+  const int wsh = F16C ? (LORA ? min(p.w.shift[e], kDeltaShiftMax) : p.w.shift[e]) : 0;
   // the exponent of tile row t (t < BM), stored to row_shift_s (the epilogue's shifts) once the
   // first steps' loads are out
   const int a_exp_row = F16C ? p.a_exp[row_src(row0 + (tid & (kWideTileM - 1)), tr.sf[4])] : 0;

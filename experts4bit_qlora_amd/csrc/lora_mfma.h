@@ -31,8 +31,9 @@ E4B_DEV void split_bf16x8(const float (&v)[8], uint4& hi, uint4& lo) {
   lo = make_uint4(l[0], l[1], l[2], l[3]);
 }
 
-// 2^e * lscale * t[m, q0 + i] (0 past the rank), i = 0..7, split. With the rank a multiple of 8
-// the eight values are two 16-byte loads, else eight element loads.
+// lscale * (2^e * t[m, q0 + i]) (0 past the rank), i = 0..7, split: the power of two goes to t, which is as
+// small as e is large. With the rank a multiple of 8 the eight values are two 16-byte loads, else
+// eight element loads.
 template <class Args>
 E4B_DEV void lora_t_piece(const Args& p, int64_t m, int q0, int e2, uint4& hi, uint4& lo) {
   float v[8];
@@ -45,9 +46,8 @@ E4B_DEV void lora_t_piece(const Args& p, int64_t m, int q0, int e2, uint4& hi, u
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = t[q0 + i < p.lr ? q0 + i : 0];
   }
-  const float sc = __builtin_amdgcn_ldexpf(p.lscale, e2);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = q0 + i < p.lr ? v[i] * sc : 0.0f;
+  for (int i = 0; i < 8; ++i) v[i] = q0 + i < p.lr ? __builtin_amdgcn_ldexpf(v[i], e2) * p.lscale : 0.0f;
   split_bf16x8(v, hi, lo);
 }
 
