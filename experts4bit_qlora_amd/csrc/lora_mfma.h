@@ -15,8 +15,45 @@
 #pragma once
 
 #include "gemm.h"
+#include "lora.h"
 
 namespace e4b {
+
+// The leading bf16 part of v, taken off it, in the upper half of the result: truncated, so it never overflows
+// and three parts hold any finite fp32 value exactly (two any fp16 one). FIRST (v may be any value): an
+// infinity or NaN is its own first part and leaves zeros.
+template <bool FIRST>
+E4B_DEV uint32_t bf16_part(float& v) {
+  if constexpr (FIRST) v = __builtin_canonicalizef(v);  // a NaN keeps a bit of its upper half
+  const uint32_t b = __float_as_uint(v);
+  const float rest = v - __uint_as_float(b & 0xffff0000u);
+  v = !FIRST || __builtin_isfinite(v) ? rest : 0.0f;
+  return b;
+}
+
+// Bf16 parts that hold an adapter value of dtype DT exactly.
+template <int DT>
+constexpr int kAdapterParts = DT == E4B_BF16 ? 1 : DT == E4B_FP16 ? 2 : 3;
+
+// 8 fp32 values as NP bf16 parts, MFMA operand pieces (value 2i in the low half of word i).
+template <int NP>
+E4B_DEV void split_parts8(const float (&v)[8], uint4 (&part)[NP]) {
+  uint32_t w[NP][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = v[2 * i], b = v[2 * i + 1];
+    static_for<NP>([&](auto q) __attribute__((always_inline)) {
+      if constexpr (int(q) == NP - 1) {
+        w[q][i] = cvt_pair<E4B_BF16>(a, b);  // what is left fits a part: exact
+      } else {
+        const uint32_t pa = bf16_part<int(q) == 0>(a), pb = bf16_part<int(q) == 0>(b);
+        w[q][i] = __builtin_amdgcn_perm(pb, pa, 0x07060302u);
+      }
+    });
+  }
+#pragma unroll
+  for (int q = 0; q < NP; ++q) part[q] = make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
+}
 
 // 8 fp32 values -> their bf16 hi and lo halves as two MFMA operand pieces (value 2i in the low
 // half of word i).
@@ -140,11 +177,10 @@ namespace e4b {
 // t[m, q] = sum_c x_m[c] * A[e, q, c] for the sorted rows m of every routing tile (one expert per
 // tile), on the matrix cores: the t of the fp16-mode LoRA path (rows past the routed ones are not
 // written). One workgroup per BM-row part of a tile, one wave per 16 rows, each wave all ranks of
-// its rows (NSM 16-rank blocks) on v_mfma_f32_16x16x32_bf16. x rows are bf16 (exact operands); A
-// (bf16, fp16 or fp32) is staged per 64-deep chunk in LDS as bf16 hi / lo halves (lo = bf16(a -
-// hi), the split of split_bf16x8), so t carries about 16 significant bits of each product of an
-// fp32 or fp16 adapter and every product of a bf16 one exactly. The chunks are double-buffered,
-// one barrier per chunk, with A two chunks and x three chunks ahead in registers: a launch has only
+// its rows (NSM 16-rank blocks) on v_mfma_f32_16x16x32_bf16. x rows are bf16 (exact operands); A is
+// staged per 64-deep chunk in LDS as its bf16 parts (one of a bf16, two of an fp16, three of an fp32
+// adapter: split_parts8), so every product is exact and t is an fp32 sum, as the VALU passes
+// (lora_a_kernel) form it. The chunks are double-buffered, one barrier per chunk, with A two chunks and x three chunks ahead in registers: a launch has only
 // a workgroup or two per CU, so the x loads in flight per wave set its rate (one chunk ahead: 43 us
 // for both of an OLMoE layer's t at 1,531 tokens, 31 us so).
 constexpr int kLoraTK = 64;  // K per chunk
@@ -155,16 +191,39 @@ constexpr int kLoraTGroups = kLoraTK / 8;
 // group spread over all banks.
 E4B_DEV int lora_t_at(int q, int g) { return q * kLoraTK + (((g ^ q) & 7) << 3); }
 
+// The sums of t and u. One fp32 accumulator over the whole row was 1.5 times as far from 64 bits as the
+// vector units' 64 partial sums; here at most four products of 32 columns add up (each half of a chunk and
+// the adapters' lower parts apart) before they go to the total, whose rounding errors are kept (two-sum).
+template <int NSM>
+struct RankSums {
+  f32x4_t acc[3][NSM], total[NSM], lost[NSM];
+  E4B_DEV RankSums() {
+    const f32x4_t zero{0.0f, 0.0f, 0.0f, 0.0f};
+    static_for<NSM>([&](auto n) __attribute__((always_inline)) {
+      acc[0][n] = acc[1][n] = acc[2][n] = total[n] = lost[n] = zero;
+    });
+  }
+  E4B_DEV void fold() {
+    static_for<2 * NSM>([&](auto j) __attribute__((always_inline)) {
+      f32x4_t &a = acc[int(j) & 1][int(j) / 2], &t = total[int(j) / 2];
+      const f32x4_t s = t + a, b = s - t;
+      lost[int(j) / 2] += (t - (s - b)) + (a - b);
+      t = s;
+      a = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    });
+  }
+  E4B_DEV float value(int n, int i) const { return total[n][i] + (lost[n][i] + acc[2][n][i]); }
+};
+
 template <int ADT, int BM, int NSM>
 __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint16_t* __restrict__ x, int gather_k,
                                                                       e4b_routing rt, const void* __restrict__ A,
                                                                       int rank, int64_t in, float* __restrict__ t) {
   constexpr int NT = BM / 16 * kWave;
-  constexpr bool LO = ADT != E4B_BF16;  // bf16 adapters have no lo half
+  constexpr int NP = kAdapterParts<ADT>;
   constexpr int NSTAGE = 16 * NSM * kLoraTGroups;  // 16-byte groups per chunk
   constexpr int SPT = (NSTAGE + NT - 1) / NT;      // staging groups per thread
-  __shared__ __align__(16) uint16_t ah[2][16 * NSM * kLoraTK];
-  __shared__ __align__(16) uint16_t al[LO ? 2 : 1][LO ? 16 * NSM * kLoraTK : 8];
+  __shared__ __align__(16) uint16_t as[NP][2][16 * NSM * kLoraTK];
   const int sub = rt.tile_m / BM;
   const int tile = static_cast<int>(blockIdx.x) / sub;
   if (tile >= rt.meta[0]) return;  // uniform
@@ -184,45 +243,31 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
 
   // staging: thread tid takes groups j = tid + NT i of the chunk's [16 NSM ranks][8 groups]
   float sets[2][SPT][8];
-  auto load_a = [&](auto set, int c) {
+  // (inlined always: a call left standing would put the sets in scratch memory)
+  auto load_a = [&](auto set, int c) __attribute__((always_inline)) {
     float (&sv)[SPT][8] = sets[decltype(set)::value];
-#pragma unroll
-    for (int i = 0; i < SPT; ++i) {
-      const int j = tid + NT * i;
-      if (NSTAGE % NT != 0 && j >= NSTAGE) break;
+    static_for<SPT>([&](auto i) __attribute__((always_inline)) {
+      const int j = tid + NT * int(i);
+      if (NSTAGE % NT != 0 && j >= NSTAGE) return;
       const int q = min(j / kLoraTGroups, rank - 1), gg = j % kLoraTGroups;
       const int64_t o = (int64_t(e) * rank + q) * in + int64_t(c) * kLoraTK + 8 * gg;
-      if constexpr (ADT == E4B_FP32) {
-        const float4 a = *reinterpret_cast<const float4*>(static_cast<const float*>(A) + o);
-        const float4 b = *reinterpret_cast<const float4*>(static_cast<const float*>(A) + o + 4);
-        sv[i][0] = a.x; sv[i][1] = a.y; sv[i][2] = a.z; sv[i][3] = a.w;
-        sv[i][4] = b.x; sv[i][5] = b.y; sv[i][6] = b.z; sv[i][7] = b.w;
-      } else {
-        const uint4 a = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(A) + o);
-        const uint32_t wv[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          sv[i][2 * h] = to_f<ADT>(static_cast<uint16_t>(wv[h]));
-          sv[i][2 * h + 1] = to_f<ADT>(static_cast<uint16_t>(wv[h] >> 16));
-        }
-      }
-    }
+      load8<ADT>(A, o, sv[i]);
+    });
   };
-  auto store_a = [&](auto set, int buf) {
+  auto store_a = [&](auto set, int buf) __attribute__((always_inline)) {
     const float (&sv)[SPT][8] = sets[decltype(set)::value];
-#pragma unroll
-    for (int i = 0; i < SPT; ++i) {
-      const int j = tid + NT * i;
-      if (NSTAGE % NT != 0 && j >= NSTAGE) break;
+    static_for<SPT>([&](auto i) __attribute__((always_inline)) {
+      const int j = tid + NT * int(i);
+      if (NSTAGE % NT != 0 && j >= NSTAGE) return;
       const int q = j / kLoraTGroups, gg = j % kLoraTGroups;
       float v[8];
 #pragma unroll
       for (int h = 0; h < 8; ++h) v[h] = q < rank ? sv[i][h] : 0.0f;
-      uint4 hi, lo;
-      split_bf16x8(v, hi, lo);
-      *reinterpret_cast<uint4*>(&ah[buf][lora_t_at(q, gg)]) = hi;
-      if constexpr (LO) *reinterpret_cast<uint4*>(&al[buf][lora_t_at(q, gg)]) = lo;
-    }
+      uint4 part[NP];
+      split_parts8<NP>(v, part);
+#pragma unroll
+      for (int h = 0; h < NP; ++h) *reinterpret_cast<uint4*>(&as[h][buf][lora_t_at(q, gg)]) = part[h];
+    });
   };
   // x fragments of a chunk: 32-deep step s takes columns 32 s + 8 g .. + 7
   auto load_x = [&](uint4 (&xf)[2], int c) {
@@ -231,9 +276,7 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
       xf[s] = *reinterpret_cast<const uint4*>(xr + int64_t(c) * kLoraTK + 32 * s + 8 * g);
   };
 
-  f32x4_t acc[NSM];
-#pragma unroll
-  for (int i = 0; i < NSM; ++i) acc[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  RankSums<NSM> sums;
   // chunk c from LDS buffer c % 2 and x set c % 4; meanwhile chunk c + 1's A goes from registers (set
   // (c + 1) % 2) into the other buffer, chunk c + 2's A and chunk c + 3's x are requested
   uint4 xs[4][2];
@@ -242,19 +285,15 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
     constexpr int cur = u & 1;
     load_a(std::integral_constant<int, cur>{}, chunk(c + 2));
     load_x(xs[(u + 3) & 3], chunk(c + 3));
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-#pragma unroll
-      for (int ns = 0; ns < NSM; ++ns) {
-        const int at = lora_t_at(16 * ns + l16, 4 * s + g);
-        const uint4 bh = *reinterpret_cast<const uint4*>(&ah[cur][at]);
-        acc[ns] = mfma_16x16x32<E4B_BF16>(xs[u][s], bh, acc[ns]);
-        if constexpr (LO) {
-          const uint4 bl = *reinterpret_cast<const uint4*>(&al[cur][at]);
-          acc[ns] = mfma_16x16x32<E4B_BF16>(xs[u][s], bl, acc[ns]);
-        }
-      }
-    }
+    static_for<2>([&](auto s) __attribute__((always_inline)) {
+      static_for<NSM>([&](auto ns) __attribute__((always_inline)) {
+        const int at = lora_t_at(16 * int(ns) + l16, 4 * int(s) + g);
+        static_for<NP>([&](auto h) __attribute__((always_inline)) {
+          f32x4_t& to = sums.acc[int(h) == 0 ? int(s) : 2][ns];
+          to = mfma_16x16x32<E4B_BF16>(xs[u][s], *reinterpret_cast<const uint4*>(&as[h][cur][at]), to);
+        });
+      });
+    });
     store_a(std::integral_constant<int, cur ^ 1>{}, cur ^ 1);  // its last readers passed the previous barrier
     __syncthreads();
   };
@@ -265,10 +304,14 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
   store_a(std::integral_constant<int, 0>{}, 0);
   __syncthreads();
   int c = 0;
-  for (; c + 4 <= nchunks; c += 4) static_for<4>([&](auto u) { step(u, c + int(u)); });
+  for (; c + 4 <= nchunks; c += 4) {
+    static_for<4>([&](auto u) { step(u, c + int(u)); });
+    sums.fold();
+  }
   static_for<3>([&](auto u) {
     if (c + int(u) < nchunks) step(u, c + int(u));
   });
+  sums.fold();
   // lane holds t[row 16 w + 4 g + i][rank 16 ns + l16]
 #pragma unroll
   for (int ns = 0; ns < NSM; ++ns) {
@@ -276,7 +319,7 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 16 * w + 4 * g + i;
-      if (q < rank && r < rows) t[int64_t(row0 + r) * rank + q] = acc[ns][i];
+      if (q < rank && r < rows) t[int64_t(row0 + r) * rank + q] = sums.value(ns, i);
     }
   }
 }

@@ -278,16 +278,6 @@ E4B_DEV int wgrad_at(int row, int col) {
          (col & 15);
 }
 
-// The leading bf16 part of v, taken off it: truncated, so it never overflows and three parts hold
-// any finite fp32 value exactly; an infinity or NaN is its own first part and leaves zeros.
-E4B_DEV uint16_t bf16_part(float& v) {
-  const uint32_t b = __float_as_uint(v);
-  const bool fin = (b & 0x7f800000u) != 0x7f800000u;
-  const uint16_t part = fin ? static_cast<uint16_t>(b >> 16) : from_f<E4B_BF16>(v);
-  v = fin ? v - __uint_as_float(b & 0xffff0000u) : 0.0f;
-  return part;
-}
-
 // out[e, j, c] = scale * sum_{m in expert e's rows} u[m, j] * a_m[c], for j < r, c < cols; zero for an
 // expert without rows. Block = (columns 128 * blockIdx.x .., expert blockIdx.y); a_m = row
 // sorted_flat[m] / gather_k of a (gather_k > 0) or row m. TRANS: out[e, c, j] (a B gradient in its
@@ -365,9 +355,9 @@ __global__ void __launch_bounds__(kWgradThreads) lora_wgrad_kernel(const float* 
       const int idx = tid + kWgradThreads * i, row = idx / RB, j = idx % RB;
       const int at = wgrad_at<RB>(row, j & ~3) + (j & 3);
       float v = m0 + row < end && j < r ? uv[i] : 0.0f;
-      us[0][at] = bf16_part(v);
-      us[1][at] = bf16_part(v);
-      us[2][at] = bf16_part(v);
+      us[0][at] = static_cast<uint16_t>(bf16_part<true>(v) >> 16);
+      us[1][at] = static_cast<uint16_t>(bf16_part<false>(v) >> 16);
+      us[2][at] = static_cast<uint16_t>(__float_as_uint(v) >> 16);  // eight bits are left
     }
   };
   // operand of a 32-row step: rows 32 s + 8 g .. + 7 of column base + lane % 16
@@ -403,8 +393,8 @@ __global__ void __launch_bounds__(kWgradThreads) lora_wgrad_kernel(const float* 
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             float v0 = lo_f<XDT>(w[i]), v1 = hi_f<XDT>(w[i]);
-            const uint16_t h0 = bf16_part(v0), h1 = bf16_part(v1);
-            h[i] = pack2(h0, h1);
+            const uint32_t h0 = bf16_part<true>(v0), h1 = bf16_part<true>(v1);
+            h[i] = __builtin_amdgcn_perm(h1, h0, 0x07060302u);
             l[i] = cvt_pair<E4B_BF16>(v0, v1);
           }
           ah[t] = make_uint4(h[0], h[1], h[2], h[3]);

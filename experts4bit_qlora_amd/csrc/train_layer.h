@@ -198,7 +198,7 @@ __global__ void __launch_bounds__(kRowThreads) combine_bwd_kernel(const void* __
 
 // u[m, q] = sum_c g_m[c] * B[e, c, q] for the sorted rows of every routing tile: lora_t_mfma_kernel with
 // the adapter matrix in the other orientation (its ranks contiguous), so a 64-deep chunk is staged in
-// LDS as it lies in memory ([64 c][ranks], bf16 hi / lo halves) and its operands come from
+// LDS as it lies in memory ([64 c][ranks], one array per bf16 part) and its operands come from
 // transposing reads instead of a transposed copy of B. VEC: whole 16-byte pieces of ranks (rank a
 // multiple of 8, B aligned), a template argument because a branch around the loads makes every
 // later wait a wait for all of them (both of an OLMoE step's u at 2,048 tokens: 105 -> 67 us).
@@ -208,11 +208,10 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_u_mfma_kernel(const uint
                                                                       float* __restrict__ u) {
   constexpr int NT = BM / 16 * kWave;
   constexpr int RB = 16 * NSM;
-  constexpr bool LO = BDT != E4B_BF16;
+  constexpr int NP = kAdapterParts<BDT>;
   constexpr int NSTAGE = kLoraTK * RB / 8;     // 8-rank groups per chunk
   constexpr int SPT = (NSTAGE + NT - 1) / NT;  // per thread
-  __shared__ __align__(16) uint16_t bh[2][kLoraTK * RB];
-  __shared__ __align__(16) uint16_t bl[LO ? 2 : 1][LO ? kLoraTK * RB : 8];
+  __shared__ __align__(16) uint16_t bs[NP][2][kLoraTK * RB];
   const int sub = rt.tile_m / BM;
   const int tile = static_cast<int>(blockIdx.x) / sub;
   if (tile >= rt.meta[0]) return;  // uniform
@@ -227,7 +226,7 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_u_mfma_kernel(const uint
   const int nchunks = static_cast<int>(n / kLoraTK);
   auto chunk = [&](int c) { return min(c, nchunks - 1); };  // past the last chunk it is re-read
   float sets[2][SPT][8];
-  auto load_b = [&](auto set, int c) {
+  auto load_b = [&](auto set, int c) __attribute__((always_inline)) {
     float (&sv)[SPT][8] = sets[decltype(set)::value];
 #pragma unroll
     for (int i = 0; i < SPT; ++i) {
@@ -245,17 +244,17 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_u_mfma_kernel(const uint
       for (int h = 0; h < 8; ++h) sv[i][h] = q0 + h < rank ? sv[i][h] : 0.0f;
     }
   };
-  auto store_b = [&](auto set, int buf) {
+  auto store_b = [&](auto set, int buf) __attribute__((always_inline)) {
     const float (&sv)[SPT][8] = sets[decltype(set)::value];
 #pragma unroll
     for (int i = 0; i < SPT; ++i) {
       const int j = tid + NT * i;
       if (NSTAGE % NT != 0 && j >= NSTAGE) break;
       const int at = wgrad_at<RB>(j / (RB / 8), 8 * (j % (RB / 8)));
-      uint4 hi, lo;
-      split_bf16x8(sv[i], hi, lo);
-      *reinterpret_cast<uint4*>(&bh[buf][at]) = hi;
-      if constexpr (LO) *reinterpret_cast<uint4*>(&bl[buf][at]) = lo;
+      uint4 part[NP];
+      split_parts8<NP>(sv[i], part);
+#pragma unroll
+      for (int h = 0; h < NP; ++h) *reinterpret_cast<uint4*>(&bs[h][buf][at]) = part[h];
     }
   };
   auto load_x = [&](uint4 (&xf)[2], int c) {
@@ -269,22 +268,21 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_u_mfma_kernel(const uint
     const uint2 hi = lds_read_tr(b + wgrad_at<RB>(row + 4, col));
     return make_uint4(lo.x, lo.y, hi.x, hi.y);
   };
-  f32x4_t acc[NSM];
-#pragma unroll
-  for (int i = 0; i < NSM; ++i) acc[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  RankSums<NSM> sums;
   uint4 xs[4][2];  // B two chunks and g three chunks ahead, as lora_t_mfma_kernel
   auto step = [&](auto uc, int c) __attribute__((always_inline)) {
     constexpr int v = decltype(uc)::value;  // c % 4
     constexpr int cur = v & 1;
     load_b(std::integral_constant<int, cur>{}, chunk(c + 2));
     load_x(xs[(v + 3) & 3], chunk(c + 3));
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int ns = 0; ns < NSM; ++ns) {
-        acc[ns] = mfma_16x16x32<E4B_BF16>(xs[v][s], operand(bh[cur], s, 16 * ns), acc[ns]);
-        if constexpr (LO) acc[ns] = mfma_16x16x32<E4B_BF16>(xs[v][s], operand(bl[cur], s, 16 * ns), acc[ns]);
-      }
+    static_for<2>([&](auto s) __attribute__((always_inline)) {
+      static_for<NSM>([&](auto ns) __attribute__((always_inline)) {
+        static_for<NP>([&](auto h) __attribute__((always_inline)) {
+          f32x4_t& to = sums.acc[int(h) == 0 ? int(s) : 2][ns];
+          to = mfma_16x16x32<E4B_BF16>(xs[v][s], operand(bs[h][cur], s, 16 * ns), to);
+        });
+      });
+    });
     store_b(std::integral_constant<int, cur ^ 1>{}, cur ^ 1);  // its last readers passed the previous barrier
     __syncthreads();
   };
@@ -295,17 +293,21 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_u_mfma_kernel(const uint
   store_b(std::integral_constant<int, 0>{}, 0);
   __syncthreads();
   int c = 0;
-  for (; c + 4 <= nchunks; c += 4) static_for<4>([&](auto q) { step(q, c + int(q)); });
+  for (; c + 4 <= nchunks; c += 4) {
+    static_for<4>([&](auto q) { step(q, c + int(q)); });
+    sums.fold();
+  }
   static_for<3>([&](auto q) {
     if (c + int(q) < nchunks) step(q, c + int(q));
   });
+  sums.fold();
 #pragma unroll
   for (int ns = 0; ns < NSM; ++ns) {
     const int q = 16 * ns + l16;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 16 * w + 4 * gr + i;
-      if (q < rank && r < rows) u[int64_t(row0 + r) * rank + q] = acc[ns][i];
+      if (q < rank && r < rows) u[int64_t(row0 + r) * rank + q] = sums.value(ns, i);
     }
   }
 }
