@@ -188,9 +188,13 @@ E4B_DEV void dgrad_wide_tile(const Dgrad16Args& p, int e, int row0, int row_end,
   if (tid < BM) row_shift_s[tid] = exp_shift(g_exp_row);
   __syncthreads();  // code2 table, code-pair table, row shifts
   if (p.lt) {
-    // the accumulators start as the tile's delta, scaled like the products
+    // the accumulators start as the tile's delta, scaled like the products; gradient buffer 1 is free until
+    // step 0, one barrier further on
+    uint16_t* const ts = As[1];
     for (int q0 = 0; q0 < p.lr; q0 += 16) {
-      uint4 bh[NS], bl[NS];
+      if (q0) __syncthreads();  // the last step's t is read
+      lora_t_stage<BM, kDgradWideThreads>(p, ts, row0, row_end - 1, row_shift_s, q0);
+      uint4 b[NS][3];
 #pragma unroll
       for (int ns = 0; ns < NS; ++ns) {
         const int64_t c = c0 + 64 * wave_c + 32 * ns + c32;
@@ -201,16 +205,18 @@ E4B_DEV void dgrad_wide_tile(const Dgrad16Args& p, int e, int row0, int row_end,
           const float x = adapter_at(p.la, p.lbdt, (int64_t(e) * p.lr + (q < p.lr ? q : 0)) * K + (c < K ? c : 0));
           v[i] = q < p.lr ? __builtin_amdgcn_ldexpf(x, wsh) : 0.0f;
         }
-        split_bf16x8(v, bh[ns], bl[ns]);
+        split_parts8<3>(v, b[ns]);
       }
+      __syncthreads();
       static_for<MS>([&](auto ms) {
-        const int r = wave_m * (BM / 2) + 32 * int(ms) + c32;
-        uint4 ah, al;
-        lora_t_piece(p, min(row0 + r, row_end - 1), q0 + 8 * half, row_shift_s[r], ah, al);
+        uint4 t[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          t[i] = reinterpret_cast<const uint4*>(ts)[(2 * i + half) * BM + wave_m * (BM / 2) + 32 * int(ms) + c32];
         static_for<NS>([&](auto ns) {
-          acc[ms][ns] = mfma_32x32x16<E4B_BF16>(bh[ns], ah, acc[ms][ns]);
-          acc[ms][ns] = mfma_32x32x16<E4B_BF16>(bh[ns], al, acc[ms][ns]);
-          acc[ms][ns] = mfma_32x32x16<E4B_BF16>(bl[ns], ah, acc[ms][ns]);
+          delta_products(p.lbdt, [&](auto i, auto j) {
+            acc[ms][ns] = mfma_32x32x16<E4B_BF16>(b[ns][j], t[i], acc[ms][ns]);
+          });
         });
       });
     }
@@ -447,8 +453,8 @@ dgrad_narrow_kernel(Dgrad16Args p) {
   __syncthreads();  // tables
   if (p.lt) {  // the delta, scaled like the products: wave w takes the 16-rank steps w, w + 4, ...
     for (int q0 = 16 * wid; q0 < p.lr; q0 += 64) {
-      uint4 ah, al;
-      lora_t_piece(p, grow, q0 + 8 * half, rsh, ah, al);
+      uint4 t[3];
+      lora_t_piece(p, grow, q0 + 8 * half, rsh, t);
       static_for<NB>([&](auto b) {
         float v[8];
 #pragma unroll
@@ -457,11 +463,9 @@ dgrad_narrow_kernel(Dgrad16Args p) {
           const float x = adapter_at(p.la, p.lbdt, (int64_t(e) * p.lr + (q < p.lr ? q : 0)) * K + cl + int(b));
           v[i] = q < p.lr ? __builtin_amdgcn_ldexpf(x, wsh) : 0.0f;
         }
-        uint4 bh, bl;
-        split_bf16x8(v, bh, bl);
-        acc[b] = mfma_32x32x16<E4B_BF16>(bh, ah, acc[b]);
-        acc[b] = mfma_32x32x16<E4B_BF16>(bh, al, acc[b]);
-        acc[b] = mfma_32x32x16<E4B_BF16>(bl, ah, acc[b]);
+        uint4 a[3];
+        split_parts8<3>(v, a);
+        delta_products(p.lbdt, [&](auto i, auto j) { acc[b] = mfma_32x32x16<E4B_BF16>(a[j], t[i], acc[b]); });
       });
     }
   }

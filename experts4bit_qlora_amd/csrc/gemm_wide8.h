@@ -206,11 +206,11 @@ E4B_DEV void wide8_tile(const GemmArgs& p, const Wide8Rows& tr, int n_tile, uint
   if (F16C && tid < BM) row_shift_s[tid] = exp_shift(a_exp_row);
   __syncthreads();  // code2 table, code-pair table, row shifts
   if constexpr (LORA) {
-    // the accumulators start as the tile's LoRA delta, scaled like the products (lora_mfma.h):
-    // the lane's t rows (clamped to the expert's rows: the rest is never stored) times their
-    // activation shifts, the B row of its column times the expert's weight shift
-    lora_delta_32x32<MS>(p, acc, e, row0 + c32, row_end - 1, [&](int ms) { return row_shift_s[c32 + 32 * ms]; }, wsh,
-                         grow, lane);
+    // the accumulators start as the tile's LoRA delta, scaled like the products (lora_mfma.h): the rows' t
+    // (clamped to the expert's rows: the rest is never stored) times their activation shifts, the B row
+    // of the lane's column times the expert's weight shift. Activation buffer 1 is free until step 0,
+    // one barrier further on
+    lora_delta_32x32<BM, NT>(p, acc, e, row0, row_end - 1, row_shift_s, wsh, grow, As[1], lane);
   }
   // step 0's activations into buffer 0; their registers take step 1
 #pragma unroll

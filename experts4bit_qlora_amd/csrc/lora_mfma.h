@@ -1,17 +1,15 @@
 // The LoRA delta of a grouped GEMM tile, on the matrix cores, in the tile's fp32 accumulators
-// (the LORA instances of gemm_wide8_kernel and gemm_narrow_kernel):
+// (the LORA instances of gemm_wide8_kernel, gemm_narrow_kernel and gemm_mfma_kernel):
 //
 //   acc[m, j] += lscale * sum_q t[m, q] * B[e, row(j), q]
 //
-// a rank-r product of the tile's t rows (t = x . A^T, fp32, from lora_a_kernel) and the B rows of
-// the tile's weight rows. Both operands are split into bf16 pairs, v = hi + lo with hi = bf16(v)
-// and lo = bf16(v - hi) (the subtraction is exact), and the product is formed as hi.hi + lo.hi +
-// hi.lo on bf16 MFMAs with fp32 accumulation: every bf16 x bf16 product is exact in fp32 and the
-// dropped lo.lo term is below 2^-16 of |t||B|, so the delta carries about 16 significant bits
-// (bf16 adapters have lo = 0 and skip the third product). The extra MFMAs are r / 16 x 3 per
-// 32 x 32 block (about 2 % of a 256 x 256 gate_up tile's at rank 16): the delta costs no pass
-// over the GEMM's output rows. Operands come straight from global memory, once per tile, at the
-// tile's start (the accumulators begin as the scaled delta).
+// a rank-r product of the tile's t rows (t = x . A^T, fp32, from lora_t_mfma_kernel below) and the B
+// rows of the tile's weight rows. Both operands are split into bf16 parts (t into three, B into as many
+// as its dtype needs: split_parts8), exactly, and multiplied part by part on bf16 MFMAs with fp32
+// accumulation: every product is exact, so the delta is an fp32 sum as the vector passes (lora.h)
+// form it. At rank 16 the eight products of an fp32 adapter are about 5 % of a 256 x 256 gate_up tile's
+// MFMAs; the delta costs no pass over the GEMM's output rows. Operands come straight from global
+// memory, once per tile, at the tile's start (the accumulators begin as the scaled delta).
 #pragma once
 
 #include "gemm.h"
@@ -55,24 +53,33 @@ E4B_DEV void split_parts8(const float (&v)[8], uint4 (&part)[NP]) {
   for (int q = 0; q < NP; ++q) part[q] = make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
 }
 
-// 8 fp32 values -> their bf16 hi and lo halves as two MFMA operand pieces (value 2i in the low
-// half of word i).
-E4B_DEV void split_bf16x8(const float (&v)[8], uint4& hi, uint4& lo) {
-  uint32_t h[4], l[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    h[i] = cvt_pair<E4B_BF16>(v[2 * i], v[2 * i + 1]);
-    l[i] = cvt_pair<E4B_BF16>(v[2 * i] - lo_f<E4B_BF16>(h[i]), v[2 * i + 1] - hi_f<E4B_BF16>(h[i]));
+// The products of a delta: mul(i, j) for part i of t and part j of the adapter (of dtype dt), all but the
+// product of the two last parts (below 2^-28 of |t||adapter|), the smaller ones first.
+template <class F>
+E4B_DEV void delta_products(int dt, F&& mul) {
+  using std::integral_constant;
+  constexpr integral_constant<int, 0> p0{};
+  constexpr integral_constant<int, 1> p1{};
+  constexpr integral_constant<int, 2> p2{};
+  if (dt == E4B_FP32) {
+    mul(p1, p2);
+    mul(p0, p2);
   }
-  hi = make_uint4(h[0], h[1], h[2], h[3]);
-  lo = make_uint4(l[0], l[1], l[2], l[3]);
+  if (dt != E4B_BF16) {
+    mul(p2, p1);
+    mul(p1, p1);
+    mul(p0, p1);
+  }
+  mul(p2, p0);
+  mul(p1, p0);
+  mul(p0, p0);
 }
 
 // lscale * (2^e * t[m, q0 + i]) (0 past the rank), i = 0..7, split: the power of two goes to t, which is as
 // small as e is large. With the rank a multiple of 8 the eight values are two 16-byte loads, else
 // eight element loads.
 template <class Args>
-E4B_DEV void lora_t_piece(const Args& p, int64_t m, int q0, int e2, uint4& hi, uint4& lo) {
+E4B_DEV void lora_t_piece(const Args& p, int64_t m, int q0, int e2, uint4 (&part)[3]) {
   float v[8];
   const float* t = p.lt + m * p.lr;
   if ((p.lr & 7) == 0) {
@@ -85,11 +92,11 @@ E4B_DEV void lora_t_piece(const Args& p, int64_t m, int q0, int e2, uint4& hi, u
   }
 #pragma unroll
   for (int i = 0; i < 8; ++i) v[i] = q0 + i < p.lr ? __builtin_amdgcn_ldexpf(v[i], e2) * p.lscale : 0.0f;
-  split_bf16x8(v, hi, lo);
+  split_parts8<3>(v, part);
 }
 
-// 2^e * B[e, row, q0 + i] (0 past the rank), i = 0..7, from the adapter dtype, split.
-E4B_DEV void lora_b_piece(const GemmArgs& p, int ex, int64_t row, int q0, int e2, uint4& hi, uint4& lo) {
+// 2^e * B[ex, row, q0 + i] (0 past the rank), i = 0..7, from the adapter dtype, split.
+E4B_DEV void lora_b_piece(const GemmArgs& p, int ex, int64_t row, int q0, int e2, uint4 (&part)[3]) {
   float v[8];
   const int64_t base = (int64_t(ex) * p.w.n + row) * p.lr;
   const int64_t q0c = q0 < p.lr ? q0 : 0;
@@ -117,29 +124,45 @@ E4B_DEV void lora_b_piece(const GemmArgs& p, int ex, int64_t row, int q0, int e2
   }
 #pragma unroll
   for (int i = 0; i < 8; ++i) v[i] = q0 + i < p.lr ? __builtin_amdgcn_ldexpf(v[i], e2) : 0.0f;
-  split_bf16x8(v, hi, lo);
+  split_parts8<3>(v, part);
 }
 
-// The delta of a wave's 32 x 32 accumulator blocks, weights first (v_mfma_f32_32x32x16: lane l
-// supplies weight / tile row l % 32 and the eight ranks 8 (l / 32) .. of each 16-rank step), scaled
-// like the fp16 mode's products: t row of block ms = min(arow0 + 32 ms, arow_last), times
-// 2^ashift(ms) (its activation row's shift, exact); B row brow, times 2^bshift (the expert's weight
-// shift). Run on zeroed accumulators before a tile's main loop, where its loads overlap the tile's
-// first loads and few registers are live; the epilogue then removes the scales from the sum.
-template <int MS, class AS>
-E4B_DEV void lora_delta_32x32(const GemmArgs& p, f32x16_t (&acc)[MS], int e, int64_t arow0, int64_t arow_last,
-                              AS&& ashift, int bshift, int64_t brow, int lane) {
-  const int g8 = 8 * (lane >> 5);
-  const bool b_lo = p.lbdt != E4B_BF16;  // a bf16 B has no lo half
+// The t operands of a workgroup's BM rows and the 16 ranks from q0, split once for all its waves, in LDS (ts:
+// 48 BM values): part i of row r, ranks 8 h .. of the step, at 16-byte piece (2 i + h) BM + r. Row r is
+// min(row0 + r, row_last), times 2^shift[r].
+template <int BM, int NT, class Args>
+E4B_DEV void lora_t_stage(const Args& p, uint16_t* ts, int64_t row0, int64_t row_last, const int* shift, int q0) {
+  for (int j = threadIdx.x; j < 2 * BM; j += NT) {
+    const int r = j % BM, h = j / BM;
+    uint4 part[3];
+    lora_t_piece(p, min(row0 + r, row_last), q0 + 8 * h, shift[r], part);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) reinterpret_cast<uint4*>(ts)[(2 * i + h) * BM + r] = part[i];
+  }
+}
+
+// The delta of the 32 x 32 accumulator blocks of eight waves that each hold all BM rows, weights first
+// (v_mfma_f32_32x32x16: lane l supplies weight / tile row l % 32 and the eight ranks 8 (l / 32) .. of
+// each 16-rank step), scaled like the fp16 mode's products: t rows times 2^shift (their activation row's,
+// exact); B row brow, times 2^bshift (the expert's weight shift). Run on zeroed accumulators before a
+// tile's main loop; the epilogue then removes the scales from the sum. ts: LDS that nothing else touches
+// until the workgroup's next barrier. With every wave splitting all the rows' t itself an OLMoE layer at
+// 1,531 tokens took 331 us, so 319.
+template <int BM, int NT>
+E4B_DEV void lora_delta_32x32(const GemmArgs& p, f32x16_t (&acc)[BM / 32], int e, int64_t row0, int64_t row_last,
+                              const int* shift, int bshift, int64_t brow, uint16_t* ts, int lane) {
+  const int half = lane >> 5;
   for (int q0 = 0; q0 < p.lr; q0 += 16) {
-    uint4 bh, bl;
-    lora_b_piece(p, e, brow, q0 + g8, bshift, bh, bl);
-    static_for<MS>([&](auto ms) {
-      uint4 ah, al;
-      lora_t_piece(p, min(arow0 + 32 * int(ms), arow_last), q0 + g8, ashift(int(ms)), ah, al);
-      acc[ms] = mfma_32x32x16<E4B_BF16>(bh, ah, acc[ms]);
-      acc[ms] = mfma_32x32x16<E4B_BF16>(bh, al, acc[ms]);
-      if (b_lo) acc[ms] = mfma_32x32x16<E4B_BF16>(bl, ah, acc[ms]);
+    if (q0) __syncthreads();  // the last step's t is read
+    lora_t_stage<BM, NT>(p, ts, row0, row_last, shift, q0);
+    uint4 b[3];
+    lora_b_piece(p, e, brow, q0 + 8 * half, bshift, b);
+    __syncthreads();
+    static_for<BM / 32>([&](auto ms) {
+      uint4 t[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) t[i] = reinterpret_cast<const uint4*>(ts)[(2 * i + half) * BM + 32 * int(ms) + (lane & 31)];
+      delta_products(p.lbdt, [&](auto i, auto j) { acc[ms] = mfma_32x32x16<E4B_BF16>(b[j], t[i], acc[ms]); });
     });
   }
 }
@@ -151,22 +174,17 @@ template <int MS, int NS, class AS>
 E4B_DEV void lora_delta_16x16(const GemmArgs& p, f32x4_t (&acc)[MS][NS], int e, int64_t arow0, int64_t arow_last,
                               AS&& ashift, int bshift, const int64_t (&brow)[NS], int lane) {
   const int g8 = 8 * (lane >> 4);
-  const bool b_lo = p.lbdt != E4B_BF16;
   for (int q0 = 0; q0 < p.lr; q0 += 32) {
-    uint4 bh[NS], bl[NS];
+    uint4 t[MS][3];
 #pragma unroll
-    for (int ns = 0; ns < NS; ++ns) lora_b_piece(p, e, brow[ns], q0 + g8, bshift, bh[ns], bl[ns]);
-#pragma unroll
-    for (int ms = 0; ms < MS; ++ms) {
-      uint4 ah, al;
-      lora_t_piece(p, min(arow0 + 16 * ms, arow_last), q0 + g8, ashift(ms), ah, al);
-#pragma unroll
-      for (int ns = 0; ns < NS; ++ns) {
-        acc[ms][ns] = mfma_16x16x32<E4B_BF16>(ah, bh[ns], acc[ms][ns]);
-        acc[ms][ns] = mfma_16x16x32<E4B_BF16>(al, bh[ns], acc[ms][ns]);
-        if (b_lo) acc[ms][ns] = mfma_16x16x32<E4B_BF16>(ah, bl[ns], acc[ms][ns]);
-      }
-    }
+    for (int ms = 0; ms < MS; ++ms) lora_t_piece(p, min(arow0 + 16 * ms, arow_last), q0 + g8, ashift(ms), t[ms]);
+    static_for<NS>([&](auto ns) {
+      uint4 b[3];
+      lora_b_piece(p, e, brow[ns], q0 + g8, bshift, b);
+      static_for<MS>([&](auto ms) {
+        delta_products(p.lbdt, [&](auto i, auto j) { acc[ms][ns] = mfma_16x16x32<E4B_BF16>(t[ms][i], b[j], acc[ms][ns]); });
+      });
+    });
   }
 }
 

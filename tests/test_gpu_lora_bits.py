@@ -8,6 +8,7 @@ import experts4bit_qlora_amd as e4b
 from experts4bit_qlora_amd import _native as N
 from experts4bit_qlora_amd import fast as F
 from experts4bit_qlora_amd import ops
+from experts4bit_qlora_amd import quant as Q
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -111,3 +112,54 @@ def test_t_is_no_further_from_64_bits_than_the_vector_units():
     got, ref = ((v.double() - want).norm() / want.norm() for v in (t1, old))
     print(f"t rel error {got:.3e}, vector units {ref:.3e}", flush=True)
     assert got <= ref
+
+
+def _zero_layer(hid, inter):
+    """Descriptors of one ungated expert whose block scales are all zero."""
+    code = Q.code_4bit("nf4", DEV)
+    return [ops.with_weight_shift(ops.nf4_qweight(torch.zeros(1, n * k // 2, dtype=torch.uint8, device=DEV),
+                                                  torch.zeros(1, n * k // 64, device=DEV), code, n, k, num_experts=1))
+            for n, k in ((inter, hid), (hid, inter))]
+
+
+# (1 + 2^-9 + 2^-18) - (1 + 2^-9), and the last bits of (1 + 2^-9)^2 less its first two terms
+CANCEL = [((1 + 2.0 ** -9 + 2.0 ** -18, 1 + 2.0 ** -9), (1.0, -1.0)),
+          ((1.0, 1.0), (1 + 2.0 ** -9 + 2.0 ** -18, -1 - 2.0 ** -9)),
+          ((1 + 2.0 ** -9, 1.0), (1 + 2.0 ** -9, -1 - 2.0 ** -8))]
+
+
+@pytest.mark.parametrize("T,hid,inter", [(150, 192, 256), (300, 256, 192), (20, 256, 256), (20, 192, 320)])
+@pytest.mark.parametrize("adt", (torch.float32, torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("case", range(len(CANCEL)))
+def test_deltas_keep_32_bits(T, hid, inter, adt, case):
+    """Deltas t . B (forward) and u . A (backward) of two ranks that cancel to 2^-18, over zero weights:
+    halved and whole 256-row tiles, 32-row tiles with K a multiple of 256 and not. Every product and sum is exact,
+    so the rows are equal. An adapter dtype that cannot hold the case's values is left out."""
+    _announce(f"delta bits T={T} hid={hid} inter={inter} {adt} case={case}")
+    (t0, t1), (b0, b1) = CANCEL[case]
+    pair = torch.tensor([b0, b1], device=DEV)
+    if not torch.equal(pair.to(adt).float(), pair):
+        pytest.skip("the dtype rounds these adapters")
+    w1, w2 = _zero_layer(hid, inter)
+    bits = torch.zeros(hid, device=DEV)
+    bits[:3] = torch.tensor([1.0, 2.0 ** -9, 2.0 ** -18])
+    x = bits.expand(T, hid).to(torch.bfloat16).contiguous()
+    pick = lambda v: torch.tensor([1.0, float(v >= 1 + 2.0 ** -9), float(v > 1 + 2.0 ** -9)], device=DEV)  # noqa: E731
+    side = lambda n: torch.nn.functional.pad(torch.stack([pick(t0), pick(t1)]), (0, n - 3))  # [2, n]  # noqa: E731
+    idx, w = torch.zeros(T, 1, dtype=torch.int64, device=DEV), torch.ones(T, 1, device=DEV)
+    one = lambda v: v.to(adt).unsqueeze(0).contiguous()  # noqa: E731
+    # forward: t = (t0, t1), B1 rows (b0, b1)
+    lora = (one(side(hid)), one(pair.expand(inter, 2)), one(torch.zeros(2, inter, device=DEV)),
+            one(torch.zeros(hid, 2, device=DEV)))
+    _, saved = ops.train_forward(x, idx, w, w1, w2, lora, 1.0, N.EPI_ACT, 0.0, torch.float32)
+    size = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    at = saved.numel() - 2 * size(8 * T) - size(2 * T * hid) - 2 * size(2 * T * inter)
+    proj = saved[at:at + 2 * T * inter].view(torch.bfloat16)
+    assert torch.all(proj == 2.0 ** -18), proj
+    # backward: u = (t0, t1) from the gradient x and B2, A2 columns (b0, b1); proj = 0, so dL/dproj = dh / 2, and with
+    # t1 = 1 in both ranks dL/dB1 = T dh / 2
+    lora = (one(torch.nn.functional.pad(torch.ones(2, 1, device=DEV), (0, hid - 1))), one(torch.zeros(inter, 2, device=DEV)),
+            one(pair[:, None].expand(2, inter)), one(side(hid).t()))
+    _, saved = ops.train_forward(x, idx, w, w1, w2, lora, 1.0, N.EPI_ACT, 0.0, torch.float32)
+    grads = ops.train_backward(x, x, w, w1, w2, lora, 1.0, N.EPI_ACT, 0.0, saved, (False,) * 3 + (True, False, False))
+    assert torch.all(grads[3].float() == torch.tensor(T * 2.0 ** -19).to(adt).float().item()), grads[3]
