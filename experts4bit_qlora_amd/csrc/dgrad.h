@@ -58,13 +58,6 @@ E4B_DEV uint2 lds_read_tr(const uint16_t* p) {
   return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(p)));
 }
 
-// A value of the adapter, in its dtype.
-E4B_DEV float adapter_at(const void* a, int dt, int64_t i) {
-  if (dt == E4B_FP32) return static_cast<const float*>(a)[i];
-  const uint16_t v = static_cast<const uint16_t*>(a)[i];
-  return dt == E4B_BF16 ? to_f<E4B_BF16>(v) : to_f<E4B_FP16>(v);
-}
-
 // Eight 16-bit columns of the lane's row from two runs of four packed into two words each (v, and w the
 // run eight columns on), the lane halves holding columns 4 (l / 32) .. of each run: after the swap
 // the lower half stores the first run's eight columns, the upper half the second's.
@@ -194,7 +187,7 @@ E4B_DEV void dgrad_wide_tile(const Dgrad16Args& p, int e, int row0, int row_end,
     for (int q0 = 0; q0 < p.lr; q0 += 16) {
       if (q0) __syncthreads();  // the last step's t is read
       lora_t_stage<BM, kDgradWideThreads>(p, ts, row0, row_end - 1, row_shift_s, q0);
-      uint4 b[NS][3];
+      uint4 b[NS][4];
 #pragma unroll
       for (int ns = 0; ns < NS; ++ns) {
         const int64_t c = c0 + 64 * wave_c + 32 * ns + c32;
@@ -205,17 +198,17 @@ E4B_DEV void dgrad_wide_tile(const Dgrad16Args& p, int e, int row0, int row_end,
           const float x = adapter_at(p.la, p.lbdt, (int64_t(e) * p.lr + (q < p.lr ? q : 0)) * K + (c < K ? c : 0));
           v[i] = q < p.lr ? __builtin_amdgcn_ldexpf(x, wsh) : 0.0f;
         }
-        split_parts8<3>(v, b[ns]);
+        delta_parts8(v, b[ns]);
       }
       __syncthreads();
       static_for<MS>([&](auto ms) {
-        uint4 t[3];
+        uint4 t[4];
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
+        for (int i = 0; i < 4; ++i)
           t[i] = reinterpret_cast<const uint4*>(ts)[(2 * i + half) * BM + wave_m * (BM / 2) + 32 * int(ms) + c32];
         static_for<NS>([&](auto ns) {
-          delta_products(p.lbdt, [&](auto i, auto j) {
-            acc[ms][ns] = mfma_32x32x16<E4B_BF16>(b[ns][j], t[i], acc[ms][ns]);
+          delta_products(p.lbdt, t, b[ns], [&](const uint4& tp, const uint4& bp) {
+            acc[ms][ns] = mfma_32x32x16<E4B_BF16>(bp, tp, acc[ms][ns]);
           });
         });
       });
@@ -453,7 +446,7 @@ dgrad_narrow_kernel(Dgrad16Args p) {
   __syncthreads();  // tables
   if (p.lt) {  // the delta, scaled like the products: wave w takes the 16-rank steps w, w + 4, ...
     for (int q0 = 16 * wid; q0 < p.lr; q0 += 64) {
-      uint4 t[3];
+      uint4 t[4];
       lora_t_piece(p, grow, q0 + 8 * half, rsh, t);
       static_for<NB>([&](auto b) {
         float v[8];
@@ -463,9 +456,9 @@ dgrad_narrow_kernel(Dgrad16Args p) {
           const float x = adapter_at(p.la, p.lbdt, (int64_t(e) * p.lr + (q < p.lr ? q : 0)) * K + cl + int(b));
           v[i] = q < p.lr ? __builtin_amdgcn_ldexpf(x, wsh) : 0.0f;
         }
-        uint4 a[3];
-        split_parts8<3>(v, a);
-        delta_products(p.lbdt, [&](auto i, auto j) { acc[b] = mfma_32x32x16<E4B_BF16>(a[j], t[i], acc[b]); });
+        uint4 a[4];
+        delta_parts8(v, a);
+        delta_products(p.lbdt, t, a, [&](const uint4& tp, const uint4& ap) { acc[b] = mfma_32x32x16<E4B_BF16>(ap, tp, acc[b]); });
       });
     }
   }

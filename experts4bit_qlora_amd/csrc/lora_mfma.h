@@ -17,6 +17,13 @@
 
 namespace e4b {
 
+// A value of the adapter, in its dtype.
+E4B_DEV float adapter_at(const void* a, int dt, int64_t i) {
+  if (dt == E4B_FP32) return static_cast<const float*>(a)[i];
+  const uint16_t v = static_cast<const uint16_t*>(a)[i];
+  return dt == E4B_BF16 ? to_f<E4B_BF16>(v) : to_f<E4B_FP16>(v);
+}
+
 // The leading bf16 part of v, taken off it, in the upper half of the result: truncated, so it never overflows
 // and three parts hold any finite fp32 value exactly (two any fp16 one). FIRST (v may be any value): an
 // infinity or NaN is its own first part and leaves zeros.
@@ -27,6 +34,18 @@ E4B_DEV uint32_t bf16_part(float& v) {
   const float rest = v - __uint_as_float(b & 0xffff0000u);
   v = !FIRST || __builtin_isfinite(v) ? rest : 0.0f;
   return b;
+}
+
+// bf16 pairs with their infinities and NaNs as zeros, for a delta's products with the other side's lower
+// parts: those are zero wherever the leading part is all of the value, and an infinity times that zero
+// would make the sum a NaN. (t, u and the weight gradients form a sum that comes out NaN again instead,
+// value by value: cleaning their operands as they are read cost the 2,048-token training step 1.5 %.)
+E4B_DEV uint32_t finite_pair(uint32_t w) {
+  const uint32_t inf = ((w & 0x7f807f80u) + 0x00800080u) & 0x80008000u;  // exponents of all ones, in bits 15 and 31
+  return w & ~((inf - (inf >> 15)) | inf);
+}
+E4B_DEV uint4 finite8(const uint4& v) {
+  return make_uint4(finite_pair(v.x), finite_pair(v.y), finite_pair(v.z), finite_pair(v.w));
 }
 
 // Bf16 parts that hold an adapter value of dtype DT exactly.
@@ -53,33 +72,37 @@ E4B_DEV void split_parts8(const float (&v)[8], uint4 (&part)[NP]) {
   for (int q = 0; q < NP; ++q) part[q] = make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
 }
 
-// The products of a delta: mul(i, j) for part i of t and part j of the adapter (of dtype dt), all but the
-// product of the two last parts (below 2^-28 of |t||adapter|), the smaller ones first.
+// The operand of a delta: three parts, and the leading one's finite values.
+E4B_DEV void delta_parts8(const float (&v)[8], uint4 (&part)[4]) {
+  uint4 p3[3];
+  split_parts8<3>(v, p3);
+  part[0] = p3[0]; part[1] = p3[1]; part[2] = p3[2];
+  part[3] = finite8(p3[0]);
+}
+
+// The products of a delta: mul(a, b) for the parts of t and b (an adapter's, of dtype dt), all but that of the
+// two last (below 2^-28 of |t||adapter|), the smaller ones first.
 template <class F>
-E4B_DEV void delta_products(int dt, F&& mul) {
-  using std::integral_constant;
-  constexpr integral_constant<int, 0> p0{};
-  constexpr integral_constant<int, 1> p1{};
-  constexpr integral_constant<int, 2> p2{};
+E4B_DEV void delta_products(int dt, const uint4 (&t)[4], const uint4 (&b)[4], F&& mul) {
   if (dt == E4B_FP32) {
-    mul(p1, p2);
-    mul(p0, p2);
+    mul(t[1], b[2]);
+    mul(t[3], b[2]);
   }
   if (dt != E4B_BF16) {
-    mul(p2, p1);
-    mul(p1, p1);
-    mul(p0, p1);
+    mul(t[2], b[1]);
+    mul(t[1], b[1]);
+    mul(t[3], b[1]);
   }
-  mul(p2, p0);
-  mul(p1, p0);
-  mul(p0, p0);
+  mul(t[2], b[3]);
+  mul(t[1], b[3]);
+  mul(t[0], b[0]);
 }
 
 // lscale * (2^e * t[m, q0 + i]) (0 past the rank), i = 0..7, split: the power of two goes to t, which is as
 // small as e is large. With the rank a multiple of 8 the eight values are two 16-byte loads, else
 // eight element loads.
 template <class Args>
-E4B_DEV void lora_t_piece(const Args& p, int64_t m, int q0, int e2, uint4 (&part)[3]) {
+E4B_DEV void lora_t_piece(const Args& p, int64_t m, int q0, int e2, uint4 (&part)[4]) {
   float v[8];
   const float* t = p.lt + m * p.lr;
   if ((p.lr & 7) == 0) {
@@ -92,11 +115,11 @@ E4B_DEV void lora_t_piece(const Args& p, int64_t m, int q0, int e2, uint4 (&part
   }
 #pragma unroll
   for (int i = 0; i < 8; ++i) v[i] = q0 + i < p.lr ? __builtin_amdgcn_ldexpf(v[i], e2) * p.lscale : 0.0f;
-  split_parts8<3>(v, part);
+  delta_parts8(v, part);
 }
 
 // 2^e * B[ex, row, q0 + i] (0 past the rank), i = 0..7, from the adapter dtype, split.
-E4B_DEV void lora_b_piece(const GemmArgs& p, int ex, int64_t row, int q0, int e2, uint4 (&part)[3]) {
+E4B_DEV void lora_b_piece(const GemmArgs& p, int ex, int64_t row, int q0, int e2, uint4 (&part)[4]) {
   float v[8];
   const int64_t base = (int64_t(ex) * p.w.n + row) * p.lr;
   const int64_t q0c = q0 < p.lr ? q0 : 0;
@@ -124,20 +147,20 @@ E4B_DEV void lora_b_piece(const GemmArgs& p, int ex, int64_t row, int q0, int e2
   }
 #pragma unroll
   for (int i = 0; i < 8; ++i) v[i] = q0 + i < p.lr ? __builtin_amdgcn_ldexpf(v[i], e2) : 0.0f;
-  split_parts8<3>(v, part);
+  delta_parts8(v, part);
 }
 
 // The t operands of a workgroup's BM rows and the 16 ranks from q0, split once for all its waves, in LDS (ts:
-// 48 BM values): part i of row r, ranks 8 h .. of the step, at 16-byte piece (2 i + h) BM + r. Row r is
+// 64 BM values): operand i of row r, ranks 8 h .. of the step, at 16-byte piece (2 i + h) BM + r. Row r is
 // min(row0 + r, row_last), times 2^shift[r].
 template <int BM, int NT, class Args>
 E4B_DEV void lora_t_stage(const Args& p, uint16_t* ts, int64_t row0, int64_t row_last, const int* shift, int q0) {
   for (int j = threadIdx.x; j < 2 * BM; j += NT) {
     const int r = j % BM, h = j / BM;
-    uint4 part[3];
+    uint4 part[4];
     lora_t_piece(p, min(row0 + r, row_last), q0 + 8 * h, shift[r], part);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) reinterpret_cast<uint4*>(ts)[(2 * i + h) * BM + r] = part[i];
+    for (int i = 0; i < 4; ++i) reinterpret_cast<uint4*>(ts)[(2 * i + h) * BM + r] = part[i];
   }
 }
 
@@ -155,14 +178,14 @@ E4B_DEV void lora_delta_32x32(const GemmArgs& p, f32x16_t (&acc)[BM / 32], int e
   for (int q0 = 0; q0 < p.lr; q0 += 16) {
     if (q0) __syncthreads();  // the last step's t is read
     lora_t_stage<BM, NT>(p, ts, row0, row_last, shift, q0);
-    uint4 b[3];
+    uint4 b[4];
     lora_b_piece(p, e, brow, q0 + 8 * half, bshift, b);
     __syncthreads();
     static_for<BM / 32>([&](auto ms) {
-      uint4 t[3];
+      uint4 t[4];
 #pragma unroll
-      for (int i = 0; i < 3; ++i) t[i] = reinterpret_cast<const uint4*>(ts)[(2 * i + half) * BM + 32 * int(ms) + (lane & 31)];
-      delta_products(p.lbdt, [&](auto i, auto j) { acc[ms] = mfma_32x32x16<E4B_BF16>(b[j], t[i], acc[ms]); });
+      for (int i = 0; i < 4; ++i) t[i] = reinterpret_cast<const uint4*>(ts)[(2 * i + half) * BM + 32 * int(ms) + (lane & 31)];
+      delta_products(p.lbdt, t, b, [&](const uint4& tp, const uint4& bp) { acc[ms] = mfma_32x32x16<E4B_BF16>(bp, tp, acc[ms]); });
     });
   }
 }
@@ -175,14 +198,16 @@ E4B_DEV void lora_delta_16x16(const GemmArgs& p, f32x4_t (&acc)[MS][NS], int e, 
                               AS&& ashift, int bshift, const int64_t (&brow)[NS], int lane) {
   const int g8 = 8 * (lane >> 4);
   for (int q0 = 0; q0 < p.lr; q0 += 32) {
-    uint4 t[MS][3];
+    uint4 t[MS][4];
 #pragma unroll
     for (int ms = 0; ms < MS; ++ms) lora_t_piece(p, min(arow0 + 16 * ms, arow_last), q0 + g8, ashift(ms), t[ms]);
     static_for<NS>([&](auto ns) {
-      uint4 b[3];
+      uint4 b[4];
       lora_b_piece(p, e, brow[ns], q0 + g8, bshift, b);
       static_for<MS>([&](auto ms) {
-        delta_products(p.lbdt, [&](auto i, auto j) { acc[ms][ns] = mfma_16x16x32<E4B_BF16>(t[ms][i], b[j], acc[ms][ns]); });
+        delta_products(p.lbdt, t[ms], b, [&](const uint4& tp, const uint4& bp) {
+          acc[ms][ns] = mfma_16x16x32<E4B_BF16>(tp, bp, acc[ms][ns]);
+        });
       });
     });
   }
@@ -330,6 +355,15 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
     if (c + int(u) < nchunks) step(u, c + int(u));
   });
   sums.fold();
+  // a sum that came out NaN, once more by multiply-adds: neither the product of an infinity and a lower part
+  // that is zero nor the rounding error of an infinite total is one of its terms
+  auto again = [&](int r, int q) {
+    const int64_t row = gather_k > 0 ? rt.sorted_flat[row0 + r] / gather_k : row0 + r;
+    float v = 0.0f;
+    for (int64_t c = 0; c < in; ++c)
+      v = __builtin_fmaf(to_f<E4B_BF16>(x[row * in + c]), adapter_at(A, ADT, (int64_t(e) * rank + q) * in + c), v);
+    return v;
+  };
   // lane holds t[row 16 w + 4 g + i][rank 16 ns + l16]
 #pragma unroll
   for (int ns = 0; ns < NSM; ++ns) {
@@ -337,7 +371,10 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 16 * w + 4 * g + i;
-      if (q < rank && r < rows) t[int64_t(row0 + r) * rank + q] = sums.value(ns, i);
+      if (q < rank && r < rows) {
+        const float v = sums.value(ns, i);
+        t[int64_t(row0 + r) * rank + q] = v == v ? v : again(r, q);
+      }
     }
   }
 }

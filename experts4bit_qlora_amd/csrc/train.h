@@ -415,6 +415,12 @@ __global__ void __launch_bounds__(kWgradThreads) lora_wgrad_kernel(const float* 
     }
     __builtin_amdgcn_sched_barrier(0);
   }
+  // a sum that came out NaN, once more by multiply-adds (lora_t_mfma_kernel)
+  auto again = [&](int j, int64_t c) {
+    float v = 0.0f;
+    for (int m = beg; m < end; ++m) v = __builtin_fmaf(u[int64_t(m) * r + j], to_f<XDT>(a[row_of(m) * cols + c]), v);
+    return v;
+  };
   // lane holds ranks 16 q + 4 g + i of column 32 wid + 16 t + lane % 16
   auto put = [&](int64_t at, float v) {
     if (odt == E4B_FP32) static_cast<float*>(out)[at] = v;
@@ -428,8 +434,10 @@ __global__ void __launch_bounds__(kWgradThreads) lora_wgrad_kernel(const float* 
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int j = 16 * q + 4 * g + i;
-        if (c < cols && j < r)
-          put(TRANS ? (int64_t(e) * cols + c) * r + j : (int64_t(e) * r + j) * cols + c, scale * acc[t][q][i]);
+        if (c < cols && j < r) {
+          const float v = acc[t][q][i];
+          put(TRANS ? (int64_t(e) * cols + c) * r + j : (int64_t(e) * r + j) * cols + c, scale * (v == v ? v : again(j, c)));
+        }
       }
   }
 }

@@ -301,13 +301,22 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_u_mfma_kernel(const uint
     if (c + int(q) < nchunks) step(q, c + int(q));
   });
   sums.fold();
+  auto again = [&](int r, int q) {  // as lora_t_mfma_kernel
+    float v = 0.0f;
+    for (int64_t c = 0; c < n; ++c)
+      v = __builtin_fmaf(to_f<E4B_BF16>(g[int64_t(row0 + r) * n + c]), adapter_at(B, BDT, (int64_t(e) * n + c) * rank + q), v);
+    return v;
+  };
 #pragma unroll
   for (int ns = 0; ns < NSM; ++ns) {
     const int q = 16 * ns + l16;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 16 * w + 4 * gr + i;
-      if (q < rank && r < rows) u[int64_t(row0 + r) * rank + q] = sums.value(ns, i);
+      if (q < rank && r < rows) {
+        const float v = sums.value(ns, i);
+        u[int64_t(row0 + r) * rank + q] = v == v ? v : again(r, q);
+      }
     }
   }
 }

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import experts4bit_qlora_amd as e4b
-from experts4bit_qlora_amd import train
+from experts4bit_qlora_amd import ops, train
 from oracle_weights import oracle_weights
 
 pytestmark = pytest.mark.gpu
@@ -113,3 +113,63 @@ def test_inference_with_all_zero_expert_weights(T, E, hid, inter, dq):
     want = _layer_fp64(mod, x, idx, w)["out"]
     assert out.isfinite().all()
     assert _rel(out, want) < 1e-2, _rel(out, want)
+
+
+def _same_specials(got, want, tol):
+    """Infinities of one sign and NaNs where ``want`` has them, the rest within ``tol`` in norm."""
+    got = got.double()
+    inf, fin = want.isinf(), want.isfinite()
+    assert bool((got.isnan() == want.isnan()).all()) and bool((got.isinf() == inf).all())
+    assert bool((got[inf] == want[inf]).all())
+    assert _rel(got[fin], want[fin]) < tol
+
+
+@pytest.mark.parametrize("T,E,hid,inter", SHAPES)
+@pytest.mark.parametrize("adt", (torch.float32, torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("r", (3, 16))
+def test_an_infinity_stays_one(T, E, hid, inter, adt, r):
+    """Weights, adapters and tokens all positive, so one infinite activation or gradient makes sums of one sign
+    infinite and leaves the others alone. The adapters fit one bf16 part: what is split off is zero.
+    The largest finite gradient is dL/dA1 = scaling u1 x over 600 rows: u1 = 512 . 22 . 0.06 = 676 for
+    gradients of 0.06, 4.9e5 in all, beyond fp16; with gradients of 0.06 . 2^-6 it is 7.6e3."""
+    _announce(f"infinities T={T} E={E} hid={hid} inter={inter} {adt} r={r}")
+    mod = _module(E, hid, inter, r, False, gate_up=torch.full((E, 2 * inter, hid), 0.01),
+                  down=torch.full((E, hid, inter), 0.01)).train()
+    for n in ADAPTERS:
+        p = getattr(mod, n)
+        setattr(mod, n, torch.nn.Parameter((torch.rand_like(p) * 0.1 + 0.01).to(torch.bfloat16).to(adt)))
+    assert e4b.enable_fast_train(mod) == 1
+    torch.manual_seed(33)
+    x = (torch.rand(T, hid, device=DEV) + 0.1).to(torch.bfloat16)
+    idx = torch.rand(T, E, device=DEV).argsort(1)[:, :2].contiguous()
+    idx[3, 0], idx[3, 1], idx[9, 0], idx[9, 1] = 0, 1, 0, 1
+    w = torch.rand(T, 2, device=DEV).to(torch.bfloat16) + 0.1
+    grad = ((torch.rand(T, hid, device=DEV) * 0.1 + 0.01) * 2.0 ** -6).to(torch.bfloat16)
+    x[3, 5] = float("inf")
+    with torch.no_grad():
+        out = mod(x, idx, w)
+    want = _layer_fp64(mod, x, idx, w)["out"]
+    assert want[3].isinf().all() and want[4].isfinite().all()
+    _same_specials(out, want, 1e-2)
+    x[3, 5] = 1.0
+    grad[9, 7] = float("inf")
+    x, w = x.requires_grad_(), w.requires_grad_()
+    out = mod(x, idx, w)
+    out.backward(grad)
+    want = _layer_fp64(mod, x, idx, w, grad)
+    assert want["x"][9].isinf().all() and want["gate_up_lora_A"][0].isinf().all()
+    for n, got in (("x", x.grad), ("w", w.grad), *((n, getattr(mod, n).grad) for n in ADAPTERS)):
+        _same_specials(got, want[n], 1e-2)
+
+
+@pytest.mark.parametrize("adt", (torch.bfloat16, torch.float16))
+def test_weight_gradients_keep_infinities(adt):
+    """u and rows of exact leading parts, one infinity in each: sums of one sign."""
+    rb = ops._routing_from_sizes([70, 5], [0, 1], 2, DEV)[0]
+    u = torch.full((75, 8), 0.5, device=DEV)
+    a = torch.full((75, 136), 0.25, device=DEV).to(adt)
+    u[3, 2], a[71, 9] = float("inf"), float("inf")
+    got = ops.lora_wgrad(u, a, rb, 75, 2, 1.0)
+    want = torch.stack([u[:70].T @ a[:70].float(), u[70:].T @ a[70:].float()])
+    assert want[0, 2].isinf().all() and want[1, :, 9].isinf().all()
+    assert torch.equal(got, want)
