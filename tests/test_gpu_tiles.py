@@ -63,3 +63,22 @@ def test_fp16_32_row_tiles_use_the_exact_weights(n, dq, epi):
         want = torch.nn.functional.silu(gate) * up
         bound = 1.1 * bg * up.abs() + bu * gate.abs() + bg * bu + 2.0 ** -20 * want.abs()  # |silu'| <= 1.1
     assert torch.all((got - want).abs() <= bound + 2.0 ** -11 * want.abs() + 2.0 ** -24)
+
+
+@pytest.mark.parametrize("dq", (False, True))
+def test_fp16_32_row_tiles_hold_the_dequantized_weights_bit_for_bit(dq):
+    """One activation of 1 per row: every output is one weight, rounded to fp32 and then to fp16 as e4b_dequant rounds
+    it (of the 417,792 products, about 25 lie where a single rounding gives another fp16 value)."""
+    g = torch.Generator().manual_seed(9)
+    E, n, K = 3, 272, 512
+    packed, absmax = Q.quantize_4bit((torch.randn(E, n * K, generator=g) * 0.05).to(DEV))
+    code = Q.code_4bit("nf4", DEV)
+    if dq:
+        q, a2, off = Q.double_quant(absmax)
+        qw = ops.nf4_dq_qweight(packed, q, a2, off, code, Q.dynamic_map().to(DEV), n, K, num_experts=E)
+    else:
+        qw = ops.nf4_qweight(packed, absmax, code, n, K, num_experts=E)
+    a = torch.eye(K, dtype=torch.float16, device=DEV).repeat(E, 1)
+    got = ops.grouped_gemm(a, qw, _routing([K] * E, 32), E * K, E * K, gather_k=1, path=N.PATH_MFMA)
+    want = ops.dequant(qw, dtype=torch.float16).view(E, n, K).transpose(1, 2).reshape(E * K, n)
+    assert torch.equal(got, want), int((got != want).sum())
