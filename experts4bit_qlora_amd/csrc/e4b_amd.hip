@@ -1850,8 +1850,20 @@ int e4b_train_backward(const void* grad_out, int32_t grad_dtype, const void* hid
   int rc = check_train(tokens, top_k, w1, w2, lora, epilogue, weight_dtype);
   if (rc) return rc;
   if (!any_dtype_ok(grad_dtype)) return fail(E4B_EINVAL, "bad gradient dtype");
-  if (tokens == 0) return E4B_OK;
   const TrainShape sh = train_shape(tokens, top_k, w1->num_experts, w1->n, w2->n, epilogue, lora->rank);
+  if (tokens == 0) {
+    const int64_t er = int64_t(sh.E) * sh.r * (lora->dtype == E4B_FP32 ? 2 : 1);
+    const std::pair<void*, int64_t> grads[] = {{grad_a1, sh.H}, {grad_b1, sh.n1}, {grad_a2, sh.I}, {grad_b2, sh.H}};
+    for (const auto& [p, cols] : grads) {
+      if (!p) continue;
+      const int64_t n = er * cols, blocks = std::min<int64_t>(cdiv(n, e4b::kRowThreads), 4096);
+      hipLaunchKernelGGL(e4b::zero_halves_kernel, dim3(static_cast<unsigned>(blocks)), dim3(e4b::kRowThreads), 0, stream,
+                         static_cast<uint16_t*>(p), n);
+      rc = check_launch("zero_halves_kernel");
+      if (rc) return rc;
+    }
+    return E4B_OK;
+  }
   if (!grad_out || !hidden || !top_k_weights || !saved || !workspace) return fail(E4B_EINVAL, "NULL pointer");
   if (!aligned16(grad_out) || !aligned16(hidden) || !aligned16(saved) || !aligned16(workspace))
     return fail(E4B_EINVAL, "grad_out, hidden, saved and workspace must be 16-byte aligned");

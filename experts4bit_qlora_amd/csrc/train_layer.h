@@ -196,6 +196,11 @@ __global__ void __launch_bounds__(kRowThreads) combine_bwd_kernel(const void* __
   put(dot);
 }
 
+// The adapter gradients of a call without tokens.
+__global__ void __launch_bounds__(kRowThreads) zero_halves_kernel(uint16_t* __restrict__ p, int64_t n) {
+  for (int64_t i = int64_t(blockIdx.x) * kRowThreads + threadIdx.x; i < n; i += int64_t(gridDim.x) * kRowThreads) p[i] = 0;
+}
+
 // u[m, q] = sum_c g_m[c] * B[e, c, q] for the sorted rows of every routing tile: lora_t_mfma_kernel with
 // the adapter matrix in the other orientation (its ranks contiguous), so a 64-deep chunk is staged in
 // LDS as it lies in memory ([64 c][ranks], one array per bf16 part) and its operands come from

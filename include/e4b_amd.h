@@ -385,7 +385,8 @@ int e4b_set_probe(int32_t site, hipEvent_t before, hipEvent_t after);
  * inner products. The backward takes dL/dout [tokens, H] in grad_dtype and writes what is asked for (a
  * NULL output is skipped): grad_hidden bf16 [tokens, H], grad_weights in weight_dtype [tokens, top_k],
  * and the adapters' gradients in their dtype and layout. Ids outside [0, E) contribute nothing and
- * get zero gradients. Nothing synchronises; both directions are deterministic. */
+ * get zero gradients, and so do the adapters of experts without rows (all of them without tokens, when
+ * only the adapters' gradients are touched). Nothing synchronises; both directions are deterministic. */
 size_t e4b_train_saved_bytes(int64_t tokens, int32_t top_k, int32_t num_experts, int64_t n1, int64_t n2,
                              int32_t epilogue, int32_t rank);
 size_t e4b_train_workspace_bytes(int64_t tokens, int32_t top_k, int32_t num_experts, int64_t n1, int64_t n2,

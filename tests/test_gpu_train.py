@@ -380,3 +380,24 @@ def test_fused_layer_gives_only_the_gradients_asked_for():
     for n in full:
         only = grads((n,))
         assert torch.equal(only[n], full[n]) and all(only[m] is None for m in only if m != n), n
+
+
+@pytest.mark.parametrize("adt", (torch.float32, torch.bfloat16))
+def test_a_backward_without_tokens_writes_zero_adapter_gradients(adt):
+    """The adapters' gradients have their size whatever the tokens: written, not left as they were allocated."""
+    _announce(f"no tokens {adt}")
+    E_, hid, inter, r = 3, 128, 64, 5
+    w1, w2 = F._for_tokens(F._qweights(_build(E_=E_, hid=hid, inter=inter, r=r).base), 64)
+    lora = [torch.ones(E_, *s, dtype=adt, device=DEV) for s in ((r, hid), (2 * inter, r), (r, inter), (hid, r))]
+    x, idx = torch.zeros(0, hid, dtype=torch.bfloat16, device=DEV), torch.zeros(0, 2, dtype=torch.int64, device=DEV)
+    w = torch.zeros(0, 2, device=DEV)
+    out, saved = ops.train_forward(x, idx, w, w1, w2, lora, 1.0, N.EPI_SWIGLU, 0.0, torch.bfloat16)
+    assert out.shape == (0, hid)
+    stale = [torch.full_like(t, float("nan")) for t in lora]
+    del stale  # the allocator hands these blocks out again
+    grads = ops.train_backward(out, x, w, w1, w2, lora, 1.0, N.EPI_SWIGLU, 0.0, saved, (True,) * 6)
+    assert grads[0].shape == x.shape and grads[1].shape == w.shape
+    for g, t in zip(grads[2:], lora):
+        assert g.shape == t.shape and g.dtype == adt and not g.any()
+    only = ops.train_backward(out, x, w, w1, w2, lora, 1.0, N.EPI_SWIGLU, 0.0, saved, (False,) * 3 + (True,) + (False,) * 2)
+    assert [t is None for t in only] == [True, True, True, False, True, True]
