@@ -161,10 +161,7 @@ def _for_tokens(descs, tokens):
     weight version); below it as they are, so decode calls never launch the exponent kernels."""
     if tokens <= _SHIFT_FREE_TOKENS:
         return descs
-    for qw in descs:
-        if qw.shift is None:
-            ops.with_weight_shift(qw)
-    return descs
+    return tuple([ops.shifted_on_stream(qw) for qw in descs])
 
 
 def _mxfp4_qweights(mod, cd):

@@ -8,6 +8,8 @@ here synchronises the device, and none computes anything itself: a missing libra
 from __future__ import annotations
 
 import ctypes
+import dataclasses
+import threading
 from dataclasses import dataclass
 
 import torch
@@ -26,6 +28,9 @@ def dtype_code(dt: torch.dtype) -> int:
 
 def _ptr(t) -> int | None:
     return None if t is None else t.data_ptr()
+
+
+_SHIFT_LOCK = threading.Lock()
 
 
 def _stream(device: torch.device) -> int:
@@ -106,6 +111,30 @@ def with_weight_shift(qw: QW) -> QW:
     N.check("e4b_weight_shift", N.lib().e4b_weight_shift(ctypes.byref(s), shift.data_ptr(), _stream(shift.device)))
     qw.shift = shift
     return qw
+
+
+def shifted_on_stream(qw: QW) -> QW:
+    """``qw`` with exponents that the current stream computed (once per stream; torch hands out a bounded
+    pool of them), so a call never reads another stream's before they are written or after they are
+    freed. Under capture the first stream's stand (a capture starts from a synchronised device);
+    without any the capture computes its own, which exist only in its replays and are not kept."""
+    if qw.fmt == N.FMT_MXFP4 or not qw.packed.is_cuda:
+        return qw
+    raw = _stream(qw.packed.device)
+    if qw.shift is not None and qw.__dict__.get("_shift_stream", raw) == raw:
+        return qw
+    if torch.cuda.is_current_stream_capturing():
+        return qw if qw.shift is not None else with_weight_shift(dataclasses.replace(qw))
+    with _SHIFT_LOCK:
+        if qw.shift is None:
+            qw.__dict__["_shift_stream"] = raw
+            return with_weight_shift(qw)
+        if qw.__dict__["_shift_stream"] == raw:
+            return qw
+        copies = qw.__dict__.setdefault("_shifted", {})
+        if raw not in copies:
+            copies[raw] = with_weight_shift(dataclasses.replace(qw, shift=None))
+        return copies[raw]
 
 
 def nf4_qweight(packed, absmax, code, n, k, num_experts=None, bias=None) -> QW:

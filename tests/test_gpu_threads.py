@@ -175,3 +175,70 @@ def test_probe_events_time_each_prefill_launch_without_changing_results():
     assert before.elapsed_time(after) == last
     with pytest.raises(N.NativeError):
         N.check("e4b_set_probe", L.e4b_set_probe(7, None, None))
+
+
+def _spoil(stream, n, value):
+    """Leave ``value`` in the block that the next allocation of ``n`` int32 on ``stream`` takes."""
+    with torch.cuda.stream(stream):
+        t = torch.full((n,), value, dtype=torch.int32, device=DEV)
+    torch.cuda.synchronize()
+    del t
+
+
+def _training(mod):
+    lora = e4b.ExpertsLoRA(mod, r=8, alpha=16, dtype=torch.float32).to(DEV).train()
+    g = torch.Generator(device=DEV).manual_seed(3)
+    with torch.no_grad():
+        for p in (lora.gate_up_lora_A, lora.gate_up_lora_B, lora.down_lora_A, lora.down_lora_B):
+            p.copy_(torch.randn(p.shape, generator=g, device=DEV) * 0.05)
+    assert e4b.enable_fast_train(lora) == 1
+    return lora
+
+
+@pytest.mark.parametrize("train", (False, True))
+def test_a_second_stream_waits_for_the_first_ones_weight_exponents(train):
+    """The first call computes the expert exponents behind 20 ms of other work on its stream; a call on another
+    stream, issued at once, must not read them earlier."""
+    E, H, inter, k = 16, 512, 256, 4
+    _announce(f"weight exponents across streams train={train}")
+    inp = _inputs(96, E, H, k, seed=31)
+
+    def call(m):
+        return m(*inp) if train else torch.no_grad()(m)(*inp)
+
+    make = (lambda: _training(_module(E, H, inter))) if train else (lambda: _module(E, H, inter))
+    want = call(make()).detach()
+    mod = make()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    _spoil(first, E, 60)
+    with torch.cuda.stream(first):
+        torch.cuda._sleep(40_000_000)
+        a = call(mod).detach()
+    with torch.cuda.stream(second):
+        b = call(mod).detach()
+        c = call(mod).detach()
+    torch.cuda.synchronize()
+    assert torch.equal(a, want) and torch.equal(b, want) and torch.equal(c, want)
+
+
+def test_a_first_call_under_capture_leaves_eager_calls_their_own_exponents():
+    """Captured before any eager call: the exponents the capture recorded exist only in its replays."""
+    E, H, inter, k = 16, 512, 256, 4
+    _announce("first call under capture")
+    inp = _inputs(96, E, H, k, seed=32)
+    with torch.no_grad():
+        want = _module(E, H, inter)(*inp)
+        mod = _module(E, H, inter)
+        mod(inp[0][:2], inp[1][:2], inp[2][:2])  # descriptors and pools; 2 tokens need no exponents
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = mod(*inp)
+        eager = mod(*inp)
+        torch.cuda.synchronize()
+        assert torch.equal(eager, want)
+        for _ in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+            assert torch.equal(mod(*inp), want)
