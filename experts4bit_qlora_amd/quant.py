@@ -145,11 +145,13 @@ def _dynamic_table_on(device):
 
 
 def _plain_on_device(w: torch.Tensor) -> bool:
-    """A device tensor that no transform or graph follows (a tensor subclass, or one that autograd
-    records, takes the torch formulation, which is the kernels' definition)."""
+    """A device tensor that no transform or graph follows (a tensor subclass, one that autograd records or
+    that carries a forward-mode tangent, and any under ``torch.jit.trace`` take the torch formulation,
+    which is the kernels' definition)."""
     return (w.is_cuda and type(w) in (torch.Tensor, torch.nn.Parameter) and w.is_floating_point()
             and not (w.requires_grad and torch.is_grad_enabled())
-            and not torch._C._functorch.is_functorch_wrapped_tensor(w))
+            and not torch._C._functorch.is_functorch_wrapped_tensor(w) and not torch.jit.is_tracing()
+            and torch.autograd.forward_ad.unpack_dual(w).tangent is None)
 
 
 def _on_kernel(w: torch.Tensor, blocksize: int) -> bool:

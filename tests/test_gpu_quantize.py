@@ -69,3 +69,20 @@ def test_double_quant_is_the_torch_formulation(shape):
     for c in cases:
         got, want = Q.double_quant(c), Q.double_quant(c, code2=Q.dynamic_map().to(DEV))
         assert all(torch.equal(p.nan_to_num(-1.0), q.nan_to_num(-1.0)) and p.dtype == q.dtype for p, q in zip(got, want))
+
+
+def test_tangents_and_traces_follow_the_torch_formulation():
+    """Forward-mode tangents of the scales, and a traced function on another input."""
+    g = torch.Generator().manual_seed(4)
+    w, t, other = (torch.randn(8, 256, generator=g).to(DEV) for _ in range(3))
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(w, t)
+        unpack = torch.autograd.forward_ad.unpack_dual
+        got, want = Q.quantize_4bit(dual)[1], Q._quantize_4bit_torch(dual, "nf4", 64)[1]
+        assert torch.equal(unpack(got).tangent, unpack(want).tangent)
+        got, want = Q.double_quant(dual), Q.double_quant(dual, code2=Q.dynamic_map().to(DEV))
+        assert torch.equal(unpack(got[1]).tangent, unpack(want[1]).tangent)
+    traced = torch.jit.trace(lambda v: Q.quantize_4bit(v), (w,), check_trace=False)
+    assert all(torch.equal(a, b) for a, b in zip(traced(other), Q.quantize_4bit(other)))
+    traced = torch.jit.trace(lambda v: Q.double_quant(v), (w.abs(),), check_trace=False)
+    assert all(torch.equal(a, b) for a, b in zip(traced(other.abs()), Q.double_quant(other.abs())))
