@@ -401,3 +401,76 @@ def test_a_backward_without_tokens_writes_zero_adapter_gradients(adt):
         assert g.shape == t.shape and g.dtype == adt and not g.any()
     only = ops.train_backward(out, x, w, w1, w2, lora, 1.0, N.EPI_SWIGLU, 0.0, saved, (False,) * 3 + (True,) + (False,) * 2)
     assert [t is None for t in only] == [True, True, True, False, True, True]
+
+
+@pytest.mark.parametrize("T,E_,top,hid,inter,cdt,kind", [
+    (60, 8, 2, 256, 512, torch.float16, "swiglu"),     # fp16 over 32-row tiles, K a multiple of 256: exact weights in registers
+    (60, 8, 2, 192, 320, torch.float16, "swiglu"),     # ... and off it
+    (900, 4, 2, 256, 128, torch.float16, "swiglu"),    # 128-row tiles
+    (300, 4, 2, 192, 128, torch.bfloat16, "gelu"),     # an activation that only the base's Python code knows
+    (300, 4, 2, 192, 128, torch.bfloat16, "ranks"),    # two ranks
+    (40, 4, 2, 256, 128, torch.bfloat16, "dtypes"),    # adapters of two dtypes
+])
+def test_per_projection_functions_match_fp64(T, E_, top, hid, inter, cdt, kind):
+    """Layers that the two-call form does not take, projection by projection: outputs and every gradient against
+    fp64 autograd, dropped ids among them. 1e-2 in norm for bf16, as above; fp16 keeps three more bits (an
+    eighth), twice that."""
+    _announce(f"per projection T={T} E={E_} hid={hid} inter={inter} {cdt} {kind}")
+    torch.manual_seed(23)
+    act = torch.nn.functional.gelu if kind == "gelu" else None
+    base = e4b.Experts4bit.from_float((torch.randn(E_, 2 * inter, hid) * 0.1).to(DEV), (torch.randn(E_, hid, inter) * 0.1).to(DEV),
+                                      compute_dtype=cdt, **({"activation": act} if act else {}))
+    mod = e4b.ExpertsLoRA(base, r=16, alpha=32, dtype=torch.float32).to(DEV).train()
+    with torch.no_grad():
+        for p in (mod.gate_up_lora_B, mod.down_lora_B):
+            p.normal_(0, 0.05)
+    if kind == "ranks":
+        mod.down_lora_A = torch.nn.Parameter(torch.randn(E_, 5, inter, device=DEV) / 5)
+        mod.down_lora_B = torch.nn.Parameter(torch.randn(E_, hid, 5, device=DEV) * 0.05)
+    if kind == "dtypes":
+        for n in ("down_lora_A", "down_lora_B"):
+            setattr(mod, n, torch.nn.Parameter(getattr(mod, n).detach().to(torch.bfloat16)))
+    assert e4b.enable_fast_train(mod) == 1
+    x = torch.randn(T, hid, device=DEV).to(cdt).requires_grad_()
+    idx = torch.rand(T, E_, device=DEV).argsort(1)[:, :top].contiguous()
+    idx[1, 0], idx[2, top - 1] = -1, E_
+    w = torch.rand(T, top, device=DEV).to(cdt).requires_grad_()
+    grad = torch.randn(T, hid, device=DEV).to(cdt)
+    assert train._layer_inputs(mod, x.detach(), idx, w) is None
+    out = mod(x, idx, w)
+    out.backward(grad)
+
+    def gated(proj):
+        g, u = proj.chunk(2, -1)
+        return act(g) * u
+
+    want = _layer_fp64(base, mod, x.detach(), idx, w.detach(), grad, gated if act else _swiglu64())
+    got = {"out": out.detach(), "x": x.grad, "w": w.grad, **{n: p.grad for n, p in mod.named_parameters() if "lora" in n}}
+    tol = GRAD_TOL if cdt == torch.bfloat16 else GRAD_TOL / 4
+    for n in want:
+        assert got[n].dtype == (out.dtype if n in ("out", "x", "w") else getattr(mod, n).dtype)
+        assert _rel(got[n], want[n]) < tol, (n, _rel(got[n], want[n]))
+    assert w.grad[1, 0] == 0 and w.grad[2, top - 1] == 0
+
+
+@pytest.mark.parametrize("T,E_", [(600, 4), (60, 8)])
+def test_wide_gradient_rows_are_no_further_from_fp64(T, E_, monkeypatch):
+    """Gradient rows whose values span 2^-30 .. 1: the fp16 mode's scaled rows (values below 2^-31 of a row's
+    largest lose bits) against the per-projection functions' bf16 rows and weights."""
+    _announce(f"wide gradient rows T={T} E={E_}")
+    args = _inputs(T, seed=13, E_=E_)
+    g_ = torch.Generator(device=DEV).manual_seed(14)
+    scale = torch.exp2(-30 * torch.rand(args[0].shape, generator=g_, device=DEV))
+    err = {}
+    for lane in ("layer", "projections"):
+        mod = _build(seed=12, E_=E_)
+        assert e4b.enable_fast_train(mod) == 1
+        if lane == "projections":
+            monkeypatch.setattr(train, "_layer_inputs", lambda *a: None)
+        hs, grad = args[0].clone().requires_grad_(), (args[3] * scale).to(torch.bfloat16)
+        mod(hs, *args[1:3]).backward(grad)
+        want = _layer_fp64(mod.base, mod, args[0], args[1], args[2], grad, _swiglu64())
+        err[lane] = {"x": _rel(hs.grad, want["x"]), **{n: _rel(p.grad, want[n]) for n, p in mod.named_parameters() if "lora" in n}}
+    print(err, flush=True)
+    for n in err["layer"]:
+        assert err["layer"][n] <= err["projections"][n], n
