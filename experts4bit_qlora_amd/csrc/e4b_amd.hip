@@ -1243,8 +1243,7 @@ bool lora_fused_ok(int32_t act_dtype, const e4b_qweight* w1, const e4b_qweight* 
 }
 
 // t = x . A^T for the sorted rows of rt's tiles on the matrix cores (bf16 x, in a multiple of 64, as
-// every k is): 64-row parts of 128-row tiles, whole
-// 32-row tiles, the ranks in 16-rank blocks.
+// every k is): 64-row parts of 128-row tiles, whole 32-row tiles, the ranks in 16-rank blocks.
 int lora_t_mfma(const void* x, int32_t gather_k, const e4b_routing& rt, const void* A, int32_t adt, int rank,
                 int64_t in, float* t, hipStream_t stream) {
   if (in <= 0 || in % e4b::kLoraTK != 0)
@@ -1447,10 +1446,11 @@ int e4b_moe_lora_forward(const void* hidden, int32_t act_dtype, int64_t tokens, 
     return check_launch("decode_down_kernel (LoRA)");
   }
 
-  // Grouped path in the fp16 matrix-core mode with each delta inside its GEMM's epilogue (bf16
-  // activations, NF4 weights carrying shifts): t1 = x . A1^T; gate_up GEMM + lscale t1 . B1^T + epilogue -> h; t2 = h . A2^T; h as
-  // scaled fp16 rows; down GEMM + lscale t2 . B2^T -> fp32 rows; combine. No fp32 gate_up rows
-  // and no pass over the down rows: the deltas ride the GEMM tiles' accumulators.
+  // Grouped path in the fp16 matrix-core mode with each delta inside its GEMM's tiles (bf16
+  // activations, NF4 weights carrying shifts): t1 = x . A1^T; gate_up GEMM + lscale t1 . B1^T +
+  // epilogue -> h; t2 = h . A2^T; h as scaled fp16 rows; down GEMM + lscale t2 . B2^T -> fp32 rows;
+  // combine. No fp32 gate_up rows and no pass over the down rows: the deltas ride the GEMM tiles'
+  // accumulators.
   const bool gemv_path = flags == E4B_PATH_GEMV || (flags == E4B_PATH_AUTO && tokens <= 4);
   if (!gemv_path && lora_fused_ok(act_dtype, w1, w2)) {
     e4b_routing rt, rbig, rsmall;

@@ -22,7 +22,7 @@ namespace {
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // 256-row tiles run a wide kernel (fp16 mode, or MXFP4 with bf16 activations: eight waves of
-// 128 x 64; otherwise four of 128 x 128), the others gemm_mfma_kernel.
+// 256 x 32; otherwise four of 128 x 128), the others gemm_mfma_kernel.
 template <int DT, int FMT, int BM, bool F16C>
 void launch_mfma_kernel(const GemmArgs& a, dim3 grid, hipStream_t s) {
   if constexpr (BM == kTileMBig && F16C) {
@@ -33,7 +33,7 @@ void launch_mfma_kernel(const GemmArgs& a, dim3 grid, hipStream_t s) {
   } else if constexpr (BM == kTileMBig && DT == E4B_BF16 && FMT == E4B_FMT_MXFP4) {
     hipLaunchKernelGGL((gemm_wide8_kernel<DT, FMT, F16C>), grid, dim3(kWide8Threads), 0, s, a);
   } else if constexpr (BM == kTileMBig) {
-    hipLaunchKernelGGL((gemm_wide_kernel<DT, FMT, F16C>), grid, dim3(kWideThreads), 0, s, a);
+    hipLaunchKernelGGL((gemm_wide_kernel<DT, FMT>), grid, dim3(kWideThreads), 0, s, a);
   } else {
     hipLaunchKernelGGL((gemm_mfma_kernel<DT, FMT, BM, F16C>), grid, dim3(gemm_threads(BM)), 0, s, a);
   }

@@ -1,5 +1,6 @@
 // Prefill grouped GEMM, wide tiles: 256 sorted rows x 256 weight rows per workgroup, four waves
-// (one per SIMD) of 128 x 128 each, on v_mfma_f32_32x32x16_{bf16,f16}.
+// (one per SIMD) of 128 x 128 each, on v_mfma_f32_32x32x16_{bf16,f16}: fp16 activations, and bf16
+// ones with NF4 weights outside the fp16 matrix-core mode (gemm_wide8.h has that mode and MXFP4 weights).
 //
 // The 128 x 256 tile of gemm_mfma_kernel gives each of its eight waves a 64 x 64 block: per
 // 64-deep step a CU then moves 48 KB of staged operands and 128 KB of MFMA fragments through
@@ -18,8 +19,8 @@
 // the buffer step s has just released, through sub-steps 0-2 of step s + 1; the activation
 // loads take 128 contiguous bytes per eight lanes (a load with one 16-byte row piece per lane
 // costs the load pipeline about twice the issue time). The decode is that of gemm_mfma_kernel
-// (dequant_bytes' byte-plane lookups, the fp16 matrix-core mode's row and expert shifts), so the
-// two kernels form the same per-element products; only the fp32 summation order differs.
+// (dequant_bytes' byte-plane lookups), so the two kernels form the same per-element products; only
+// the fp32 summation order differs.
 //
 // The output layout of a 32 x 32 MFMA: lane l holds column l % 32 of rows
 // 8 * (i / 4) + 4 * (l / 32) + i % 4, i = 0..15, of its tile.
@@ -43,12 +44,9 @@ E4B_DEV int lds_at_w(int row, int col) { return row * kTileK + ((((col >> 3) ^ r
 
 // One tile. HALF: a tile of at most 128 rows (an expert's last, partial tile) as 128 rows x 256
 // weight rows, each wave 128 x 64 (two 32 x 32 MFMA columns), instead of padding it to 256 rows.
-template <int DT, int FMT, bool F16C, bool HALF>
+template <int DT, int FMT, bool HALF>
 E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2][kWideTileM * kTileK],
-                       uint16_t (&Ws)[2][kWideTileN * kTileK], float* code2_s, int* row_shift_s,
-                       const uint32_t* ptab) {
-  constexpr bool PTAB = F16C;  // fp16 mode: weights decoded through the LDS table of code pairs
-  constexpr int CT = F16C ? E4B_FP16 : DT;
+                       uint16_t (&Ws)[2][kWideTileN * kTileK], float* code2_s) {
   constexpr int BM = kWideTileM, BN = kWideTileN;
   constexpr int MS = 4, NS = HALF ? 2 : 4;  // 32 x 32 MFMA tiles per wave: 128 x 32 NS
   constexpr int WCOL = 32 * NS;             // weight rows per wave
@@ -78,16 +76,16 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
   // 32 i + t / 8, columns 8 (t % 8) .. + 7, so eight lanes read one row's 128 contiguous bytes
   // (one lane per row, 16 bytes from each of 64 rows per load, costs the load pipeline about
   // twice the issue time). aoff[i]: that piece of step 0, in 16-byte units of p.a.
-  // The rows' sources (and tile row t's, for the row shifts) are loaded together at clamped
+  // The rows' sources are loaded together at clamped
   // indices, before row_end is known, and dropped for rows past the expert's end: a load behind
   // the row test, divided inside that branch, was waited on alone, one round trip per piece.
   const int apart = tid & 7;
   const bool gather = p.gather_k > 0;
   const int mlast = static_cast<int>(p.M) - 1;
-  int sf[AP + 1];
+  int sf[AP];
 #pragma unroll
-  for (int i = 0; i <= AP; ++i) {
-    const int r = min(row0 + (i < AP ? 32 * i + (tid >> 3) : tid), mlast);
+  for (int i = 0; i < AP; ++i) {
+    const int r = min(row0 + 32 * i + (tid >> 3), mlast);
     const int v = p.rt.sorted_flat[r];
     sf[i] = gather ? v : r;
   }
@@ -96,12 +94,6 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
 #pragma unroll
   for (int i = 0; i < AP; ++i)
     aoff[i] = static_cast<uint32_t>((row_src(row0 + 32 * i + (tid >> 3), sf[i]) * k) / 8 + apart);
-  int wsh = 0;
-  if constexpr (F16C) {
-    wsh = p.w.shift[e];
-    // row_shift_s: the shift of tile row tid, for the epilogue
-    row_shift_s[tid] = exp_shift(p.a_exp[row_src(row0 + tid, sf[AP])]);
-  }
   // W: thread tid stages LDS weight row tid (for a gated epilogue rows 0..127 are the gate rows
   // of the tile's 128 output columns and rows 128..255 their up rows); rows past n_out read
   // weight row 0 and feed only columns that are never stored
@@ -158,53 +150,34 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
       const float prod = code2_s[sq[set]] * sa[set];
       scale = prod + offset;
     }
-    if constexpr (F16C) scale = __builtin_amdgcn_ldexpf(scale, wsh);
     return scale;
   };
   // Staging of one step, in pieces the main loop spreads over the MFMAs: the activation row
-  // (eight 16-byte stores; converted to scaled fp16 in fp16 mode 1) and the weight row, one
-  // packed word (eight values, one 16-byte store) at a time.
+  // (eight 16-byte stores) and the weight row, one packed word (eight values, one 16-byte store) at a
+  // time.
   auto store_a = [&](int buf, int i) {
     if (i >= AP) return;  // (i is a constant at every call)
     *reinterpret_cast<u32x4_t*>(&As[buf][lds_at_w(32 * i + (tid >> 3), 8 * apart)]) = areg[i];
   };
-  // A weight word in two halves, so the table lookups of the fp16 mode can be issued a chunk
-  // before the multiplies that wait for them: fetch_w leaves in r the looked-up code pairs
-  // (fp16 mode) or the decoded values, put_w applies the scale pair t.lo[0] (fp16 mode) and
-  // stores the word's eight values.
+  // A weight word in two halves: fetch_w leaves its decoded values in r, put_w stores them.
   auto fetch_w = [&](int set, int wi, const NibPlanes& t, uint32_t (&r)[4]) {
     if constexpr (FMT == E4B_FMT_MXFP4) {  // words 0-3: the first 32-value block, 4-7: the second
-      fp4_word<CT>(wq[set][wi], e8m0_to_f32(wi < 4 ? (sq[set] & 0xffu) : (sq[set] >> 8)), r);
-    } else if constexpr (PTAB) {  // byte b's code pair from the lane's table copy
-      const uint32_t* tab = ptab + (lane & (kPairCopies - 1));
-      const uint32_t w = wq[set][wi];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) r[b] = tab[((w >> (8 * b)) & 0xffu) * kPairCopies];
+      fp4_word<DT>(wq[set][wi], e8m0_to_f32(wi < 4 ? (sq[set] & 0xffu) : (sq[set] >> 8)), r);
     } else {
       nib_word<FMT>(t, wq[set][wi], r);
     }
   };
-  auto put_w = [&](int buf, int wi, const NibPlanes& t, const uint32_t (&r)[4]) {
-    uint32_t o[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) o[b] = PTAB ? pk_mul_f16(r[b], t.lo[0]) : r[b];
-    *reinterpret_cast<uint4*>(&Ws[buf][lds_at_w(tid, 8 * wi)]) = make_uint4(o[0], o[1], o[2], o[3]);
+  auto put_w = [&](int buf, int wi, const uint32_t (&r)[4]) {
+    *reinterpret_cast<uint4*>(&Ws[buf][lds_at_w(tid, 8 * wi)]) = make_uint4(r[0], r[1], r[2], r[3]);
   };
   auto store_w = [&](int set, int buf, int wi, const NibPlanes& t) {
     uint32_t r[4];
     fetch_w(set, wi, t, r);
-    put_w(buf, wi, t, r);
+    put_w(buf, wi, r);
   };
   auto planes = [&](float scale) {
-    if constexpr (FMT == E4B_FMT_MXFP4) {
-      return NibPlanes{};
-    } else if constexpr (PTAB) {  // the table decode needs only the scale, as an fp16 pair
-      NibPlanes t{};
-      t.lo[0] = cvt_pair<E4B_FP16>(scale, scale);
-      return t;
-    } else {
-      return nib_planes<CT, !F16C>(code, scale);
-    }
+    if constexpr (FMT == E4B_FMT_MXFP4) return NibPlanes{};
+    else return nib_planes<DT>(code, scale);
   };
   auto stage = [&](int set, int buf, float scale) {
     const NibPlanes t = planes(scale);
@@ -236,11 +209,11 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
       bv[ns] = *reinterpret_cast<const uint4*>(&Ws[buf][w_frag + nbase[ns] * kTileK + (fcol ^ bpar[ns])]);
   };
   auto mfma_row = [&](int ms, const uint4 (&av)[MS], const uint4 (&bv)[NS]) {
-    static_for<NS>([&](auto ns) { acc[ms][ns] = mfma_32x32x16<CT>(av[ms], bv[ns], acc[ms][ns]); });
+    static_for<NS>([&](auto ns) { acc[ms][ns] = mfma_32x32x16<DT>(av[ms], bv[ns], acc[ms][ns]); });
   };
   auto mfmas = [&](const uint4 (&av)[MS], const uint4 (&bv)[NS]) {
     static_for<MS>([&](auto ms) {
-      static_for<NS>([&](auto ns) { acc[ms][ns] = mfma_32x32x16<CT>(av[ms], bv[ns], acc[ms][ns]); });
+      static_for<NS>([&](auto ns) { acc[ms][ns] = mfma_32x32x16<DT>(av[ms], bv[ns], acc[ms][ns]); });
     });
   };
 
@@ -252,7 +225,7 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
   load_a_all(0);
   load_w(0, 0);
   load_w(1, min<int64_t>(1, klast));
-  __syncthreads();  // code2 table, row shifts
+  __syncthreads();  // code2 table
   stage(0, 0, block_scale(0));
   load_a_all(min<int64_t>(1, klast));
   load_w(0, min<int64_t>(2, klast));
@@ -285,7 +258,7 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
     const int64_t ka = min<int64_t>(kb + 2, klast);
     read_frags(cur, 1, fa1, fb1);
     mfma_row(0, fa0, fb0);
-    put_w(cur ^ 1, 2, tp, lk);
+    put_w(cur ^ 1, 2, lk);
     fetch_w(sS, 3, tp, lk);
     load_a(ka, 0);
     load_a(ka, 1);
@@ -295,7 +268,7 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
     load_a(ka, 3);
     __builtin_amdgcn_sched_barrier(0);
     mfma_row(2, fa0, fb0);
-    put_w(cur ^ 1, 3, tp, lk);
+    put_w(cur ^ 1, 3, lk);
     fetch_w(sS, 4, tp, lk);
     __builtin_amdgcn_sched_barrier(0);
     mfma_row(3, fa0, fb0);
@@ -306,7 +279,7 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
     // code2 read is then long done when sub-step 3 stages the step)
     read_frags(cur, 2, fa0, fb0);
     mfma_row(0, fa1, fb1);
-    put_w(cur ^ 1, 4, tp, lk);
+    put_w(cur ^ 1, 4, lk);
     fetch_w(sS, 5, tp, lk);
     __builtin_amdgcn_sched_barrier(0);
     mfma_row(1, fa1, fb1);
@@ -315,7 +288,7 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
     const float sc = block_scale(sT);
     __builtin_amdgcn_sched_barrier(0);
     mfma_row(2, fa1, fb1);
-    put_w(cur ^ 1, 5, tp, lk);
+    put_w(cur ^ 1, 5, lk);
     fetch_w(sS, 6, tp, lk);
     __builtin_amdgcn_sched_barrier(0);
     mfma_row(3, fa1, fb1);
@@ -323,11 +296,11 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
     // sub-step 2
     read_frags(cur, 3, fa1, fb1);
     mfma_row(0, fa0, fb0);
-    put_w(cur ^ 1, 6, tp, lk);
+    put_w(cur ^ 1, 6, lk);
     fetch_w(sS, 7, tp, lk);
     __builtin_amdgcn_sched_barrier(0);
     mfma_row(1, fa0, fb0);
-    put_w(cur ^ 1, 7, tp, lk);
+    put_w(cur ^ 1, 7, lk);
     __builtin_amdgcn_sched_barrier(0);
     mfma_row(2, fa0, fb0);
     load_w(sS, knext);  // the weight registers of set sS are free after word 7
@@ -344,13 +317,13 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
     fetch_w(sT, 0, tp, lk);
     __builtin_amdgcn_sched_barrier(0);
     mfma_row(1, fa1, fb1);
-    put_w(cur, 0, tp, lk);
+    put_w(cur, 0, lk);
     fetch_w(sT, 1, tp, lk);
     store_a(cur, 2);
     store_a(cur, 3);
     __builtin_amdgcn_sched_barrier(0);
     mfma_row(2, fa1, fb1);
-    put_w(cur, 1, tp, lk);
+    put_w(cur, 1, lk);
     fetch_w(sT, 2, tp, lk);
     store_a(cur, 4);
     store_a(cur, 5);
@@ -373,14 +346,6 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
   // every store issued before it.
   const int lane_e = static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
   auto row_of = [&](int ms, int i) { return wave_m * 128 + ms * 32 + 8 * (i >> 2) + 4 * (lane_e >> 5) + (i & 3); };
-  if constexpr (F16C) {
-    static_for<MS>([&](auto ms) {
-      static_for<16>([&](auto i) {
-        const int d = -(row_shift_s[row_of(ms, i)] + wsh);
-        static_for<NS>([&](auto ns) { acc[ms][ns][int(i)] = __builtin_amdgcn_ldexpf(acc[ms][ns][int(i)], d); });
-      });
-    });
-  }
   const bool has_bias = p.w.bias != nullptr;
   const uint16_t* bias = static_cast<const uint16_t*>(p.w.bias);
   if (pair && p.epi == E4B_EPI_SWIGLU && !has_bias && !p.out_f32) {  // gate_up: silu(g) * u -> dt
@@ -442,31 +407,20 @@ E4B_DEV void wide_tile(const GemmArgs& p, int tile, int n_tile, uint16_t (&As)[2
   });
 }
 
-template <int DT, int FMT, bool F16C = false>
+template <int DT, int FMT>
 __global__ void __launch_bounds__(kWideThreads) gemm_wide_kernel(GemmArgs p) {
-  static_assert(!F16C || (DT == E4B_BF16 && FMT != E4B_FMT_MXFP4), "fp16 mode: bf16 activations, NF4 weights");
   constexpr int BM = kWideTileM, BN = kWideTileN;
   __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * kTileK];
   __shared__ __attribute__((aligned(16))) uint16_t Ws[2][BN * kTileK];
   __shared__ float code2_s[(FMT == E4B_FMT_NF4_DQ) ? 256 : 1];
-  __shared__ int row_shift_s[F16C ? BM : 1];
-  __shared__ uint32_t ptab[F16C ? 256 * kPairCopies : 1];
   const int cols = is_gated(p.epi) ? BN / 2 : BN;
   const int n_tiles = static_cast<int>((p.n_out + cols - 1) / cols);
   const TileItem item = tile_item(p.rt, n_tiles);
   if (!item.ok) return;
   const int tile = item.tile, n_tile = item.n_tile;
-  if constexpr (F16C) {
-    // the table of code pairs: pass j fills entries 16 j .. 16 j + 15, all copies; entry
-    // 16 j + t / 16 of copy t % 16 (high nibble j, low nibble t / 16)
-    static_assert(kWideThreads == 16 * kPairCopies, "table fill");
-    const float lo = p.w.code[threadIdx.x / kPairCopies];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) ptab[j * kWideThreads + threadIdx.x] = cvt_pair<E4B_FP16>(p.w.code[j], lo);
-  }
   const int rows = p.rt.offsets[item.e + 1] - item.row0;  // the tile's rows, capped at BM below
-  if (rows <= BM / 2) wide_tile<DT, FMT, F16C, true>(p, tile, n_tile, As, Ws, code2_s, row_shift_s, ptab);
-  else wide_tile<DT, FMT, F16C, false>(p, tile, n_tile, As, Ws, code2_s, row_shift_s, ptab);
+  if (rows <= BM / 2) wide_tile<DT, FMT, true>(p, tile, n_tile, As, Ws, code2_s);
+  else wide_tile<DT, FMT, false>(p, tile, n_tile, As, Ws, code2_s);
 }
 
 }  // namespace e4b

@@ -140,10 +140,11 @@ def _train_tile_m(M: int, E: int) -> int:
 
 
 def fused_experts_train_forward(lora_mod, hidden_states, top_k_index, top_k_weights):
-    """Training-capable fused forward of an ``ExpertsLoRA`` (``fast.py:453-556``): both projections
-    through ``_GroupedLoraProj``, the base's own epilogue between them, the fp32 router-weighted
-    combine, all differentiable; evicted storage or a non-bf16/fp16 compute dtype runs the saved
-    reference forward."""
+    """Training-capable fused forward of an ``ExpertsLoRA`` (``fast.py:453-556``): the whole layer through
+    ``_FusedLoraLayer`` where ``_layer_inputs`` takes it, else both projections through
+    ``_GroupedLoraProj`` with the base's own epilogue between them and the fp32 router-weighted combine,
+    all differentiable; evicted storage or a non-bf16/fp16 compute dtype runs the saved reference
+    forward."""
     from . import fast as F
     from .lora import _epilogue
 

@@ -129,17 +129,15 @@ CANCEL = [((1 + 2.0 ** -9 + 2.0 ** -18, 1 + 2.0 ** -9), (1.0, -1.0)),
 
 
 @pytest.mark.parametrize("T,hid,inter", [(150, 192, 256), (300, 256, 192), (20, 256, 256), (20, 192, 320)])
-@pytest.mark.parametrize("adt", (torch.float32, torch.float16, torch.bfloat16))
-@pytest.mark.parametrize("case", range(len(CANCEL)))
+@pytest.mark.parametrize("adt,case", [(torch.float32, 0), (torch.float32, 1), (torch.float32, 2), (torch.float16, 0),
+                                      (torch.float16, 2), (torch.bfloat16, 0)])  # the adapters that dtype holds exactly
 def test_deltas_keep_32_bits(T, hid, inter, adt, case):
     """Deltas t . B (forward) and u . A (backward) of two ranks that cancel to 2^-18, over zero weights:
     halved and whole 256-row tiles, 32-row tiles with K a multiple of 256 and not. Every product and sum is exact,
-    so the rows are equal. An adapter dtype that cannot hold the case's values is left out."""
+    so the rows are equal."""
     _announce(f"delta bits T={T} hid={hid} inter={inter} {adt} case={case}")
     (t0, t1), (b0, b1) = CANCEL[case]
     pair = torch.tensor([b0, b1], device=DEV)
-    if not torch.equal(pair.to(adt).float(), pair):
-        pytest.skip("the dtype rounds these adapters")
     w1, w2 = _zero_layer(hid, inter)
     bits = torch.zeros(hid, device=DEV)
     bits[:3] = torch.tensor([1.0, 2.0 ** -9, 2.0 ** -18])
