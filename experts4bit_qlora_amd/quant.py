@@ -20,6 +20,7 @@ from __future__ import annotations
 import functools
 
 import torch
+from torch.autograd import forward_ad as _forward_ad
 
 NF4_CODE = (
     -1.0, -0.6961928009986877, -0.5250730514526367, -0.39491748809814453,
@@ -150,8 +151,8 @@ def _plain_on_device(w: torch.Tensor) -> bool:
     which is the kernels' definition)."""
     return (w.is_cuda and type(w) in (torch.Tensor, torch.nn.Parameter) and w.is_floating_point()
             and not (w.requires_grad and torch.is_grad_enabled())
-            and not torch._C._functorch.is_functorch_wrapped_tensor(w) and not torch.jit.is_tracing()
-            and torch.autograd.forward_ad.unpack_dual(w).tangent is None)
+            and not torch._C._functorch.is_functorch_wrapped_tensor(w) and not torch._C._is_tracing()
+            and (_forward_ad._current_level < 0 or _forward_ad.unpack_dual(w).tangent is None))
 
 
 def _on_kernel(w: torch.Tensor, blocksize: int) -> bool:
