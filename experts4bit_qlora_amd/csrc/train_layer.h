@@ -300,7 +300,7 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_u_mfma_kernel(const uint
   int c = 0;
   for (; c + 4 <= nchunks; c += 4) {
     static_for<4>([&](auto q) { step(q, c + int(q)); });
-    sums.fold();
+    if (c & 4) sums.fold();  // every second trip
   }
   static_for<3>([&](auto q) {
     if (c + int(q) < nchunks) step(q, c + int(q));
