@@ -238,13 +238,14 @@ E4B_DEV int lora_t_at(int q, int g) { return q * kLoraTK + (((g ^ q) & 7) << 3);
 // vector units' 64 partial sums; here at most eight products of 32 columns add up (each half of a chunk and
 // the adapters' lower parts apart) before they go to the total, whose rounding errors are kept (two-sum):
 // 0.7 times the vector units' error. (Four before each: 0.5 times, and 2 us more per 258-row launch.)
-template <int NSM>
+template <int NSM, bool LOW>
 struct RankSums {
-  f32x4_t acc[3][NSM], total[NSM], lost[NSM];
+  f32x4_t acc[LOW ? 3 : 2][NSM], total[NSM], lost[NSM];
   E4B_DEV RankSums() {
     const f32x4_t zero{0.0f, 0.0f, 0.0f, 0.0f};
     static_for<NSM>([&](auto n) __attribute__((always_inline)) {
-      acc[0][n] = acc[1][n] = acc[2][n] = total[n] = lost[n] = zero;
+      acc[0][n] = acc[1][n] = total[n] = lost[n] = zero;
+      if constexpr (LOW) acc[2][n] = zero;
     });
   }
   E4B_DEV void fold() {
@@ -256,7 +257,7 @@ struct RankSums {
       a = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     });
   }
-  E4B_DEV float value(int n, int i) const { return total[n][i] + (lost[n][i] + acc[2][n][i]); }
+  E4B_DEV float value(int n, int i) const { return total[n][i] + (LOW ? lost[n][i] + acc[LOW ? 2 : 0][n][i] : lost[n][i]); }
 };
 
 template <int ADT, int BM, int NSM>
@@ -285,30 +286,38 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
   const int nchunks = static_cast<int>(in / kLoraTK);
   auto chunk = [&](int c) { return min(c, nchunks - 1); };  // past the last chunk it is re-read
 
-  // staging: thread tid takes groups j = tid + NT i of the chunk's [16 NSM ranks][8 groups]
-  float sets[2][SPT][8];
-  // (inlined always: a call left standing would put the sets in scratch memory)
+  // staging: thread tid takes groups j = tid + NT i of the chunk's [16 NSM ranks][8 groups], as loaded until
+  // they are stored (inlined always: a call left standing would put the sets in scratch memory)
+  constexpr int kRaw = ADT == E4B_FP32 ? 2 : 1;
+  uint4 sets[2][SPT][kRaw];
   auto load_a = [&](auto set, int c) __attribute__((always_inline)) {
-    float (&sv)[SPT][8] = sets[decltype(set)::value];
     static_for<SPT>([&](auto i) __attribute__((always_inline)) {
       const int j = tid + NT * int(i);
       if (NSTAGE % NT != 0 && j >= NSTAGE) return;
       const int q = min(j / kLoraTGroups, rank - 1), gg = j % kLoraTGroups;
-      const int64_t o = (int64_t(e) * rank + q) * in + int64_t(c) * kLoraTK + 8 * gg;
-      load8<ADT>(A, o, sv[i]);
+      const uint4* const src =
+          reinterpret_cast<const uint4*>(static_cast<const char*>(A) + ((int64_t(e) * rank + q) * in + int64_t(c) * kLoraTK + 8 * gg) *
+                                                                           (ADT == E4B_FP32 ? 4 : 2));
+#pragma unroll
+      for (int h = 0; h < kRaw; ++h) sets[decltype(set)::value][i][h] = src[h];
     });
   };
   auto store_a = [&](auto set, int buf) __attribute__((always_inline)) {
-    const float (&sv)[SPT][8] = sets[decltype(set)::value];
     static_for<SPT>([&](auto i) __attribute__((always_inline)) {
       const int j = tid + NT * int(i);
       if (NSTAGE % NT != 0 && j >= NSTAGE) return;
       const int q = j / kLoraTGroups, gg = j % kLoraTGroups;
-      float v[8];
-#pragma unroll
-      for (int h = 0; h < 8; ++h) v[h] = q < rank ? sv[i][h] : 0.0f;
+      const uint4 (&raw)[kRaw] = sets[decltype(set)::value][i];
       uint4 part[NP];
-      split_parts8<NP>(v, part);
+      if constexpr (ADT == E4B_BF16) {  // its own only part
+        part[0] = q < rank ? raw[0] : make_uint4(0, 0, 0, 0);
+      } else {
+        float v[8];
+        load8<ADT>(raw, 0, v);
+#pragma unroll
+        for (int h = 0; h < 8; ++h) v[h] = q < rank ? v[h] : 0.0f;
+        split_parts8<NP>(v, part);
+      }
 #pragma unroll
       for (int h = 0; h < NP; ++h) *reinterpret_cast<uint4*>(&as[h][buf][lora_t_at(q, gg)]) = part[h];
     });
@@ -320,7 +329,7 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
       xf[s] = *reinterpret_cast<const uint4*>(xr + int64_t(c) * kLoraTK + 32 * s + 8 * g);
   };
 
-  RankSums<NSM> sums;
+  RankSums<NSM, (NP > 1)> sums;
   // chunk c from LDS buffer c % 2 and x set c % 4; meanwhile chunk c + 1's A goes from registers (set
   // (c + 1) % 2) into the other buffer, chunk c + 2's A and chunk c + 3's x are requested
   uint4 xs[4][2];

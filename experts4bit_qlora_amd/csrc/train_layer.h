@@ -273,7 +273,7 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_u_mfma_kernel(const uint
     const uint2 hi = lds_read_tr(b + wgrad_at<RB>(row + 4, col));
     return make_uint4(lo.x, lo.y, hi.x, hi.y);
   };
-  RankSums<NSM> sums;
+  RankSums<NSM, (NP > 1)> sums;
   uint4 xs[4][2];  // B two chunks and g three chunks ahead, as lora_t_mfma_kernel
   auto step = [&](auto uc, int c) __attribute__((always_inline)) {
     constexpr int v = decltype(uc)::value;  // c % 4
