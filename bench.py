@@ -631,9 +631,10 @@ def gptoss_benches(steps, warmup, gptoss_layers=4):
 def train_bench(steps, warmup, tokens=2048, rank=16, ref_steps=3):
     """The training lane on one OLMoE-geometry layer (E=64, H=2048, I=1024, top-8): ExpertsLoRA
     with rank-16 fp32 adapters (B nonzero), a 2048-token micro-batch, loss = sum(out * fixed
-    weights). Times the fused forward + backward (enable_fast_train) and the module's reference
-    per-expert loop (same GPU, same module) with events, and the grouped dgrad of each projection
-    alone: algorithmic FLOP 2 * M * n * k per launch / its average time, against the dense bf16
+    weights). Times the fused forward + backward with that loss (enable_fast_train) and the module's
+    reference per-expert loop (same GPU, same module) with events, and the standalone grouped dgrad
+    (e4b_grouped_dgrad, which fp16 layers and custom activations train through) of each projection:
+    algorithmic FLOP 2 * M * n * k per launch / its average time, against the dense bf16
     peak."""
     import torch
 

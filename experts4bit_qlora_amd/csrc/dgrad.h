@@ -23,8 +23,9 @@
 //
 // Against dgrad_mfma_kernel (train.h: e4b_grouped_dgrad's exact bf16 weights, decoded in registers
 // and transposed by v_perm before staging, the delta added by a pass of its own): both OLMoE projections
-// at 2,048 tokens, rank 16, took 612 us there plus 141 us of delta passes, and take 297 us of wide
-// launches here with 253 us of narrow ones beside them on a second stream.
+// at 2,048 tokens, rank 16, took 612 us there plus 141 us of delta passes, and take 361 us of wide
+// launches here (600 and 496 TFLOP/s) with the narrow ones (76 us alone, 1.0-1.8 TB/s of weights) beside
+// them on a second stream.
 #pragma once
 
 #include "gemm.h"
