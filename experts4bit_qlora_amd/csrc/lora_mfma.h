@@ -213,19 +213,16 @@ E4B_DEV void lora_delta_16x16(const GemmArgs& p, f32x4_t (&acc)[MS][NS], int e, 
   }
 }
 
-}  // namespace e4b
-
-namespace e4b {
-
 // t[m, q] = sum_c x_m[c] * A[e, q, c] for the sorted rows m of every routing tile (one expert per
 // tile), on the matrix cores: the t of the fp16-mode LoRA path (rows past the routed ones are not
 // written). One workgroup per BM-row part of a tile, one wave per 16 rows, each wave all ranks of
 // its rows (NSM 16-rank blocks) on v_mfma_f32_16x16x32_bf16. x rows are bf16 (exact operands); A is
 // staged per 64-deep chunk in LDS as its bf16 parts (one of a bf16, two of an fp16, three of an fp32
 // adapter: split_parts8), so every product is exact and t is an fp32 sum, as the VALU passes
-// (lora_a_kernel) form it. The chunks are double-buffered, one barrier per chunk, with A two chunks and x three chunks ahead in registers: a launch has only
-// a workgroup or two per CU, so the x loads in flight per wave set its rate (one chunk ahead: 43 us
-// for both of an OLMoE layer's t at 1,531 tokens, 31 us so).
+// (lora_a_kernel) form it. The chunks are double-buffered, one barrier per chunk, with A two chunks and
+// x three chunks ahead in registers: a launch has only a workgroup or two per CU, so the x loads in flight
+// per wave set its rate. Both of an OLMoE layer's t at 1,531 tokens: 43 us one chunk ahead, 31 so; 38
+// with an fp32 adapter's third part and the compensated totals.
 constexpr int kLoraTK = 64;  // K per chunk
 constexpr int kLoraTGroups = kLoraTK / 8;
 
@@ -237,7 +234,7 @@ E4B_DEV int lora_t_at(int q, int g) { return q * kLoraTK + (((g ^ q) & 7) << 3);
 // The sums of t and u. One fp32 accumulator over the whole row was 1.5 times as far from 64 bits as the
 // vector units' 64 partial sums; here at most eight products of 32 columns add up (each half of a chunk and
 // the adapters' lower parts apart) before they go to the total, whose rounding errors are kept (two-sum):
-// 0.7 times the vector units' error. (Four before each: 0.5 times, and 2 us more per 258-row launch.)
+// 0.7 times the vector units' error. (Four: 0.5 times, and 1.5 us more per launch at 258 tokens.)
 template <int NSM, bool LOW>
 struct RankSums {
   f32x4_t acc[LOW ? 3 : 2][NSM], total[NSM], lost[NSM];
@@ -295,9 +292,8 @@ __global__ void __launch_bounds__(BM / 16 * kWave) lora_t_mfma_kernel(const uint
       const int j = tid + NT * int(i);
       if (NSTAGE % NT != 0 && j >= NSTAGE) return;
       const int q = min(j / kLoraTGroups, rank - 1), gg = j % kLoraTGroups;
-      const uint4* const src =
-          reinterpret_cast<const uint4*>(static_cast<const char*>(A) + ((int64_t(e) * rank + q) * in + int64_t(c) * kLoraTK + 8 * gg) *
-                                                                           (ADT == E4B_FP32 ? 4 : 2));
+      const int64_t o = (int64_t(e) * rank + q) * in + int64_t(c) * kLoraTK + 8 * gg;  // 8 values: kRaw pieces
+      const uint4* const src = static_cast<const uint4*>(A) + o / 8 * kRaw;
 #pragma unroll
       for (int h = 0; h < kRaw; ++h) sets[decltype(set)::value][i][h] = src[h];
     });
